@@ -24,6 +24,7 @@
 // derivative Wd = dW/dd by pushing the tangent g' = dg/dd through the same
 // chain (a second accumulator set sharing every A fragment).
 #include "common.h"
+#include "filter_gate.h"
 #include "split16.h"
 
 #include <hip/hip_fp16.h>
@@ -50,6 +51,7 @@ constexpr int kFT = kF / 16;     // feature tiles of 16
 constexpr int kWaves = 8;        // waves per workgroup
 constexpr int kThreads = kWaves * MLCG_WAVE;
 constexpr int kMaxK = 128;
+constexpr float kWeightBound = 65504.0f;  // of the split kernels (the fp16 maximum)
 
 // Radial basis (per basis function k, distance d, envelope C(d)):
 //   basis 0, Gaussian (gaussian.py:83-102): g_k = C exp(c (d - centers[k])^2),
@@ -175,6 +177,19 @@ __device__ __forceinline__ void rbf_eval(const RbfParams& rp, bool on, float cen
     g = e * crbf;
     gd = e * (dcrbf + 2.0f * rp.alpha * wid * u * ex * crbf);
   }
+}
+
+// The exponential-normal basis with its inner exponential in double: g depends
+// on exp(alpha (lo - d)) - centre with a factor 2 beta u of some 45, so that
+// the half ulp of a float there already costs g 1.4e-6.
+__device__ __forceinline__ void rbf_expnormal_fine(const RbfParams& rp, float cen, float wid,
+                                                   float d, float crbf, float dcrbf, float& g,
+                                                   float& gd) {
+  const double ex = exp((double)rp.alpha * ((double)rp.rbf_lo - (double)d));
+  const float u = (float)(ex - (double)cen);
+  const float e = __expf(-wid * (u * u));
+  g = e * crbf;
+  gd = e * (dcrbf + 2.0f * rp.alpha * wid * u * (float)ex * crbf);
 }
 
 // rbf_eval for a compile-time basis kind (no branch on rp.basis).
@@ -346,7 +361,8 @@ __global__ __launch_bounds__(kThreads) void filter_fwd_f32_kernel(
     const int32_t* __restrict__ pj, const int32_t* __restrict__ n_pairs_dev,
     int64_t max_pairs, RbfParams rp, const float* __restrict__ W1,
     const float* __restrict__ b1, const float* __restrict__ W2, float* __restrict__ Wout,
-    float* __restrict__ Wdout, float* __restrict__ dist_out) {
+    float* __restrict__ Wdout, float* __restrict__ dist_out, FilterGate gate) {
+  if (gate_closed(gate)) return;
   extern __shared__ float lds[];
   const int KS = (rp.K + 3) / 4;
   float* w1s = lds;
@@ -411,6 +427,188 @@ __global__ __launch_bounds__(kThreads) void filter_fwd_f32_kernel(
         nt_store4(wdr + 16 * t, od);
       }
       if (dist_out && q == 0) dist_out[p] = d;
+    }
+  }
+}
+
+// The filter at the nodes of a uniform distance grid (filter_table.hip): node
+// k < nodes at k h, node `nodes` at rc.  Per block of the batch (blockIdx.y)
+// four planes [nodes + 1][128]: W, dW/dd, and H, dH/dd of the activations
+// times the CFConv envelope, which only the check of the grid reads.  fp32
+// MFMA throughout.
+//
+// ~10^3 tiles of 16 nodes in all, so the launch is latency bound: staging the
+// weights in LDS as the pair kernels do cost 60 us of the 75 us it took.  Here
+// wave w of 8 owns feature tile w of both products: its slices of W1 and W2
+// (13 + 32 registers) are read straight into the A fragments, the activations
+// pass through LDS once, and a workgroup takes two node tiles.
+constexpr int kTableBlocks = 8;
+constexpr int kTableTiles = 2;
+constexpr int kTableStride = kF + 4;  // floats per node row in LDS (bank spread)
+struct FilterTableBatch {
+  const float* W1[kTableBlocks];
+  const float* b1[kTableBlocks];
+  const float* W2[kTableBlocks];
+};
+
+// Envelope (identity, or cosine with lower bound 0) and basis function in double.
+__device__ __forceinline__ void cutoff_f64(int kind, float hi, double d, double& c, double& dc) {
+  c = 1.0;
+  dc = 0.0;
+  if (kind == MLCG_CUT_COSINE) {
+    const double ih = 1.0 / (double)hi;
+    double sn, cs;
+    sincospi(d * ih, &sn, &cs);
+    const double m = d < (double)hi ? 1.0 : 0.0;
+    c = 0.5 * (cs + 1.0) * m;
+    dc = -0.5 * sn * (3.14159265358979323846 * ih) * m;
+  }
+}
+
+__device__ __forceinline__ void rbf_f64(const RbfParams& rp, int k, double d, double crbf,
+                                        double dcrbf, double& g, double& gd) {
+  const double cen = rp.centers[k];
+  if (rp.basis == 0) {
+    const double wid = rp.widths[0], diff = d - cen;
+    const double e = exp(wid * diff * diff);
+    g = e * crbf;
+    gd = e * (2.0 * wid * diff * crbf + dcrbf);
+  } else {
+    const double wid = rp.widths[k], alpha = rp.alpha;
+    const double ex = exp(alpha * ((double)rp.rbf_lo - d)), u = ex - cen;
+    const double e = exp(-wid * u * u);
+    g = e * crbf;
+    gd = e * (dcrbf + 2.0 * alpha * wid * u * ex * crbf);
+  }
+}
+
+template <int KSMAX>
+__global__ __launch_bounds__(kThreads) void filter_table_kernel(
+    FilterTableBatch fb, int nodes, float h, float rc, RbfParams rp, float* __restrict__ tables,
+    unsigned* __restrict__ gates) {
+  __shared__ __align__(16) float hs[kTableTiles][2][16 * kTableStride];
+  __shared__ float gs[kTableTiles][2][4 * KSMAX][16];
+  __shared__ unsigned smax[kWaves];
+  const int blk = blockIdx.y;
+  const int w = threadIdx.x / MLCG_WAVE, l = mlcg_lane();
+  const int q = l >> 4, n = l & 15;
+  const int K = rp.K;
+  const float* W1 = fb.W1[blk] + (16 * w + n) * K;
+  const float* W2 = fb.W2[blk] + (16 * w + n) * kF + 4 * q;
+  float a1[KSMAX];
+  float4 a2[kFT];
+#pragma unroll
+  for (int s = 0; s < KSMAX; ++s) a1[s] = 4 * s + q < K ? W1[4 * s + q] : 0.0f;
+#pragma unroll
+  for (int u = 0; u < kFT; ++u) a2[u] = *reinterpret_cast<const float4*>(W2 + 16 * u);
+  const float4 bias = *reinterpret_cast<const float4*>(fb.b1[blk] + 16 * w + 4 * q);
+  const float bv[4] = {bias.x, bias.y, bias.z, bias.w};
+  // the basis at the nodes, each wave its k steps: in double, since a node's
+  // rounding is shared by every pair near it and does not average out over the
+  // pairs (exponential-normal basis in fp32: the forces' parameter gradients
+  // 4e-6 off instead of 6e-7)
+#pragma unroll
+  for (int t = 0; t < kTableTiles; ++t) {
+    const int k = (blockIdx.x * kTableTiles + t) * 16 + n;
+    const double d = k < nodes ? (double)k * (double)h : (double)rc;
+    double crbf, dcrbf;
+    cutoff_f64(rp.rbf_kind, rp.rbf_hi, d, crbf, dcrbf);
+    for (int s = w; s < KSMAX; s += kWaves) {
+      double g = 0.0, gd = 0.0;
+      if (4 * s + q < K) rbf_f64(rp, 4 * s + q, d, crbf, dcrbf, g, gd);
+      gs[t][0][4 * s + q][n] = (float)g;
+      gs[t][1][4 * s + q][n] = (float)gd;
+    }
+  }
+  __syncthreads();
+  const int64_t plane = (int64_t)(nodes + 1) * kF;
+  float* out = tables + (int64_t)blk * 4 * plane + 16 * w + 4 * q;
+  float cc[kTableTiles], dcc[kTableTiles];
+  unsigned steep = 0u;  // |a'| h as bits: a NaN stays the largest
+  // a weight past the split kernels' range closes the gate: they report it
+  float big = 0.0f;
+#pragma unroll
+  for (int s = 0; s < KSMAX; ++s) big = fmaxf(big, fabsf(a1[s]));
+#pragma unroll
+  for (int u = 0; u < kFT; ++u)
+    big = fmaxf(big, fmaxf(fmaxf(fabsf(a2[u].x), fabsf(a2[u].y)),
+                           fmaxf(fabsf(a2[u].z), fabsf(a2[u].w))));
+  if (!(big < kWeightBound)) steep = __float_as_uint(__builtin_huge_valf());
+#pragma unroll
+  for (int t = 0; t < kTableTiles; ++t) {
+    const int k = (blockIdx.x * kTableTiles + t) * 16 + n;
+    double c64, dc64;
+    cutoff_f64(rp.conv_kind, rp.conv_hi, k < nodes ? (double)k * (double)h : (double)rc, c64,
+               dc64);
+    cc[t] = (float)c64;
+    dcc[t] = (float)dc64;
+    floatx4 a = {0.f, 0.f, 0.f, 0.f}, ad = {0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+    for (int s = 0; s < KSMAX; ++s) {
+      a = __builtin_amdgcn_mfma_f32_16x16x4f32(a1[s], gs[t][0][4 * s + q][n], a, 0, 0, 0);
+      ad = __builtin_amdgcn_mfma_f32_16x16x4f32(a1[s], gs[t][1][4 * s + q][n], ad, 0, 0, 0);
+    }
+    float4 hv, hd, hc, hdc;
+    float* pv = &hv.x;
+    float* pd = &hd.x;
+    float* pc = &hc.x;
+    float* pdc = &hdc.x;
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+      float s, d1, d2;
+      mlcg_act(rp.act, a[i] + bv[i], s, d1, d2);
+      const unsigned u = __float_as_uint(fabsf(ad[i]) * h);
+      steep = steep > u ? steep : u;
+      pv[i] = s;
+      pd[i] = d1 * ad[i];
+      pc[i] = s * cc[t];
+      pdc[i] = pd[i] * cc[t] + s * dcc[t];
+    }
+    *reinterpret_cast<float4*>(&hs[t][0][n * kTableStride + 16 * w + 4 * q]) = hv;
+    *reinterpret_cast<float4*>(&hs[t][1][n * kTableStride + 16 * w + 4 * q]) = hd;
+    if (k <= nodes) {
+      *reinterpret_cast<float4*>(out + 2 * plane + (int64_t)k * kF) = hc;
+      *reinterpret_cast<float4*>(out + 3 * plane + (int64_t)k * kF) = hdc;
+    }
+  }
+  // one atomic per workgroup: ~2000 on one address took longer than the rest
+#pragma unroll
+  for (int o = 32; o > 0; o >>= 1) {
+    const unsigned u = __shfl_xor(steep, o, MLCG_WAVE);
+    steep = steep > u ? steep : u;
+  }
+  if (l == 0) smax[w] = steep;
+  __syncthreads();
+  if (threadIdx.x == 0) {
+    for (int i = 1; i < kWaves; ++i) steep = steep > smax[i] ? steep : smax[i];
+    atomicMax(gates + blk * kGateWords + 8, steep);
+  }
+#pragma unroll
+  for (int t = 0; t < kTableTiles; ++t) {
+    const int k = (blockIdx.x * kTableTiles + t) * 16 + n;
+    floatx4 v = {0.f, 0.f, 0.f, 0.f}, vd = {0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+    for (int u = 0; u < kFT; ++u) {
+      const float4 x =
+          *reinterpret_cast<const float4*>(&hs[t][0][n * kTableStride + 16 * u + 4 * q]);
+      const float4 y =
+          *reinterpret_cast<const float4*>(&hs[t][1][n * kTableStride + 16 * u + 4 * q]);
+      v = __builtin_amdgcn_mfma_f32_16x16x4f32(a2[u].x, x.x, v, 0, 0, 0);
+      vd = __builtin_amdgcn_mfma_f32_16x16x4f32(a2[u].x, y.x, vd, 0, 0, 0);
+      v = __builtin_amdgcn_mfma_f32_16x16x4f32(a2[u].y, x.y, v, 0, 0, 0);
+      vd = __builtin_amdgcn_mfma_f32_16x16x4f32(a2[u].y, y.y, vd, 0, 0, 0);
+      v = __builtin_amdgcn_mfma_f32_16x16x4f32(a2[u].z, x.z, v, 0, 0, 0);
+      vd = __builtin_amdgcn_mfma_f32_16x16x4f32(a2[u].z, y.z, vd, 0, 0, 0);
+      v = __builtin_amdgcn_mfma_f32_16x16x4f32(a2[u].w, x.w, v, 0, 0, 0);
+      vd = __builtin_amdgcn_mfma_f32_16x16x4f32(a2[u].w, y.w, vd, 0, 0, 0);
+    }
+    if (k <= nodes) {
+      float* o = out + (int64_t)k * kF;
+      *reinterpret_cast<float4*>(o) =
+          float4{v[0] * cc[t], v[1] * cc[t], v[2] * cc[t], v[3] * cc[t]};
+      *reinterpret_cast<float4*>(o + plane) =
+          float4{vd[0] * cc[t] + v[0] * dcc[t], vd[1] * cc[t] + v[1] * dcc[t],
+                 vd[2] * cc[t] + v[2] * dcc[t], vd[3] * cc[t] + v[3] * dcc[t]};
     }
   }
 }
@@ -483,7 +681,8 @@ __global__ __launch_bounds__(kThreads16, kWaves16 * MLCG_F16_GROUPS_PER_CU / 4) 
     const int32_t* __restrict__ pj, const int32_t* __restrict__ n_pairs_dev,
     int64_t max_pairs, RbfParams rp, const float* __restrict__ W1,
     const float* __restrict__ b1, const float* __restrict__ W2, __half* __restrict__ Wout,
-    __half* __restrict__ Wdout, float* __restrict__ dist_out) {
+    __half* __restrict__ Wdout, float* __restrict__ dist_out, FilterGate gate) {
+  if (gate_closed(gate)) return;
   extern __shared__ float lds[];
   _Float16* w1h = reinterpret_cast<_Float16*>(lds);
   _Float16* w2h = w1h + kFT * KS32 * MLCG_WAVE * 8;
@@ -680,7 +879,6 @@ __device__ __forceinline__ floatx4 mfma_x3(halfx8 ah, halfx8 ahs, halfx8 al, hal
 __device__ unsigned mlcg_numerics_word;
 constexpr unsigned kFlagBwdRange = 1u;
 constexpr unsigned kFlagWeightRange = 2u;
-constexpr float kWeightBound = 65504.0f;
 
 __device__ __forceinline__ void raise_numerics_flag(unsigned bits) {
   atomicOr(&mlcg_numerics_word, bits);
@@ -717,7 +915,8 @@ __global__ __launch_bounds__(kThreadsX3) void filter_fwd_x3_kernel(
     const int32_t* __restrict__ pj, const int32_t* __restrict__ n_pairs_dev,
     int64_t max_pairs, RbfParams rp, const float* __restrict__ W1,
     const float* __restrict__ b1, const float* __restrict__ W2, float* __restrict__ Wout,
-    float* __restrict__ Wdout, float* __restrict__ dist_out) {
+    float* __restrict__ Wdout, float* __restrict__ dist_out, FilterGate gate) {
+  if (gate_closed(gate)) return;
   extern __shared__ float lds[];
   const int K = rp.K;
   constexpr int KS32 = kX3Blocks;
@@ -1206,7 +1405,9 @@ __global__ __launch_bounds__(kBwdThreads) void filter_bwd_fused_kernel(
     const int32_t* __restrict__ pj, const int32_t* __restrict__ n_pairs_dev,
     int64_t max_pairs, RbfParams rp, const float* __restrict__ W1,
     const float* __restrict__ b1, const float* __restrict__ W2, PairAdjoint adj,
-    float* __restrict__ abar_out, float* __restrict__ adbar_out, float* __restrict__ partial) {
+    float* __restrict__ abar_out, float* __restrict__ adbar_out, float* __restrict__ partial,
+    FilterGate gate) {
+  if (gate_closed(gate)) return;
   constexpr int KTMAX = (4 * KSMAX + 15) / 16;
   // basis rows span the compile-time maximum width (rows k >= K hold zeros),
   // so the k loops below run without data-dependent branches
@@ -1370,6 +1571,9 @@ __global__ __launch_bounds__(kBwdThreads) void filter_bwd_fused_kernel(
   float rw = 1.0f, trun = 0.0f;
   float ra = 1.0f, arun = 0.0f;  // the same for ab in step 6 (no beta: |g| <= 1)
 
+  // on the nodes of a table the exponential-normal basis takes its inner
+  // exponential in double: a node's rounding is shared by every pair near it
+  const bool fine_basis = !kNodes && BASIS != 0 && gate.words != nullptr && rp.basis == 1;
   const bool tangent = kNodes && adj.g1 != nullptr;
   const bool has_yd = tangent && adj.yd != nullptr;
   // stand-ins for absent tangent arrays: valid memory, values never used
@@ -1406,7 +1610,11 @@ __global__ __launch_bounds__(kBwdThreads) void filter_bwd_fused_kernel(
       if (s < KSMAX) {
         float cen = bcen[e], wid = bwid[e];
         if (!kBasisRegs) basis_params(rp, 4 * s + q, cen, wid);
-        rbf_any<BASIS>(rp, 4 * s + q < K, cen, wid, d, crbf, dcrbf, g, gd);  // zero for k >= K
+        if (fine_basis) {  // uniform
+          if (4 * s + q < K) rbf_expnormal_fine(rp, cen, wid, d, crbf, dcrbf, g, gd);
+        } else {
+          rbf_any<BASIS>(rp, 4 * s + q < K, cen, wid, d, crbf, dcrbf, g, gd);  // zero for k >= K
+        }
       }
       bv.g[e] = g;
       bv.gd[e] = gd;
@@ -1924,7 +2132,8 @@ constexpr int kRedOut = 64;
 
 __global__ __launch_bounds__(256) void filter_bwd_reduce_kernel(
     const float* __restrict__ partial, int groups, int K, float* __restrict__ dW1,
-    float* __restrict__ db1, float* __restrict__ dW2) {
+    float* __restrict__ db1, float* __restrict__ dW2, FilterGate gate) {
+  if (gate_closed(gate)) return;
   __shared__ float part[4][kRedOut];
   const int Kp16 = bwd_kp16(K);
   const int stride = bwd_partial_floats(K);
@@ -2061,14 +2270,16 @@ extern "C" int mlcg_numerics_flags(int* out, int clear, void* stream) {
   return mlcg_launch_status();
 }
 
-extern "C" int mlcg_filter_fwd(const float* pos, const int32_t* pair_ij, int64_t pair_stride,
+namespace {
+
+int filter_fwd_impl(const float* pos, const int32_t* pair_ij, int64_t pair_stride,
                                const int32_t* n_pairs_dev, int64_t max_pairs, int basis,
                                const float* centers, const float* widths, float alpha,
                                int num_rbf, int rbf_cut_kind, float rbf_lo, float rbf_hi,
                                int conv_cut_kind, float conv_lo, float conv_hi, int act,
                                const float* W1, const float* b1, const float* W2,
                                int num_filters, int f16, void* W_out, void* Wd_out,
-                               float* dist_out, void* stream) {
+                               float* dist_out, const FilterGate& gate, void* stream) {
   if (!valid_params(basis, num_rbf, rbf_cut_kind, conv_cut_kind, act, num_filters))
     return MLCG_ERR_UNSUPPORTED;
   MLCG_REQUIRE(max_pairs >= 0 && pair_stride >= max_pairs);
@@ -2089,7 +2300,7 @@ extern "C" int mlcg_filter_fwd(const float* pos, const int32_t* pair_ij, int64_t
 #define MLCG_X3_LAUNCH(B, A)                                                               \
   hipLaunchKernelGGL((filter_fwd_x3_kernel<B, A>), dim3(gx), dim3(kThreadsX3), lds, s, pos,  \
                      pair_ij, pair_ij + pair_stride, n_pairs_dev, max_pairs, rp, W1, b1, W2, \
-                     static_cast<float*>(W_out), static_cast<float*>(Wd_out), dist_out)
+                     static_cast<float*>(W_out), static_cast<float*>(Wd_out), dist_out, gate)
     if (basis == 0 && act == 0) MLCG_X3_LAUNCH(0, 0);
     else if (basis == 0) MLCG_X3_LAUNCH(0, 1);
     else if (act == 0) MLCG_X3_LAUNCH(1, 0);
@@ -2102,7 +2313,7 @@ extern "C" int mlcg_filter_fwd(const float* pos, const int32_t* pair_ij, int64_t
     allow_lds_once();
     hipLaunchKernelGGL(filter_fwd_f32_kernel, dim3(groups), dim3(kThreads), lds, s, pos,
                        pair_ij, pair_ij + pair_stride, n_pairs_dev, max_pairs, rp, W1, b1, W2,
-                       static_cast<float*>(W_out), static_cast<float*>(Wd_out), dist_out);
+                       static_cast<float*>(W_out), static_cast<float*>(Wd_out), dist_out, gate);
   } else {
     // K padded to 64 or 128 (two or four 32-wide k blocks)
     const int KS32 = num_rbf <= 64 ? 2 : 4;
@@ -2116,7 +2327,7 @@ extern "C" int mlcg_filter_fwd(const float* pos, const int32_t* pair_ij, int64_t
   hipLaunchKernelGGL((filter_fwd_f16_kernel<KB, B, A>), dim3(groups16), dim3(kThreads16), lds, \
                      s, pos, pair_ij, pair_ij + pair_stride, n_pairs_dev, max_pairs, rp, W1,   \
                      b1, W2, static_cast<__half*>(W_out), static_cast<__half*>(Wd_out),       \
-                     dist_out)
+                     dist_out, gate)
 #define MLCG_F16_KB(KB)                                       \
   if (basis == 0 && act == 0) MLCG_F16_LAUNCH(KB, 0, 0);      \
   else if (basis == 0) MLCG_F16_LAUNCH(KB, 0, 1);             \
@@ -2129,6 +2340,65 @@ extern "C" int mlcg_filter_fwd(const float* pos, const int32_t* pair_ij, int64_t
     }
 #undef MLCG_F16_KB
 #undef MLCG_F16_LAUNCH
+  }
+  return mlcg_launch_status();
+}
+
+}  // namespace
+
+extern "C" int mlcg_filter_fwd(const float* pos, const int32_t* pair_ij, int64_t pair_stride,
+                               const int32_t* n_pairs_dev, int64_t max_pairs, int basis,
+                               const float* centers, const float* widths, float alpha,
+                               int num_rbf, int rbf_cut_kind, float rbf_lo, float rbf_hi,
+                               int conv_cut_kind, float conv_lo, float conv_hi, int act,
+                               const float* W1, const float* b1, const float* W2,
+                               int num_filters, int f16, void* W_out, void* Wd_out,
+                               float* dist_out, void* stream) {
+  return filter_fwd_impl(pos, pair_ij, pair_stride, n_pairs_dev, max_pairs, basis, centers, widths, alpha, num_rbf, rbf_cut_kind, rbf_lo, rbf_hi, conv_cut_kind, conv_lo, conv_hi, act, W1, b1, W2, num_filters, f16, W_out, Wd_out, dist_out, FilterGate{nullptr, 0}, stream);
+}
+
+extern "C" int mlcg_filter_fwd_gated(const float* pos, const int32_t* pair_ij, int64_t pair_stride,
+                               const int32_t* n_pairs_dev, int64_t max_pairs, int basis,
+                               const float* centers, const float* widths, float alpha,
+                               int num_rbf, int rbf_cut_kind, float rbf_lo, float rbf_hi,
+                               int conv_cut_kind, float conv_lo, float conv_hi, int act,
+                               const float* W1, const float* b1, const float* W2,
+                               int num_filters, int f16, void* W_out, void* Wd_out,
+                               float* dist_out, const uint32_t* gate, int gate_want, void* stream) {
+  return filter_fwd_impl(pos, pair_ij, pair_stride, n_pairs_dev, max_pairs, basis, centers, widths, alpha, num_rbf, rbf_cut_kind, rbf_lo, rbf_hi, conv_cut_kind, conv_lo, conv_hi, act, W1, b1, W2, num_filters, f16, W_out, Wd_out, dist_out, FilterGate{gate, gate_want}, stream);
+}
+
+extern "C" int mlcg_filter_table(const void* const* weights, int num_blocks, int nodes, float h,
+                                 float rc, int basis, const float* centers, const float* widths,
+                                 float alpha, int num_rbf, int rbf_cut_kind, float rbf_lo,
+                                 float rbf_hi, int conv_cut_kind, float conv_lo, float conv_hi,
+                                 int act, int num_filters, float* tables, uint32_t* gates,
+                                 void* stream) {
+  if (!valid_params(basis, num_rbf, rbf_cut_kind, conv_cut_kind, act, num_filters))
+    return MLCG_ERR_UNSUPPORTED;
+  MLCG_REQUIRE(weights && num_blocks >= 1 && nodes >= 16 && h > 0.0f && rc > 0.0f);
+  MLCG_REQUIRE(centers && widths && tables && gates);
+  RbfParams rp = make_params(basis, centers, widths, alpha, num_rbf, rbf_cut_kind, rbf_lo,
+                             rbf_hi, conv_cut_kind, conv_lo, conv_hi, act);
+  const int64_t per = 4LL * (nodes + 1) * kF;
+  for (int first = 0; first < num_blocks; first += kTableBlocks) {
+    const int n = num_blocks - first < kTableBlocks ? num_blocks - first : kTableBlocks;
+    FilterTableBatch fb = {};
+    for (int b = 0; b < n; ++b) {
+      fb.W1[b] = static_cast<const float*>(weights[3 * (first + b)]);
+      fb.b1[b] = static_cast<const float*>(weights[3 * (first + b) + 1]);
+      fb.W2[b] = static_cast<const float*>(weights[3 * (first + b) + 2]);
+      MLCG_REQUIRE(fb.W1[b] && fb.b1[b] && fb.W2[b]);
+    }
+    const dim3 grid(mlcg_div_up(nodes + 1, 16 * kTableTiles), n);
+    float* t = tables + first * per;
+    uint32_t* g = gates + first * kGateWords;
+    if (num_rbf <= 64)
+      hipLaunchKernelGGL(filter_table_kernel<16>, grid, dim3(kThreads), 0, mlcg_stream(stream),
+                         fb, nodes, h, rc, rp, t, g);
+    else
+      hipLaunchKernelGGL(filter_table_kernel<32>, grid, dim3(kThreads), 0, mlcg_stream(stream),
+                         fb, nodes, h, rc, rp, t, g);
   }
   return mlcg_launch_status();
 }
@@ -2148,7 +2418,7 @@ int launch_filter_bwd(const float* pos, const int32_t* pair_ij, int64_t pair_str
                       const float* W2, int num_filters, const PairAdjoint& adj, bool nodes,
                       float* dW1, float* db1, float* dW2, float* abar_out, float* adbar_out,
                       float* workspace, int64_t workspace_floats, bool fp32_strict,
-                      void* stream) {
+                      const FilterGate& gate, void* stream) {
   if (!valid_params(basis, num_rbf, rbf_cut_kind, conv_cut_kind, act, num_filters))
     return MLCG_ERR_UNSUPPORTED;
   MLCG_REQUIRE(max_pairs >= 0 && pair_stride >= max_pairs);
@@ -2170,7 +2440,7 @@ int launch_filter_bwd(const float* pos, const int32_t* pair_ij, int64_t pair_str
   hipLaunchKernelGGL((filter_bwd_fused_kernel<KS, NODES, B, A>), dim3(grid),                 \
                      dim3(kBwdThreads), lds, s, pos, pair_ij, pair_ij + pair_stride,         \
                      n_pairs_dev, max_pairs, rp, W1, b1, W2, adj, abar_out, adbar_out,       \
-                     workspace)
+                     workspace, gate)
 #define MLCG_BWD_SMALL(NODES)                                   \
   if (basis == 0 && act == 0) MLCG_BWD_LAUNCH(16, NODES, 0, 0); \
   else if (basis == 0) MLCG_BWD_LAUNCH(16, NODES, 0, 1);        \
@@ -2189,11 +2459,30 @@ int launch_filter_bwd(const float* pos, const int32_t* pair_ij, int64_t pair_str
 #undef MLCG_BWD_LAUNCH
   const int total = kF * kF + kF * num_rbf + kF;
   hipLaunchKernelGGL(filter_bwd_reduce_kernel, dim3((total + kRedOut - 1) / kRedOut), dim3(256),
-                     0, s, workspace, groups, num_rbf, dW1, db1, dW2);
+                     0, s, workspace, groups, num_rbf, dW1, db1, dW2, gate);
   return mlcg_launch_status();
 }
 
 }  // namespace
+
+static int filter_bwd_impl(const float* pos, const int32_t* pair_ij, int64_t pair_stride,
+                               const int32_t* n_pairs_dev, int64_t max_pairs, int basis,
+                               const float* centers, const float* widths, float alpha,
+                               int num_rbf, int rbf_cut_kind, float rbf_lo, float rbf_hi,
+                               int conv_cut_kind, float conv_lo, float conv_hi, int act,
+                               const float* W1, const float* b1, const float* W2,
+                               int num_filters, const float* Wbar, const float* Wdbar,
+                               float* dW1, float* db1, float* dW2, float* abar_out,
+                               float* adbar_out, float* workspace, int64_t workspace_floats,
+                               int fp32_strict, const FilterGate& gate, void* stream) {
+  MLCG_REQUIRE(max_pairs == 0 || (Wbar && Wdbar));
+  PairAdjoint adj{Wbar, Wdbar, nullptr, nullptr, nullptr, nullptr, nullptr};
+  return launch_filter_bwd(pos, pair_ij, pair_stride, n_pairs_dev, max_pairs, basis, centers,
+                           widths, alpha, num_rbf, rbf_cut_kind, rbf_lo, rbf_hi, conv_cut_kind,
+                           conv_lo, conv_hi, act, W1, b1, W2, num_filters, adj, false, dW1, db1,
+                           dW2, abar_out, adbar_out, workspace, workspace_floats,
+                           fp32_strict != 0, gate, stream);
+}
 
 extern "C" int mlcg_filter_bwd(const float* pos, const int32_t* pair_ij, int64_t pair_stride,
                                const int32_t* n_pairs_dev, int64_t max_pairs, int basis,
@@ -2205,13 +2494,42 @@ extern "C" int mlcg_filter_bwd(const float* pos, const int32_t* pair_ij, int64_t
                                float* dW1, float* db1, float* dW2, float* abar_out,
                                float* adbar_out, float* workspace, int64_t workspace_floats,
                                int fp32_strict, void* stream) {
-  MLCG_REQUIRE(max_pairs == 0 || (Wbar && Wdbar));
-  PairAdjoint adj{Wbar, Wdbar, nullptr, nullptr, nullptr, nullptr, nullptr};
+  return filter_bwd_impl(pos, pair_ij, pair_stride, n_pairs_dev, max_pairs, basis, centers, widths, alpha, num_rbf, rbf_cut_kind, rbf_lo, rbf_hi, conv_cut_kind, conv_lo, conv_hi, act, W1, b1, W2, num_filters, Wbar, Wdbar, dW1, db1, dW2, abar_out, adbar_out, workspace, workspace_floats, fp32_strict, FilterGate{nullptr, 0}, stream);
+}
+
+extern "C" int mlcg_filter_bwd_gated(const float* pos, const int32_t* pair_ij, int64_t pair_stride,
+                               const int32_t* n_pairs_dev, int64_t max_pairs, int basis,
+                               const float* centers, const float* widths, float alpha,
+                               int num_rbf, int rbf_cut_kind, float rbf_lo, float rbf_hi,
+                               int conv_cut_kind, float conv_lo, float conv_hi, int act,
+                               const float* W1, const float* b1, const float* W2,
+                               int num_filters, const float* Wbar, const float* Wdbar,
+                               float* dW1, float* db1, float* dW2, float* abar_out,
+                               float* adbar_out, float* workspace, int64_t workspace_floats,
+                               int fp32_strict, const uint32_t* gate, int gate_want, void* stream) {
+  return filter_bwd_impl(pos, pair_ij, pair_stride, n_pairs_dev, max_pairs, basis, centers, widths, alpha, num_rbf, rbf_cut_kind, rbf_lo, rbf_hi, conv_cut_kind, conv_lo, conv_hi, act, W1, b1, W2, num_filters, Wbar, Wdbar, dW1, db1, dW2, abar_out, adbar_out, workspace, workspace_floats, fp32_strict, FilterGate{gate, gate_want}, stream);
+}
+
+static int filter_bwd_cfconv_impl(const float* pos, const int32_t* pair_ij,
+                                      int64_t pair_stride, const int32_t* n_pairs_dev,
+                                      int64_t max_pairs, int basis, const float* centers,
+                                      const float* widths, float alpha, int num_rbf,
+                                      int rbf_cut_kind, float rbf_lo, float rbf_hi,
+                                      int conv_cut_kind, float conv_lo, float conv_hi, int act,
+                                      const float* W1, const float* b1, const float* W2,
+                                      int num_filters, const float* gagg2, const float* y,
+                                      const float* gagg1, const float* ydot,
+                                      const float* ddot, float* dW1, float* db1, float* dW2,
+                                      float* abar_out, float* adbar_out, float* workspace,
+                                      int64_t workspace_floats, int fp32_strict, const FilterGate& gate, void* stream) {
+  MLCG_REQUIRE(max_pairs == 0 || (gagg2 && y));
+  MLCG_REQUIRE(!gagg1 || ddot);
+  PairAdjoint adj{nullptr, nullptr, gagg2, y, gagg1, gagg1 ? ydot : nullptr, ddot};
   return launch_filter_bwd(pos, pair_ij, pair_stride, n_pairs_dev, max_pairs, basis, centers,
                            widths, alpha, num_rbf, rbf_cut_kind, rbf_lo, rbf_hi, conv_cut_kind,
-                           conv_lo, conv_hi, act, W1, b1, W2, num_filters, adj, false, dW1, db1,
+                           conv_lo, conv_hi, act, W1, b1, W2, num_filters, adj, true, dW1, db1,
                            dW2, abar_out, adbar_out, workspace, workspace_floats,
-                           fp32_strict != 0, stream);
+                           fp32_strict != 0, gate, stream);
 }
 
 extern "C" int mlcg_filter_bwd_cfconv(const float* pos, const int32_t* pair_ij,
@@ -2226,14 +2544,22 @@ extern "C" int mlcg_filter_bwd_cfconv(const float* pos, const int32_t* pair_ij,
                                       const float* ddot, float* dW1, float* db1, float* dW2,
                                       float* abar_out, float* adbar_out, float* workspace,
                                       int64_t workspace_floats, int fp32_strict, void* stream) {
-  MLCG_REQUIRE(max_pairs == 0 || (gagg2 && y));
-  MLCG_REQUIRE(!gagg1 || ddot);
-  PairAdjoint adj{nullptr, nullptr, gagg2, y, gagg1, gagg1 ? ydot : nullptr, ddot};
-  return launch_filter_bwd(pos, pair_ij, pair_stride, n_pairs_dev, max_pairs, basis, centers,
-                           widths, alpha, num_rbf, rbf_cut_kind, rbf_lo, rbf_hi, conv_cut_kind,
-                           conv_lo, conv_hi, act, W1, b1, W2, num_filters, adj, true, dW1, db1,
-                           dW2, abar_out, adbar_out, workspace, workspace_floats,
-                           fp32_strict != 0, stream);
+  return filter_bwd_cfconv_impl(pos, pair_ij, pair_stride, n_pairs_dev, max_pairs, basis, centers, widths, alpha, num_rbf, rbf_cut_kind, rbf_lo, rbf_hi, conv_cut_kind, conv_lo, conv_hi, act, W1, b1, W2, num_filters, gagg2, y, gagg1, ydot, ddot, dW1, db1, dW2, abar_out, adbar_out, workspace, workspace_floats, fp32_strict, FilterGate{nullptr, 0}, stream);
+}
+
+extern "C" int mlcg_filter_bwd_cfconv_gated(const float* pos, const int32_t* pair_ij,
+                                      int64_t pair_stride, const int32_t* n_pairs_dev,
+                                      int64_t max_pairs, int basis, const float* centers,
+                                      const float* widths, float alpha, int num_rbf,
+                                      int rbf_cut_kind, float rbf_lo, float rbf_hi,
+                                      int conv_cut_kind, float conv_lo, float conv_hi, int act,
+                                      const float* W1, const float* b1, const float* W2,
+                                      int num_filters, const float* gagg2, const float* y,
+                                      const float* gagg1, const float* ydot,
+                                      const float* ddot, float* dW1, float* db1, float* dW2,
+                                      float* abar_out, float* adbar_out, float* workspace,
+                                      int64_t workspace_floats, int fp32_strict, const uint32_t* gate, int gate_want, void* stream) {
+  return filter_bwd_cfconv_impl(pos, pair_ij, pair_stride, n_pairs_dev, max_pairs, basis, centers, widths, alpha, num_rbf, rbf_cut_kind, rbf_lo, rbf_hi, conv_cut_kind, conv_lo, conv_hi, act, W1, b1, W2, num_filters, gagg2, y, gagg1, ydot, ddot, dW1, db1, dW2, abar_out, adbar_out, workspace, workspace_floats, fp32_strict, FilterGate{gate, gate_want}, stream);
 }
 
 // ---------------------------------------------------------------------------
@@ -2255,28 +2581,33 @@ constexpr int kRgWaves = 4;
 constexpr int kRgThreads = kRgWaves * MLCG_WAVE;
 constexpr int kRgMaxGroups = 512;
 
-__device__ __forceinline__ void basis_param_derivs(const RbfParams& rp, float cen, float wid,
-                                                   float d, float C, float dC, float& g_c,
-                                                   float& g_w, float& gd_c, float& gd_w) {
+__device__ __forceinline__ float exp_of(float x) { return __expf(x); }
+__device__ __forceinline__ double exp_of(double x) { return exp(x); }
+
+// T: double on the nodes of a table (see rbf_expnormal_fine), else float.
+template <typename T>
+__device__ __forceinline__ void basis_param_derivs(const RbfParams& rp, T cen, T wid, T d, T C,
+                                                   T dC, T& g_c, T& g_w, T& gd_c, T& gd_w) {
   if (rp.basis == 0) {
-    const float c = wid;
-    const float x = d - cen;
-    const float e = __expf(c * x * x);
-    const float q = 2.0f * c * x * C + dC;            // g' = e q
-    g_c = -2.0f * c * x * C * e;                       // dg/dcenter
-    g_w = x * x * C * e;                               // dg/dc
-    gd_c = -e * (2.0f * c * x * q + 2.0f * c * C);     // dg'/dcenter
-    gd_w = e * (x * x * q + 2.0f * x * C);             // dg'/dc
+    const T c = wid;
+    const T x = d - cen;
+    const T e = exp_of(c * x * x);
+    const T q = T(2) * c * x * C + dC;            // g' = e q
+    g_c = T(-2) * c * x * C * e;                   // dg/dcenter
+    g_w = x * x * C * e;                           // dg/dc
+    gd_c = -e * (T(2) * c * x * q + T(2) * c * C);  // dg'/dcenter
+    gd_w = e * (x * x * q + T(2) * x * C);         // dg'/dc
   } else {
-    const float ex = __expf(rp.alpha * (rp.rbf_lo - d));
-    const float u = ex - cen;
-    const float b = wid;
-    const float e = __expf(-b * u * u);
-    const float r = dC + 2.0f * rp.alpha * b * u * ex * C;  // g' = e r
-    g_c = 2.0f * b * u * C * e;
+    const T alpha = rp.alpha;
+    const T ex = exp_of(alpha * (T(rp.rbf_lo) - d));
+    const T u = ex - cen;
+    const T b = wid;
+    const T e = exp_of(-b * u * u);
+    const T r = dC + T(2) * alpha * b * u * ex * C;  // g' = e r
+    g_c = T(2) * b * u * C * e;
     g_w = -u * u * C * e;
-    gd_c = e * (2.0f * b * u * r - 2.0f * rp.alpha * b * ex * C);
-    gd_w = e * (-u * u * r + 2.0f * rp.alpha * u * ex * C);
+    gd_c = e * (T(2) * b * u * r - T(2) * alpha * b * ex * C);
+    gd_w = e * (-u * u * r + T(2) * alpha * u * ex * C);
   }
 }
 
@@ -2284,7 +2615,9 @@ template <int KT>
 __global__ __launch_bounds__(kRgThreads) void rbf_grad_kernel(
     const float* __restrict__ dist, const int32_t* __restrict__ n_pairs_dev, int64_t max_pairs,
     RbfParams rp, const float* __restrict__ W1, const float* __restrict__ abar,
-    const float* __restrict__ adbar, float* __restrict__ partial) {
+    const float* __restrict__ adbar, float* __restrict__ partial, FilterGate gate) {
+  if (gate_closed(gate)) return;
+  const bool at_nodes = gate.words != nullptr && gate.want != 0;
   __shared__ float w1s[kF * (16 * KT + 1)];  // W1 as [f][k], zero past K
   const int K = rp.K;
   const int kr = 16 * KT + 1;
@@ -2338,12 +2671,23 @@ __global__ __launch_bounds__(kRgThreads) void rbf_grad_kernel(
       const float d = dist[p];
       float C, dC;
       mlcg_cutoff(rp.rbf_kind, rp.rbf_lo, rp.rbf_hi, d, C, dC);
+      double C64 = 0.0, dC64 = 0.0;
+      if (at_nodes) cutoff_f64(rp.rbf_kind, rp.rbf_hi, d, C64, dC64);
 #pragma unroll
       for (int kt = 0; kt < KT; ++kt) {
         const int k = 16 * kt + n;
         if (k >= K) continue;
         float g_c, g_w, gd_c, gd_w;
-        basis_param_derivs(rp, cen[kt], wid[kt], d, C, dC, g_c, g_w, gd_c, gd_w);
+        if (at_nodes) {  // uniform
+          double c64, w64, cd64, wd64;
+          basis_param_derivs<double>(rp, cen[kt], wid[kt], d, C64, dC64, c64, w64, cd64, wd64);
+          g_c = (float)c64;
+          g_w = (float)w64;
+          gd_c = (float)cd64;
+          gd_w = (float)wd64;
+        } else {
+          basis_param_derivs<float>(rp, cen[kt], wid[kt], d, C, dC, g_c, g_w, gd_c, gd_w);
+        }
         sc[kt] += gb[kt][i] * g_c + gdb[kt][i] * gd_c;
         sw[kt] += gb[kt][i] * g_w + gdb[kt][i] * gd_w;
       }
@@ -2374,7 +2718,8 @@ __global__ __launch_bounds__(kRgThreads) void rbf_grad_kernel(
 // out[x] (+)= sum over the groups' partials, in group order.
 __global__ void rbf_grad_reduce_kernel(const float* __restrict__ partial, int groups, int kp,
                                        int K, int accumulate, float* __restrict__ dcenters,
-                                       float* __restrict__ dwidths) {
+                                       float* __restrict__ dwidths, FilterGate gate) {
+  if (gate_closed(gate)) return;
   const int x = threadIdx.x;
   if (x >= 2 * kp) return;
   const int which = x / kp, k = x % kp;
@@ -2398,14 +2743,14 @@ extern "C" int64_t mlcg_rbf_param_grad_workspace_floats(int64_t max_pairs, int n
   return (int64_t)rg_groups(max_pairs) * 2 * 16 * ((num_rbf + 15) / 16);
 }
 
-extern "C" int mlcg_rbf_param_grad(const float* dist, const int32_t* n_pairs_dev,
+static int rbf_param_grad_impl(const float* dist, const int32_t* n_pairs_dev,
                                    int64_t max_pairs, int basis, const float* centers,
                                    const float* widths, float alpha, int num_rbf,
                                    int rbf_cut_kind, float rbf_lo, float rbf_hi,
                                    const float* W1, int num_filters, const float* abar,
                                    const float* adbar, int accumulate, float* dcenters,
                                    float* dwidths, float* workspace, int64_t workspace_floats,
-                                   void* stream) {
+                                   const FilterGate& gate, void* stream) {
   if (!valid_params(basis, num_rbf, rbf_cut_kind, 0, 0, num_filters))
     return MLCG_ERR_UNSUPPORTED;
   MLCG_REQUIRE(max_pairs >= 0 && centers && widths && W1 && dcenters && dwidths && workspace);
@@ -2420,7 +2765,7 @@ extern "C" int mlcg_rbf_param_grad(const float* dist, const int32_t* n_pairs_dev
 #define MLCG_RG(KTV)                                                                        \
   case KTV:                                                                                 \
     hipLaunchKernelGGL(rbf_grad_kernel<KTV>, dim3(groups), dim3(kRgThreads), 0, s, dist,   \
-                       n_pairs_dev, max_pairs, rp, W1, abar, adbar, workspace);             \
+                       n_pairs_dev, max_pairs, rp, W1, abar, adbar, workspace, gate);       \
     break;
     MLCG_RG(1)
     MLCG_RG(2)
@@ -2435,6 +2780,28 @@ extern "C" int mlcg_rbf_param_grad(const float* dist, const int32_t* n_pairs_dev
       return MLCG_ERR_UNSUPPORTED;
   }
   hipLaunchKernelGGL(rbf_grad_reduce_kernel, dim3(1), dim3(256), 0, s, workspace, groups,
-                     16 * KT, num_rbf, accumulate, dcenters, dwidths);
+                     16 * KT, num_rbf, accumulate, dcenters, dwidths, gate);
   return mlcg_launch_status();
+}
+
+extern "C" int mlcg_rbf_param_grad(const float* dist, const int32_t* n_pairs_dev,
+                                   int64_t max_pairs, int basis, const float* centers,
+                                   const float* widths, float alpha, int num_rbf,
+                                   int rbf_cut_kind, float rbf_lo, float rbf_hi,
+                                   const float* W1, int num_filters, const float* abar,
+                                   const float* adbar, int accumulate, float* dcenters,
+                                   float* dwidths, float* workspace, int64_t workspace_floats,
+                                   void* stream) {
+  return rbf_param_grad_impl(dist, n_pairs_dev, max_pairs, basis, centers, widths, alpha, num_rbf, rbf_cut_kind, rbf_lo, rbf_hi, W1, num_filters, abar, adbar, accumulate, dcenters, dwidths, workspace, workspace_floats, FilterGate{nullptr, 0}, stream);
+}
+
+extern "C" int mlcg_rbf_param_grad_gated(const float* dist, const int32_t* n_pairs_dev,
+                                   int64_t max_pairs, int basis, const float* centers,
+                                   const float* widths, float alpha, int num_rbf,
+                                   int rbf_cut_kind, float rbf_lo, float rbf_hi,
+                                   const float* W1, int num_filters, const float* abar,
+                                   const float* adbar, int accumulate, float* dcenters,
+                                   float* dwidths, float* workspace, int64_t workspace_floats,
+                                   const uint32_t* gate, int gate_want, void* stream) {
+  return rbf_param_grad_impl(dist, n_pairs_dev, max_pairs, basis, centers, widths, alpha, num_rbf, rbf_cut_kind, rbf_lo, rbf_hi, W1, num_filters, abar, adbar, accumulate, dcenters, dwidths, workspace, workspace_floats, FilterGate{gate, gate_want}, stream);
 }

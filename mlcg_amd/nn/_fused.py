@@ -69,6 +69,13 @@ class FusedSpec:
     f16: bool = False
     basis_trainable: bool = False  # Params.basis carries (centers, widths)
     strict_fp32: bool = False  # filter forward on the fp32 MFMA throughout
+    # the filters' distance grid: its shape (ops.filter_grid_shape of filt, None
+    # without one) and its tensors per device index
+    grid_shape: Optional[tuple] = None
+    grids: dict = field(default_factory=dict)
+
+    def __post_init__(self):
+        self.grid_shape = ops.filter_grid_shape(self.filt)
 
 
 @dataclass
@@ -120,6 +127,11 @@ class State:
     graph: ops.PairGraph
     filt: Optional[ops.FilterSpec] = None
     dist: Optional[torch.Tensor] = None
+    # filters through a table: the grid, the pairs in stencil order, the
+    # blocks' gate words
+    grid: Optional[ops.FilterGrid] = None
+    bins: Optional[ops.PairBins] = None
+    gates: Optional[torch.Tensor] = None
     W: List[torch.Tensor] = field(default_factory=list)
     Wd: List[torch.Tensor] = field(default_factory=list)
     x: List[torch.Tensor] = field(default_factory=list)    # block inputs
@@ -242,13 +254,101 @@ def _lin_dact2_lin(x, A, z, s, act, e, f, B, imgs=(None, None)):
     return v, ops.node_linear(v, B, transpose=True)
 
 
+_SIDE_STREAMS = {}
+
+
+def _side_stream(main: torch.cuda.Stream) -> torch.cuda.Stream:
+    """The second stream (default priority) that goes with a caller's stream."""
+    key = (main.device.index, main.cuda_stream)
+    if key not in _SIDE_STREAMS:
+        _SIDE_STREAMS[key] = torch.cuda.Stream(device=main.device)
+    return _SIDE_STREAMS[key]
+
+
+# None: by the rule of _table_pays; True / False: wherever there is a grid / never.
+_FILTER_TABLE: Optional[bool] = None
+
+
+def _table_pays(spec: FusedSpec, pairs: int, nodes: int, reverse: bool) -> bool:
+    """Whether the filters go through a table (csrc/filter_table.hip) instead of
+    one network evaluation per pair.  The table costs its nodes and the ordering
+    of the pairs once per call and, with a reverse sweep, some launches per
+    block; it saves time per pair and block.  Measured (device us, 35-bead
+    chains, Gaussian basis, 2561 nodes, direct / table): energies and forces,
+    3 blocks 42 k pairs 274 / 292, 84 k 393 / 375, 1 block 84 k 142 / 178;
+    force-matching step, 3 blocks 42 k 775 / 805, 84 k 1130 / 1043, 1 block 84 k
+    396 / 411; exponential-normal basis (7681 nodes), 2 blocks, trainable, 27 k
+    687 / 702, 55 k 918 / 772 (the gradient of the basis is then taken at the
+    nodes too, which saves three times as much a pair)."""
+    work = pairs * spec.num_blocks
+    if not reverse:
+        return work >= 48 * nodes + 64_000
+    return work * (3 if spec.basis_trainable else 1) >= 32 * nodes + 22_000 * spec.num_blocks
+
+
+def _table_grid(spec: FusedSpec, filt, graph: ops.PairGraph, pos: torch.Tensor, reverse: bool):
+    """The distance grid of this call's filters, or None where each pair's
+    filter is evaluated directly: too few pairs, strict fp32 filters, a filter
+    without a grid (ops.filter_grid_shape), or a stream capture that no call
+    has preceded (the grid's tensors come from the host)."""
+    shape = spec.grid_shape
+    if shape is None or spec.strict_fp32 or not pos.is_cuda or not graph.pair_capacity:
+        return None
+    if not (_table_pays(spec, graph.pair_capacity, shape[0], reverse) if _FILTER_TABLE is None
+            else _FILTER_TABLE and spec.num_blocks):
+        return None
+    grid = spec.grids.get(pos.device.index)
+    if grid is None and not torch.cuda.is_current_stream_capturing():
+        grid = spec.grids[pos.device.index] = ops.filter_grid(filt, pos.device)
+    return grid
+
+
+def _start_tables(spec: FusedSpec, P: Params, st: "State", pos, graph) -> torch.Tensor:
+    """The blocks' filter tables (returned) and their gate words, on the side
+    stream while the caller's stream orders the pairs: the tables depend on the
+    weights alone.  Their buffers belong to the caller's stream, which waits for
+    the side stream before it goes on."""
+    main = torch.cuda.current_stream(pos.device)
+    side = _side_stream(main)
+    out = ops.filter_table_buffers(st.grid, len(P.blocks))
+    side.wait_stream(main)
+    with torch.cuda.stream(side):
+        ops.filter_tables(st.grid, st.filt, [(bp.W1, bp.b1, bp.W2) for bp in P.blocks], out=out)
+    st.bins = ops.pair_bins(pos, graph, st.grid)
+    st.dist = st.bins.dist
+    main.wait_stream(side)
+    st.gates = out[1]
+    return out[0]
+
+
+def _block_filters(spec: FusedSpec, P: Params, st: "State", pos, graph, tables, k: int,
+                   out=None):
+    """(W, Wd) of block k, from its table where that serves."""
+    bp = P.blocks[k]
+    if st.grid is None:
+        W, Wd, dist = ops.filter_fwd(pos, graph, st.filt, bp.W1, bp.b1, bp.W2, f16=spec.f16,
+                                     want_dist=(k == 0), strict_fp32=spec.strict_fp32, out=out)
+        if k == 0:
+            st.dist = dist
+        return W, Wd
+    if out is None:
+        dt = torch.float16 if spec.f16 else torch.float32
+        shape = (graph.pair_capacity, ops.NUM_FILTERS)
+        out = (torch.empty(shape, dtype=dt, device=pos.device),
+               torch.empty(shape, dtype=dt, device=pos.device))
+    ops.filter_table_rows(st.grid, st.bins, graph, tables[k], st.gates[k], out)
+    ops.filter_fwd(pos, graph, st.filt, bp.W1, bp.b1, bp.W2, f16=spec.f16, want_dist=False,
+                   out=out, gate=st.gates[k])
+    return out
+
+
 # Filter forwards of blocks 1.. on the side stream (MLCG_FILTER_AHEAD=0 keeps
 # them in block order on the caller's stream).
 _FILTER_AHEAD = os.environ.get("MLCG_FILTER_AHEAD", "1") != "0"
 
 
-def _filters_ahead(spec: FusedSpec, P: Params, pos: torch.Tensor, graph: ops.PairGraph,
-                   filt) -> dict:
+def _filters_ahead(spec: FusedSpec, P: Params, st: "State", pos: torch.Tensor,
+                   graph: ops.PairGraph, tables) -> dict:
     """Issues the filter forwards of blocks 1.. on the side stream at the start
     of the forward: they depend only on the pair distances and the block's
     filter weights, not on node features, so they run beside block 0's node
@@ -259,10 +359,7 @@ def _filters_ahead(spec: FusedSpec, P: Params, pos: torch.Tensor, graph: ops.Pai
     if not (_FILTER_AHEAD and pos.is_cuda and len(P.blocks) > 1):
         return {}
     main = torch.cuda.current_stream(pos.device)
-    key = (pos.device.index, main.cuda_stream)
-    if key not in _SIDE_STREAMS:
-        _SIDE_STREAMS[key] = torch.cuda.Stream(device=pos.device)
-    side = _SIDE_STREAMS[key]
+    side = _side_stream(main)
     cap = graph.pair_capacity
     dt = torch.float16 if spec.f16 else torch.float32
     outs = {k: (torch.empty(cap, ops.NUM_FILTERS, dtype=dt, device=pos.device),
@@ -272,10 +369,7 @@ def _filters_ahead(spec: FusedSpec, P: Params, pos: torch.Tensor, graph: ops.Pai
     ahead = {}
     with torch.cuda.stream(side):
         for k in range(1, len(P.blocks)):
-            bp = P.blocks[k]
-            W, Wd, _ = ops.filter_fwd(pos, graph, filt, bp.W1, bp.b1, bp.W2, f16=spec.f16,
-                                      want_dist=False, strict_fp32=spec.strict_fp32,
-                                      out=outs[k])
+            W, Wd = _block_filters(spec, P, st, pos, graph, tables, k, out=outs[k])
             ev = torch.cuda.Event()
             ev.record(side)
             ahead[k] = (W, Wd, ev)
@@ -311,8 +405,10 @@ def _wi(st: "State", k: int, name: str, transpose: bool) -> Optional[torch.Tenso
 
 def forward(spec: FusedSpec, P: Params, pos: torch.Tensor, types: torch.Tensor,
             graph: ops.PairGraph, save: bool = True,
-            rev_seed: Optional[torch.Tensor] = None) -> Tuple[torch.Tensor, State]:
-    """Energies [B] and the saved state.  With rev_seed, the output network's
+            rev_seed: Optional[torch.Tensor] = None,
+            reverse: bool = True) -> Tuple[torch.Tensor, State]:
+    """Energies [B] and the saved state; reverse: a parameter sweep (reverse2) is
+    likely to follow, which only the choice of the filters' route looks at.  With rev_seed, the output network's
     kernel also forms the adjoint a following reverse1(seed=rev_seed) starts
     from."""
     st = State(pos=pos, types=types, graph=graph, filt=filter_spec(spec, P))
@@ -326,18 +422,17 @@ def forward(spec: FusedSpec, P: Params, pos: torch.Tensor, types: torch.Tensor,
     # the weight images before the side stream's filter forwards, which would
     # otherwise hold every CU while this short launch waits for one
     st.wimg = _weight_images(P, x, transposed=save)
-    ahead = _filters_ahead(spec, P, pos, graph, st.filt)
+    st.grid = _table_grid(spec, st.filt, graph, pos, reverse)
+    tables = None
+    if st.grid is not None:
+        tables = _start_tables(spec, P, st, pos, graph)
+    ahead = _filters_ahead(spec, P, st, pos, graph, tables)
     for k, bp in enumerate(P.blocks):
         if k in ahead:
             W, Wd, done = ahead[k]
-            dist = None
         else:
-            W, Wd, dist = ops.filter_fwd(pos, graph, st.filt, bp.W1, bp.b1, bp.W2,
-                                         f16=spec.f16, want_dist=(k == 0),
-                                         strict_fp32=spec.strict_fp32)
+            W, Wd = _block_filters(spec, P, st, pos, graph, tables, k)
             done = None
-        if k == 0:
-            st.dist = dist
         y = ops.node_linear(x, bp.A1, w_image=_wi(st, k, "A1", False))
         if done is not None:
             torch.cuda.current_stream(pos.device).wait_event(done)
@@ -538,7 +633,6 @@ def reverse2(spec: FusedSpec, P: Params, st: State, tw: Optional[torch.Tensor],
     return _blocks_reverse2(spec, P, st, tw, hbar2, g_out_w, g_out_b)
 
 
-_SIDE_STREAMS = {}
 # Weight-gradient reductions of reverse2 on the side stream (False, the
 # default, runs them in order on the caller's stream; results are the same bit
 # for bit).  Measured on config 2: in order, the eager step's device time is
@@ -560,10 +654,7 @@ class _SideStream:
 
     def __init__(self, device: torch.device):
         self.main = torch.cuda.current_stream(device)
-        key = (device.index, self.main.cuda_stream)
-        if key not in _SIDE_STREAMS:
-            _SIDE_STREAMS[key] = torch.cuda.Stream(device=device)
-        self.side = _SIDE_STREAMS[key]
+        self.side = _side_stream(self.main)
         self.held = []
 
     def run(self, fn, *inputs):
@@ -593,6 +684,36 @@ def _node_tmm_batch(probs, rows, device):
     if all(ok(t) for pr in probs for t in pr[:4]):
         return ops.node_tmm_batch(probs, rows, device)
     return [ops.node_tmm(a1, b1, a2, b2, colsum=cs) for a1, b1, a2, b2, cs in probs]
+
+
+def _filter_reverse(spec, st, bp, k, gagg2, g1, yd, dd, g_basis):
+    """(gW1, gb1, gW2, g_basis) of block k's filter from the node adjoints; the
+    basis parameters are shared by all blocks, so g_basis accumulates."""
+    graph, filt, train_basis = st.graph, st.filt, spec.basis_trainable
+    if st.grid is None:
+        res = ops.filter_bwd_cfconv(st.pos, graph, filt, bp.W1, bp.b1, bp.W2, gagg2, st.y[k], g1,
+                                    yd, dd, pair_adjoints=train_basis,
+                                    strict_fp32=spec.strict_fp32)
+        if train_basis:
+            g_basis = ops.rbf_param_grad(st.dist, graph, filt, bp.W1, res[3], res[4],
+                                         out=g_basis)
+        return (*res[:3], g_basis)
+    # through the table's nodes where it serves, else pair by pair: of each
+    # couple of launches one returns at once
+    grid, gate = st.grid, st.gates[k]
+    wbar, wdbar = ops.filter_table_reverse(grid, st.bins, graph, gagg2, st.y[k], g1, yd, dd, gate)
+    at_nodes = ops.filter_bwd(grid.pos, grid.graph, filt, bp.W1, bp.b1, bp.W2, wbar, wdbar,
+                              pair_adjoints=train_basis, gate=gate)
+    by_pair = ops.filter_bwd_cfconv(st.pos, graph, filt, bp.W1, bp.b1, bp.W2, gagg2, st.y[k], g1,
+                                    yd, dd, pair_adjoints=train_basis, gate=gate,
+                                    out=at_nodes[:3])
+    if train_basis:
+        first = g_basis is None
+        g_basis = ops.rbf_param_grad(grid.dist, grid.graph, filt, bp.W1, *at_nodes[3:],
+                                     out=g_basis, gate=gate, gate_want=1)
+        ops.rbf_param_grad(st.dist, graph, filt, bp.W1, *by_pair[3:], out=g_basis,
+                           accumulate=not first, gate=gate, gate_want=0)
+    return (*at_nodes[:3], g_basis)
 
 
 def _blocks_reverse2(spec, P, st, tw, xbar2, g_out_w, g_out_b):
@@ -636,14 +757,7 @@ def _blocks_reverse2(spec, P, st, tw, xbar2, g_out_w, g_out_b):
             lambda: _node_tmm_batch(probs, N, st.pos.device), *held)
         xbar2 = ops.node_linear(ybar2, bp.A1, transpose=True, residual=xbar2,
                                 w_image=_wi(st, k, "A1", True))
-        res = ops.filter_bwd_cfconv(st.pos, graph, st.filt, bp.W1, bp.b1, bp.W2, gagg2,
-                                    st.y[k], g1, yd, dd, pair_adjoints=spec.basis_trainable,
-                                    strict_fp32=spec.strict_fp32)
-        gW1, gb1, gW2 = res[:3]
-        if spec.basis_trainable:
-            # basis parameters are shared by all blocks: accumulate
-            g_basis = ops.rbf_param_grad(st.dist, graph, st.filt, bp.W1, res[3], res[4],
-                                         out=g_basis)
+        gW1, gb1, gW2, g_basis = _filter_reverse(spec, st, bp, k, gagg2, g1, yd, dd, g_basis)
         g_blocks[k] = [gW1, gb1, gW2, gA1, gA2, gc2, gA3, gc3]
     if P.emb.shape[0] <= 128 and P.emb.shape[1] == 128 and st.types.dtype == torch.int64:
         # fixed summation order; an out-of-table type raises a numerics flag
@@ -704,7 +818,8 @@ class EnergyForces(torch.autograd.Function):
     def forward(ctx, spec, pos, types, batch, graph, training, *flat):
         P = Params.unflat(spec, list(flat))
         ones = _ones(pos.shape[0], pos.device)
-        E, st = forward(spec, P, pos, types, graph, save=True, rev_seed=ones)
+        E, st = forward(spec, P, pos, types, graph, save=True, rev_seed=ones,
+                        reverse=bool(training))
         F = reverse1(spec, P, st, ones, keep_adjoints=bool(training))
         if training:
             ctx.spec, ctx.P, ctx.st, ctx.batch = spec, P, st, batch

@@ -9,6 +9,7 @@ torch's caching allocator and launches on torch's current stream.
 from __future__ import annotations
 
 import ctypes
+import math
 from dataclasses import dataclass
 from typing import List, Optional, Tuple
 
@@ -859,17 +860,29 @@ BASIS_GAUSSIAN, BASIS_EXPNORMAL = 0, 1
 FILTER_FP32, FILTER_FP16, FILTER_FP32_STRICT = 0, 1, 2
 
 
+def _call_gated(name: str, args: tuple, gate: Optional[torch.Tensor], want: int, dev) -> None:
+    """Entry point `name`, or with `gate` its gated form: the launch does its
+    work only if the table serves (want 1) or does not (want 0)."""
+    if gate is None:
+        call(name, *args, stream_handle(dev))
+    else:
+        call(name + "_gated", *args, ptr(gate), want, stream_handle(dev))
+
+
 def filter_fwd(pos: torch.Tensor, graph: PairGraph, spec: FilterSpec, W1: torch.Tensor,
                b1: torch.Tensor, W2: torch.Tensor, f16: bool = False,
                want_dist: bool = True, strict_fp32: bool = False,
                out: Optional[Tuple[torch.Tensor, torch.Tensor]] = None,
+               gate: Optional[torch.Tensor] = None,
                ) -> Tuple[torch.Tensor, torch.Tensor, Optional[torch.Tensor]]:
     """W [P, F], dW/dd [P, F] (fp32, or fp16 when f16) and distances [P].
     fp32 results come from split-fp16 products (about 22 significant bits
     per operand, fp32 accumulation) unless strict_fp32 asks for the fp32
     MFMA throughout (mlcg_filter_fwd's FP32_STRICT mode).  `out` = (W, Wd)
     written in place of new tensors (a caller that launches on another
-    stream allocates them on the stream that consumes them)."""
+    stream allocates them on the stream that consumes them).  With `gate` (a
+    block's gate words, filter_tables) the kernel returns at once when the
+    block's table serves."""
     pos = _validate_pos(pos)
     F = W1.shape[0]
     _check(F == NUM_FILTERS, lambda: f"num_filters must be {NUM_FILTERS} for the HIP filter kernel")
@@ -887,12 +900,13 @@ def filter_fwd(pos: torch.Tensor, graph: PairGraph, spec: FilterSpec, W1: torch.
                "filter_fwd out tensors must be contiguous [pair_capacity, 128] of the result dtype")
     dist = torch.empty(cap, dtype=torch.float32, device=pos.device) if want_dist else None
     W1c, b1c, W2c = (t.detach().float().contiguous() for t in (W1, b1, W2))
-    call("mlcg_filter_fwd", ptr(pos), ptr(graph.pair_ij), cap, ptr(graph.n_pairs_dev), cap,
-         *spec.basis_args(), spec.num_rbf, spec.rbf_cut_kind, spec.rbf_lo,
-         spec.rbf_hi, spec.conv_cut_kind, spec.conv_lo, spec.conv_hi, spec.act, ptr(W1c),
-         ptr(b1c), ptr(W2c), F,
-         FILTER_FP16 if f16 else (FILTER_FP32_STRICT if strict_fp32 else FILTER_FP32),
-         ptr(W), ptr(Wd), ptr(dist), stream_handle(pos.device))
+    args = (ptr(pos), ptr(graph.pair_ij), cap, ptr(graph.n_pairs_dev), cap,
+            *spec.basis_args(), spec.num_rbf, spec.rbf_cut_kind, spec.rbf_lo,
+            spec.rbf_hi, spec.conv_cut_kind, spec.conv_lo, spec.conv_hi, spec.act, ptr(W1c),
+            ptr(b1c), ptr(W2c), F,
+            FILTER_FP16 if f16 else (FILTER_FP32_STRICT if strict_fp32 else FILTER_FP32),
+            ptr(W), ptr(Wd), ptr(dist))
+    _call_gated("mlcg_filter_fwd", args, gate, 0, pos.device)
     return W, Wd, dist
 
 
@@ -940,14 +954,23 @@ def _pair_adjoint_outputs(want: bool, cap: int, F: int, dev):
             torch.empty(cap, F, dtype=torch.float32, device=dev))
 
 
+def _filter_grads(F: int, K: int, dev):
+    return (torch.empty(F, K, dtype=torch.float32, device=dev),
+            torch.empty(F, dtype=torch.float32, device=dev),
+            torch.empty(F, F, dtype=torch.float32, device=dev))
+
+
 def filter_bwd(pos: torch.Tensor, graph: PairGraph, spec: FilterSpec, W1: torch.Tensor,
                b1: torch.Tensor, W2: torch.Tensor, Wbar: torch.Tensor,
-               Wdbar: torch.Tensor, pair_adjoints: bool = False, strict_fp32: bool = False):
+               Wdbar: torch.Tensor, pair_adjoints: bool = False, strict_fp32: bool = False,
+               gate: Optional[torch.Tensor] = None, out=None):
     """Gradients (dW1 [F, K], db1 [F], dW2 [F, F]) of <Wbar, W> + <Wdbar, dW/dd>;
     with pair_adjoints also the first-layer pair adjoints (abar, adbar)
     [P, F] that rbf_param_grad consumes.  strict_fp32 runs every product on
     the fp32 MFMA instead of split-fp16 products (which hold activations and
-    derivatives below 2^19, see check_numerics)."""
+    derivatives below 2^19, see check_numerics).  With `gate` the launch writes
+    its results, into `out` = (dW1, db1, dW2) when given, only if the block's
+    table serves."""
     pos = _validate_pos(pos)
     F = W1.shape[0]
     K = spec.num_rbf
@@ -958,16 +981,15 @@ def filter_bwd(pos: torch.Tensor, graph: PairGraph, spec: FilterSpec, W1: torch.
     nws = int(_lib.load().mlcg_filter_bwd_workspace_floats(cap, K))
     _check(nws > 0, lambda: f"num_rbf={K} is not supported by the filter backward")
     ws = torch.empty(nws, dtype=torch.float32, device=dev)
-    dW1 = torch.empty(F, K, dtype=torch.float32, device=dev)
-    db1 = torch.empty(F, dtype=torch.float32, device=dev)
-    dW2 = torch.empty(F, F, dtype=torch.float32, device=dev)
+    dW1, db1, dW2 = _filter_grads(F, K, dev) if out is None else out
     W1c, b1c, W2c = (t.detach().float().contiguous() for t in (W1, b1, W2))
     ab, adb = _pair_adjoint_outputs(pair_adjoints, cap, F, dev)
-    call("mlcg_filter_bwd", ptr(pos), ptr(graph.pair_ij), cap, ptr(graph.n_pairs_dev), cap,
-         *spec.basis_args(), K, spec.rbf_cut_kind, spec.rbf_lo, spec.rbf_hi,
-         spec.conv_cut_kind, spec.conv_lo, spec.conv_hi, spec.act, ptr(W1c), ptr(b1c),
-         ptr(W2c), F, ptr(Wbar.contiguous()), ptr(Wdbar.contiguous()), ptr(dW1), ptr(db1),
-         ptr(dW2), ptr(ab), ptr(adb), ptr(ws), nws, int(strict_fp32), stream_handle(dev))
+    args = (ptr(pos), ptr(graph.pair_ij), cap, ptr(graph.n_pairs_dev), cap,
+            *spec.basis_args(), K, spec.rbf_cut_kind, spec.rbf_lo, spec.rbf_hi,
+            spec.conv_cut_kind, spec.conv_lo, spec.conv_hi, spec.act, ptr(W1c), ptr(b1c),
+            ptr(W2c), F, ptr(Wbar.contiguous()), ptr(Wdbar.contiguous()), ptr(dW1), ptr(db1),
+            ptr(dW2), ptr(ab), ptr(adb), ptr(ws), nws, int(strict_fp32))
+    _call_gated("mlcg_filter_bwd", args, gate, 1, dev)
     if pair_adjoints:
         return dW1, db1, dW2, ab, adb
     return dW1, db1, dW2
@@ -978,10 +1000,12 @@ def filter_bwd_cfconv(pos: torch.Tensor, graph: PairGraph, spec: FilterSpec,
                       gagg2: torch.Tensor, y: torch.Tensor, gagg1: Optional[torch.Tensor],
                       ydot: Optional[torch.Tensor],
                       ddot: Optional[torch.Tensor], pair_adjoints: bool = False,
-                      strict_fp32: bool = False):
+                      strict_fp32: bool = False, gate: Optional[torch.Tensor] = None,
+                      out=None):
     """filter_bwd with Wbar_p = g2_i y_j + g2_j y_i + g1_i yd_j + g1_j yd_i and
     Wdbar_p = dd_p (g1_i y_j + g1_j y_i) formed in the kernel from node arrays
-    (pair_adjoints and strict_fp32 as in filter_bwd)."""
+    (pair_adjoints, strict_fp32 and out as in filter_bwd).  With `gate` the launch
+    writes its results only if the block's table does not serve."""
     pos = _validate_pos(pos)
     F = W1.shape[0]
     K = spec.num_rbf
@@ -990,18 +1014,16 @@ def filter_bwd_cfconv(pos: torch.Tensor, graph: PairGraph, spec: FilterSpec,
     nws = int(_lib.load().mlcg_filter_bwd_workspace_floats(cap, K))
     _check(nws > 0, lambda: f"num_rbf={K} is not supported by the filter backward")
     ws = torch.empty(nws, dtype=torch.float32, device=dev)
-    dW1 = torch.empty(F, K, dtype=torch.float32, device=dev)
-    db1 = torch.empty(F, dtype=torch.float32, device=dev)
-    dW2 = torch.empty(F, F, dtype=torch.float32, device=dev)
+    dW1, db1, dW2 = _filter_grads(F, K, dev) if out is None else out
     W1c, b1c, W2c = (t.detach().float().contiguous() for t in (W1, b1, W2))
     c = lambda t: None if t is None else t.contiguous()  # noqa: E731
     ab, adb = _pair_adjoint_outputs(pair_adjoints, cap, F, dev)
-    call("mlcg_filter_bwd_cfconv", ptr(pos), ptr(graph.pair_ij), cap, ptr(graph.n_pairs_dev),
-         cap, *spec.basis_args(), K, spec.rbf_cut_kind, spec.rbf_lo, spec.rbf_hi,
-         spec.conv_cut_kind, spec.conv_lo, spec.conv_hi, spec.act, ptr(W1c), ptr(b1c),
-         ptr(W2c), F, ptr(c(gagg2)), ptr(c(y)), ptr(c(gagg1)), ptr(c(ydot)), ptr(ddot),
-         ptr(dW1), ptr(db1), ptr(dW2), ptr(ab), ptr(adb), ptr(ws), nws, int(strict_fp32),
-         stream_handle(dev))
+    args = (ptr(pos), ptr(graph.pair_ij), cap, ptr(graph.n_pairs_dev),
+            cap, *spec.basis_args(), K, spec.rbf_cut_kind, spec.rbf_lo, spec.rbf_hi,
+            spec.conv_cut_kind, spec.conv_lo, spec.conv_hi, spec.act, ptr(W1c), ptr(b1c),
+            ptr(W2c), F, ptr(c(gagg2)), ptr(c(y)), ptr(c(gagg1)), ptr(c(ydot)), ptr(ddot),
+            ptr(dW1), ptr(db1), ptr(dW2), ptr(ab), ptr(adb), ptr(ws), nws, int(strict_fp32))
+    _call_gated("mlcg_filter_bwd_cfconv", args, gate, 0, dev)
     if pair_adjoints:
         return dW1, db1, dW2, ab, adb
     return dW1, db1, dW2
@@ -1009,9 +1031,13 @@ def filter_bwd_cfconv(pos: torch.Tensor, graph: PairGraph, spec: FilterSpec,
 
 def rbf_param_grad(dist: torch.Tensor, graph: PairGraph, spec: FilterSpec, W1: torch.Tensor,
                    abar: torch.Tensor, adbar: torch.Tensor,
-                   out: Optional[Tuple[torch.Tensor, torch.Tensor]] = None):
+                   out: Optional[Tuple[torch.Tensor, torch.Tensor]] = None,
+                   accumulate: Optional[bool] = None, gate: Optional[torch.Tensor] = None,
+                   gate_want: int = 0):
     """(dcenters [K], dwidths [K]) of the basis from the first-layer pair
-    adjoints (mlcg_rbf_param_grad); added into `out` when given."""
+    adjoints (mlcg_rbf_param_grad); added into `out` when given (accumulate:
+    False stores into it instead).  With `gate` the launch does its work only
+    if the block's table serves (gate_want 1) or does not (0)."""
     require_device(dist, abar, adbar)
     K = spec.num_rbf
     cap = graph.pair_capacity
@@ -1021,16 +1047,184 @@ def rbf_param_grad(dist: torch.Tensor, graph: PairGraph, spec: FilterSpec, W1: t
     nws = int(_lib.load().mlcg_rbf_param_grad_workspace_floats(cap, K))
     _check(nws > 0, lambda: f"num_rbf={K} is not supported")
     ws = torch.empty(nws, dtype=torch.float32, device=dev)
-    accumulate = out is not None
+    accumulate = out is not None if accumulate is None else accumulate
     if out is None:
         out = (torch.empty(K, dtype=torch.float32, device=dev),
                torch.empty(K, dtype=torch.float32, device=dev))
     W1c = W1.detach().float().contiguous()
-    call("mlcg_rbf_param_grad", ptr(dist), ptr(graph.n_pairs_dev), cap, *spec.basis_args(), K,
-         spec.rbf_cut_kind, spec.rbf_lo, spec.rbf_hi, ptr(W1c), NUM_FILTERS,
-         ptr(abar.contiguous()), ptr(adbar.contiguous()), int(accumulate), ptr(out[0]),
-         ptr(out[1]), ptr(ws), nws, stream_handle(dev))
+    args = (ptr(dist), ptr(graph.n_pairs_dev), cap, *spec.basis_args(), K,
+            spec.rbf_cut_kind, spec.rbf_lo, spec.rbf_hi, ptr(W1c), NUM_FILTERS,
+            ptr(abar.contiguous()), ptr(adbar.contiguous()), int(accumulate), ptr(out[0]),
+            ptr(out[1]), ptr(ws), nws)
+    _call_gated("mlcg_rbf_param_grad", args, gate, gate_want, dev)
     return out
+
+
+# --------------------------------------------------------------------------
+# Filter through a table over the distance (csrc/filter_table.hip)
+
+GATE_WORDS = 12
+TABLE_MAX_NODES = 8192 + 3
+
+
+@dataclass
+class FilterGrid:
+    """Distance grid 0, h, .., (nodes - 1) h of a filter table over [0, rc], all
+    exact in float32.  `cut`: distance from which the filter is exactly zero.
+    pos / graph describe the nodes as pairs, for the kernels that take pairs;
+    dist holds their distances."""
+
+    nodes: int
+    h: float
+    rc: float
+    cut: float
+    pos: torch.Tensor
+    dist: torch.Tensor
+    graph: PairGraph
+
+
+def filter_grid_shape(spec: FilterSpec) -> Optional[Tuple[int, float, float, float]]:
+    """(nodes, h, rc, cut) of the table grid for this filter, or None when it
+    has no table: an envelope with a kink inside (0, rc), or a grid past
+    TABLE_MAX_NODES.  h is, down to 11 significant bits (then k h is exact),
+    the smallest width of the basis functions over 52 (Gaussian) or over 32
+    (exponential-normal, whose functions widen from zero distance on): the
+    check then passes with a margin of 30 and 4, i.e. for filters 2.4 and 1.4
+    times as sharp as their basis."""
+    rc = float(spec.rbf_hi)
+    K = int(spec.num_rbf)
+    if not (0.0 < rc < 1e30) or K < 2:
+        return None
+    if spec.rbf_cut_kind == 1 and spec.rbf_lo != 0.0:
+        return None
+    if spec.conv_cut_kind == 1 and (spec.conv_lo != 0.0 or spec.conv_hi < rc):
+        return None
+    if spec.basis == BASIS_GAUSSIAN:
+        fine = rc / (K - 1) / 52.0
+    else:
+        if not spec.alpha > 0.0:
+            return None
+        fine = math.sqrt(2.0) / (K * spec.alpha) / 32.0
+    ulp = 2.0 ** (math.floor(math.log2(fine)) - 10)
+    h = math.floor(fine / ulp) * ulp
+    nodes = int(math.floor(rc / h)) + 1
+    if nodes < 64 or nodes > TABLE_MAX_NODES:
+        return None
+    return nodes, h, rc, float(spec.conv_hi) if spec.conv_cut_kind == 1 else 3.0e38
+
+
+def filter_grid(spec: FilterSpec, device) -> Optional[FilterGrid]:
+    """The grid with its device tensors (made on the host and copied, with one
+    synchronisation, so that any stream may use them)."""
+    shape = filter_grid_shape(spec)
+    if shape is None:
+        return None
+    nodes, h, rc, cut = shape
+    dist = torch.arange(nodes, dtype=torch.float32) * h
+    pos = torch.zeros(nodes, 3)
+    pos[:, 0] = dist
+    pair_ij = torch.zeros(2, nodes, dtype=torch.int32)
+    pair_ij[1] = torch.arange(nodes, dtype=torch.int32)
+    count = torch.full((1,), nodes, dtype=torch.int32)
+    pos, dist, pair_ij, count = (t.to(device) for t in (pos, dist, pair_ij, count))
+    torch.cuda.current_stream(device).synchronize()
+    graph = PairGraph(edge_index=None, rowptr=None, col=None, pair_ij=pair_ij, pairptr=count,
+                      eid2pair=None, frame_ptr=None, num_nodes=0, num_edges=2 * nodes,
+                      num_pairs=nodes)
+    return FilterGrid(nodes=nodes, h=h, rc=rc, cut=cut, pos=pos, dist=dist, graph=graph)
+
+
+@dataclass
+class PairBins:
+    """Pairs in the order of their interpolation stencil (pair_bins)."""
+
+    records: torch.Tensor  # [P, 4] int32: pair, i, j, distance bits
+    start: torch.Tensor    # [nodes - 2] int32: first record of every stencil
+    runs: torch.Tensor     # [nodes - 2] int32: first run of every stencil
+    dist: torch.Tensor     # [P] float32, in pair order
+
+
+def pair_bins(pos: torch.Tensor, graph: PairGraph, grid: FilterGrid) -> PairBins:
+    pos = _validate_pos(pos)
+    cap = graph.pair_capacity
+    dev = pos.device
+    nws = int(_lib.load().mlcg_pair_bins_workspace_ints(cap, grid.nodes))
+    _check(nws > 0, lambda: f"pair_bins: unsupported shape (pairs {cap}, nodes {grid.nodes})")
+    ws = torch.empty(nws, dtype=torch.int32, device=dev)
+    dist = torch.empty(cap, dtype=torch.float32, device=dev)
+    start, runs = torch.empty(2, grid.nodes - 2, dtype=torch.int32, device=dev)
+    records = torch.empty(cap, 4, dtype=torch.int32, device=dev)
+    call("mlcg_pair_bins", ptr(pos), ptr(graph.pair_ij), cap, ptr(graph.n_pairs_dev), cap,
+         grid.h, grid.nodes, ptr(dist), ptr(start), ptr(runs), ptr(records), ptr(ws), nws,
+         stream_handle(dev))
+    return PairBins(records, start, runs, dist)
+
+
+def filter_table_buffers(grid: FilterGrid, blocks: int) -> Tuple[torch.Tensor, torch.Tensor]:
+    """(tables [L, 4, nodes + 1, F], gates [L, GATE_WORDS] cleared) for
+    filter_tables."""
+    dev = grid.pos.device
+    return (torch.empty(blocks, 4, grid.nodes + 1, NUM_FILTERS, dtype=torch.float32, device=dev),
+            torch.zeros(blocks, GATE_WORDS, dtype=torch.int32, device=dev))
+
+
+def filter_tables(grid: FilterGrid, spec: FilterSpec, weights, out=None
+                  ) -> Tuple[torch.Tensor, torch.Tensor]:
+    """The blocks' filters, weights = [(W1, b1, W2), ...], at the grid's nodes on
+    the fp32 MFMA, and the check of their interpolation (csrc/filter_gate.h);
+    `out` = filter_table_buffers(grid, len(weights)) by default (a caller that
+    launches on another stream allocates them on the stream that consumes
+    them)."""
+    dev = grid.pos.device
+    L = len(weights)
+    F = NUM_FILTERS
+    flat = [t.detach().float().contiguous() for w in weights for t in w]
+    for k in range(L):
+        W1, b1, W2 = flat[3 * k:3 * k + 3]
+        _check(tuple(W1.shape) == (F, spec.num_rbf) and tuple(W2.shape) == (F, F)
+               and tuple(b1.shape) == (F,), "filter weights have unexpected shapes")
+    require_device(*flat)
+    tables, gates = filter_table_buffers(grid, L) if out is None else out
+    ptrs = (ctypes.c_void_p * len(flat))(*[ptr(t) for t in flat])
+    call("mlcg_filter_table", ptrs, L, grid.nodes, grid.h, grid.rc, *spec.basis_args(),
+         spec.num_rbf, spec.rbf_cut_kind, spec.rbf_lo, spec.rbf_hi, spec.conv_cut_kind,
+         spec.conv_lo, spec.conv_hi, spec.act, F, ptr(tables), ptr(gates), stream_handle(dev))
+    call("mlcg_filter_table_check", ptr(tables), L, grid.nodes, grid.h, grid.rc, ptr(gates),
+         stream_handle(dev))
+    return tables, gates
+
+
+def filter_table_rows(grid: FilterGrid, bins: PairBins, graph: PairGraph, table: torch.Tensor,
+                      gate: torch.Tensor, out: Tuple[torch.Tensor, torch.Tensor]) -> None:
+    """W, dW/dd of the pairs interpolated from a block's table into `out`
+    (fp32 or fp16); nothing is written if the table does not serve."""
+    W, Wd = out
+    cap = graph.pair_capacity
+    _check(W.dtype == Wd.dtype and tuple(W.shape) == tuple(Wd.shape) == (cap, NUM_FILTERS)
+           and W.is_contiguous() and Wd.is_contiguous(),
+           "filter_table_rows out tensors must be contiguous [pair_capacity, 128]")
+    call("mlcg_filter_table_rows", ptr(bins.records), ptr(graph.n_pairs_dev), cap, grid.h,
+         grid.nodes, grid.cut, ptr(table), ptr(gate), int(W.dtype == torch.float16), ptr(W),
+         ptr(Wd), stream_handle(W.device))
+
+
+def filter_table_reverse(grid: FilterGrid, bins: PairBins, graph: PairGraph,
+                         gagg2: torch.Tensor, y: torch.Tensor, gagg1: Optional[torch.Tensor],
+                         ydot: Optional[torch.Tensor], ddot: Optional[torch.Tensor],
+                         gate: torch.Tensor) -> Tuple[torch.Tensor, torch.Tensor]:
+    """Adjoints (Wbar, Wdbar) [nodes, F] of a block's table values from the
+    node arrays of filter_bwd_cfconv."""
+    dev = y.device
+    cap = graph.pair_capacity
+    nws = int(_lib.load().mlcg_filter_table_reverse_workspace_floats(cap, grid.nodes))
+    ws = torch.empty(nws, dtype=torch.float32, device=dev)
+    wbar = torch.empty(grid.nodes, NUM_FILTERS, dtype=torch.float32, device=dev)
+    wdbar = torch.empty(grid.nodes, NUM_FILTERS, dtype=torch.float32, device=dev)
+    g2, yc, g1, yd = (None if t is None else t.contiguous() for t in (gagg2, y, gagg1, ydot))
+    call("mlcg_filter_table_reverse", ptr(bins.records), ptr(bins.start), ptr(bins.runs), cap,
+         grid.h, grid.nodes, grid.cut, ptr(g2), ptr(yc), ptr(g1), ptr(yd), ptr(ddot),
+         ptr(gate), ptr(wbar), ptr(wdbar), ptr(ws), nws, stream_handle(dev))
+    return wbar, wdbar
 
 
 # --------------------------------------------------------------------------

@@ -1,0 +1,250 @@
+"""The filters' table over the pair distance: ordering of the pairs,
+interpolated rows, the reverse onto the table's nodes and the gate that sends
+a model whose filters the table cannot hold to the pair-by-pair kernels.
+
+Tolerances: rows and gradients against float64.  A row is a sum of four table
+values (each within the fp32 evaluation's 1e-6 of the largest, weights summing
+to at most 1.25 in magnitude) plus an interpolation error below 2.5e-7 of it:
+2e-6 of the largest value, 4e-6 for derivatives.  Gradients are sums over the
+pairs of fp32 products: 3e-6 of each tensor's norm.
+"""
+
+import math
+
+import pytest
+import torch
+
+from tests.helpers import make_cfg, make_model, rel_err
+from oracle import schnet_ref as R
+
+pytestmark = pytest.mark.gpu
+
+RC = 12.0
+
+
+def _model(basis="gaussian", act="tanh", num_rbf=50, seed=3, trainable=False, blocks=1, scale=1.0):
+    cfg = make_cfg(num_blocks=blocks, rc=RC, num_rbf=num_rbf, basis=basis, act=act)
+    sd = R.random_state_dict(cfg, seed=seed)
+    for k in sd:
+        if k.endswith("filter_network.layers.0.weight"):
+            sd[k] = sd[k] * scale
+    return make_model(cfg, sd, trainable_basis=trainable)
+
+
+def _pairs(dist):
+    """A pair list with the given distances: pair p joins nodes 2p and 2p + 1."""
+    from mlcg_amd import ops
+
+    n = dist.numel()
+    pos = torch.zeros(2 * n, 3)
+    pos[1::2, 0] = dist
+    ids = torch.arange(2 * n, dtype=torch.int32)
+    graph = ops.PairGraph(edge_index=None, rowptr=None, col=None,
+                          pair_ij=torch.stack([ids[0::2], ids[1::2]]).contiguous().cuda(),
+                          pairptr=torch.tensor([n], dtype=torch.int32).cuda(), eid2pair=None,
+                          frame_ptr=None, num_nodes=0, num_edges=2 * n, num_pairs=n)
+    return pos.cuda(), graph
+
+
+def _distances(n, h, seed=0):
+    """Spread distances with the places where an index can go wrong: zero, the
+    first and last cells, nodes themselves, the cutoff and its neighbours, and
+    a third of the pairs at one bond length."""
+    g = torch.Generator().manual_seed(seed)
+    d = torch.rand(n, generator=g) * RC
+    rc = torch.tensor(RC)
+    edge = torch.tensor([0.0, h, 1.5 * h, 2 * h, 3.5 * h, RC - h, RC - 2.5 * h, RC / 2, RC,
+                         float(torch.nextafter(rc, torch.zeros(()))), 0.3 * h])
+    d[:min(n, edge.numel())] = edge[:n]
+    d[n - n // 3:] = 3.8
+    return d
+
+
+def _filters64(model, d):
+    """W, dW/dd [P, F] in float64."""
+    p = {k: v.detach().double().cpu() for k, v in model.state_dict().items()}
+    act = torch.tanh if isinstance(model.interaction_blocks[0].activation, torch.nn.Tanh) else (
+        lambda x: torch.nn.functional.softplus(x) - math.log(2.0))
+    net = "interaction_blocks.0.conv.filter_network.layers."
+
+    def f(t):
+        cut = (0.5 * (torch.cos(t * math.pi / RC) + 1.0) * (t < RC)).unsqueeze(1)
+        if "rbf_layer.coeff" in p:
+            g = torch.exp(p["rbf_layer.coeff"] * (t.unsqueeze(1) - p["rbf_layer.offset"]) ** 2)
+        else:
+            x = torch.exp(-5.0 / RC * t).unsqueeze(1)
+            g = torch.exp(-p["rbf_layer.betas"] * (x - p["rbf_layer.means"]) ** 2)
+        h = act(g * cut @ p[net + "0.weight"].t() + p[net + "0.bias"])
+        return h @ p[net + "2.weight"].t() * cut
+
+    t = d.double()
+    return torch.func.jvp(f, (t,), (torch.ones_like(t),))
+
+
+def _setup(model, dist):
+    from mlcg_amd import ops
+
+    spec, P = model.fused_spec(), model.fused_params()
+    grid = ops.filter_grid(spec.filt, torch.device("cuda:0"))
+    pos, graph = _pairs(dist)
+    b = P.blocks[0]
+    tables, gates = ops.filter_tables(grid, spec.filt, [(b.W1, b.b1, b.W2)])
+    return spec, b, grid, pos, graph, tables, gates, ops.pair_bins(pos, graph, grid)
+
+
+@pytest.mark.parametrize("n", [1, 63, 64, 65, 1025, 20000])
+def test_pairs_in_stencil_order(n):
+    from mlcg_amd import ops
+
+    model = _model()
+    grid = ops.filter_grid(model.fused_spec().filt, torch.device("cuda:0"))
+    dist = _distances(n, grid.h)
+    pos, graph = _pairs(dist)
+    bins = ops.pair_bins(pos, graph, grid)
+    assert torch.equal(bins.dist.cpu(), dist)
+    inv_h = 1.0 / torch.tensor(grid.h, dtype=torch.float32)
+    key = ((dist * inv_h).int() - 1).clamp(0, grid.nodes - 4)
+    order = torch.sort(key, stable=True).indices
+    counts = torch.bincount(key, minlength=grid.nodes - 3)
+    assert torch.equal(bins.records[:, 0].cpu().long(), order)
+    assert torch.equal(bins.records[:, 2].cpu().long(), 2 * order + 1)
+    assert torch.equal(bins.records[:, 3].cpu().view(torch.float32), dist[order])
+    start = torch.cat([torch.zeros(1, dtype=torch.long), counts.cumsum(0)])
+    runs = torch.cat([torch.zeros(1, dtype=torch.long), ((counts + 63) // 64).cumsum(0)])
+    assert torch.equal(bins.start.cpu().long(), start)
+    assert torch.equal(bins.runs.cpu().long(), runs)
+
+
+@pytest.mark.parametrize("basis,act,num_rbf,n", [
+    ("gaussian", "tanh", 50, 1), ("gaussian", "tanh", 50, 3001), ("gaussian", "ssp", 33, 3001),
+    ("gaussian", "tanh", 100, 257), ("expnormal", "tanh", 64, 3001), ("expnormal", "ssp", 20, 65)])
+def test_rows_match_float64(basis, act, num_rbf, n):
+    from mlcg_amd import ops
+
+    model = _model(basis, act, num_rbf)
+    dist = _distances(n, ops.filter_grid_shape(model.fused_spec().filt)[1])
+    _, _, grid, _, graph, tables, gates, bins = _setup(model, dist)
+    for dt, rel in ((torch.float32, 1.0), (torch.float16, 600.0)):  # fp16: 2^-11 = 4.9e-4
+        out = tuple(torch.full((n, 128), float("nan"), dtype=dt, device="cuda") for _ in range(2))
+        ops.filter_table_rows(grid, bins, graph, tables[0], gates[0], out)
+        for got, ref, tol in zip(out, _filters64(model, dist), (2e-6, 4e-6)):
+            # the scale is the function's, not that of the few sampled pairs
+            d = torch.linspace(0, RC, 4001)
+            big = _filters64(model, d)[0 if tol == 2e-6 else 1].abs().max()
+            err = (got.double().cpu() - ref).abs().max()
+            assert err <= tol * rel * big, (dt, float(err / big))
+    assert bool((out[0][dist.cuda() >= RC] == 0).all())
+
+
+@pytest.mark.parametrize("n,one", [(1, False), (65, False), (5000, False), (3000, True)])
+@pytest.mark.parametrize("tangent,ydot", [(True, True), (True, False), (False, False)])
+def test_reverse_matches_pairwise_gradients(n, one, tangent, ydot):
+    from mlcg_amd import ops
+
+    model = _model("expnormal" if n == 65 else "gaussian")
+    h = ops.filter_grid_shape(model.fused_spec().filt)[1]
+    dist = torch.full((n,), 3.8) if one else _distances(n, h, seed=n)
+    spec, b, grid, pos, graph, _, gates, bins = _setup(model, dist)
+    g = torch.Generator("cuda").manual_seed(n)
+    g2, y, g1, yd = (torch.randn(2 * n, 128, device="cuda", generator=g) for _ in range(4))
+    dd = torch.randn(n, device="cuda", generator=g)
+    args = (g2, y, g1 if tangent else None, yd if ydot else None, dd if tangent else None)
+    wbar, wdbar = ops.filter_table_reverse(grid, bins, graph, *args, gates[0])
+    again = ops.filter_table_reverse(grid, bins, graph, *args, gates[0])
+    assert torch.equal(wbar, again[0]) and torch.equal(wdbar, again[1])
+    got = ops.filter_bwd(grid.pos, grid.graph, spec.filt, b.W1, b.b1, b.W2, wbar, wdbar)
+    # float64: the pair adjoints through the network
+    i, j = graph.pair_ij.long().cpu()
+    g2, y, g1, yd, dd = (t.double().cpu() for t in (g2, y, g1, yd, dd))
+    Wb = g2[i] * y[j] + g2[j] * y[i]
+    Wdb = torch.zeros_like(Wb)
+    if tangent:
+        Wdb = dd.unsqueeze(1) * (g1[i] * y[j] + g1[j] * y[i])
+        if ydot:
+            Wb = Wb + g1[i] * yd[j] + g1[j] * yd[i]
+    m64 = {k: v.detach().double().cpu() for k, v in model.state_dict().items()}
+    net = "interaction_blocks.0.conv.filter_network.layers."
+    W = [m64[net + k].requires_grad_(True) for k in ("0.weight", "0.bias", "2.weight")]
+    t = dist.double()
+
+    def basis(t):
+        cut = (0.5 * (torch.cos(t * math.pi / RC) + 1.0) * (t < RC)).unsqueeze(1)
+        if "rbf_layer.coeff" in m64:
+            return torch.exp(m64["rbf_layer.coeff"]
+                             * (t.unsqueeze(1) - m64["rbf_layer.offset"]) ** 2) * cut
+        x = torch.exp(-5.0 / RC * t).unsqueeze(1)
+        return torch.exp(-m64["rbf_layer.betas"] * (x - m64["rbf_layer.means"]) ** 2) * cut
+
+    G, Gd = torch.func.jvp(basis, (t,), (torch.ones_like(t),))
+    cut = (0.5 * (torch.cos(t * math.pi / RC) + 1.0) * (t < RC)).unsqueeze(1)
+    dcut = (-0.5 * math.pi / RC * torch.sin(t * math.pi / RC) * (t < RC)).unsqueeze(1)
+    H = torch.tanh(G @ W[0].t() + W[1])
+    Q, Qd = H @ W[2].t(), ((1 - H * H) * (Gd @ W[0].t())) @ W[2].t()
+    ref = torch.autograd.grad((Wb * Q * cut).sum() + (Wdb * (Qd * cut + Q * dcut)).sum(), W)
+    for name, x, r in zip(("W1", "b1", "W2"), got, ref):
+        assert rel_err(x, r) <= 3e-6, (name, rel_err(x, r))
+
+
+def _batch(frames=40, beads=20):
+    import numpy as np
+
+    from mlcg_amd import synthetic
+
+    rng = np.random.default_rng(5)
+    pos = synthetic.self_avoiding_walk(frames, beads, rng)
+    types = rng.integers(1, 21, size=(frames, beads))
+    forces = rng.standard_normal((frames * beads, 3)).astype(np.float32)
+    return synthetic._flatten(pos, types, 5, forces).to_torch("cuda")
+
+
+def _step(model, table):
+    from mlcg_amd import nn
+    from mlcg_amd.nn import _fused
+
+    saved, _fused._FILTER_TABLE = _fused._FILTER_TABLE, table
+    try:
+        model.zero_grad(set_to_none=True)
+        gm = nn.GradientsOut(model).train()
+        d = gm(_batch())
+        out = d.out["SchNet"]
+        torch.nn.functional.mse_loss(out["forces"], d.forces).backward()
+        return [out["energy"].detach(), out["forces"].detach()] + [
+            p.grad.clone() for p in model.parameters()]
+    finally:
+        _fused._FILTER_TABLE = saved
+
+
+@pytest.mark.parametrize("basis,trainable", [("gaussian", False), ("gaussian", True),
+                                             ("expnormal", True)])
+def test_step_through_table_matches_pairwise(basis, trainable):
+    """A whole step on both routes: the two differ by the roundings of the
+    filters (4e-7) and their derivatives, 1e-5 of each tensor's norm."""
+    model = _model(basis, trainable=trainable, blocks=2)
+    for a, b in zip(_step(model, True), _step(model, False)):
+        assert rel_err(a, b) <= 1e-5, rel_err(a, b)
+
+
+@pytest.mark.parametrize("poison", ["sharp", "inf", "nan"])
+def test_closed_gate_gives_the_pairwise_result(poison):
+    """A filter the grid cannot hold (first-layer weights of several hundred, a
+    non-finite weight) takes the pair-by-pair kernels: bit for bit."""
+    model = _model(blocks=2, scale=400.0 if poison == "sharp" else 1.0)
+    if poison != "sharp":
+        with torch.no_grad():
+            model.interaction_blocks[1].conv.filter_network.layers[2].weight[3, 5] = float(poison)
+    for a, b in zip(_step(model, True), _step(model, False)):
+        assert torch.equal(a.nan_to_num(7.0), b.nan_to_num(7.0))
+    from mlcg_amd import ops
+    ops.numerics_flags("cuda", clear=True)  # the poisoned weights raise them on both routes
+
+
+def test_gate_is_the_blocks_own():
+    """One block's filters are too sharp for the grid, the other's are not."""
+    from mlcg_amd import ops
+
+    model = _model(blocks=2)
+    with torch.no_grad():
+        model.interaction_blocks[0].conv.filter_network.layers[0].weight.mul_(400.0)
+    for a, b in zip(_step(model, True), _step(model, False)):
+        assert rel_err(a, b) <= 1e-5, rel_err(a, b)
+    ops.numerics_flags("cuda", clear=True)

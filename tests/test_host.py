@@ -488,3 +488,38 @@ def test_simulation_compile_model_options(monkeypatch):
     d.pos[0, 0] = float("nan")
     with pytest.raises(RuntimeError, match="forces"):
         sim.compile_model(d)
+
+
+def _filter_spec(**kw):
+    import torch
+
+    from mlcg_amd import ops
+
+    base = dict(centers=torch.zeros(50), widths=torch.zeros(1), num_rbf=50, rbf_cut_kind=1,
+                rbf_lo=0.0, rbf_hi=20.0, conv_cut_kind=1, conv_lo=0.0, conv_hi=20.0, act=0)
+    base.update(kw)
+    return ops.FilterSpec(**base)
+
+
+@pytest.mark.parametrize("kw,ok", [
+    ({}, True), ({"num_rbf": 128}, True), ({"rbf_hi": 2.0, "conv_hi": 2.0}, True),
+    ({"basis": 1, "alpha": 5 / 30.0, "num_rbf": 64, "rbf_hi": 30.0, "conv_hi": 30.0}, True),
+    ({"basis": 1, "alpha": 5 / 12.0, "num_rbf": 64, "rbf_hi": 12.0, "conv_hi": 12.0}, True),
+    ({"conv_cut_kind": 0}, True), ({"conv_hi": 25.0}, True),
+    ({"rbf_lo": 1.0}, False), ({"conv_lo": 1.0}, False),    # an envelope's kink inside
+    ({"conv_hi": 18.0}, False), ({"rbf_hi": 3e38, "rbf_cut_kind": 0}, False),
+    ({"num_rbf": 1}, False), ({"basis": 1, "alpha": 0.0}, False),
+    ({"basis": 1, "alpha": 5 / 30.0, "num_rbf": 128, "rbf_hi": 30.0, "conv_hi": 30.0}, False),
+])
+def test_filter_grid_shape(kw, ok):
+    import numpy as np
+
+    from mlcg_amd import ops
+
+    shape = ops.filter_grid_shape(_filter_spec(**kw))
+    assert (shape is not None) == ok
+    if ok:
+        n, h, rc, cut = shape
+        assert 64 <= n <= ops.TABLE_MAX_NODES and (n - 1) * h <= rc < n * h
+        k = np.arange(n)
+        assert (k.astype(np.float32) * np.float32(h) == k * h).all()  # exact node distances
