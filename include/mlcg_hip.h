@@ -263,6 +263,12 @@ int mlcg_pair_reverse_map(const int32_t* pair_ij, int64_t pair_stride,
                           const int32_t* rowptr, const int32_t* col,
                           int32_t* eid2pair, void* stream);
 
+/* out[e] = values[i] for the edges e < n_edges of every row i (the frame of
+ * each edge's centre, neighbor_list.py:85-94). */
+int mlcg_edge_values(const int32_t* rowptr, const int64_t* values,
+                     int64_t n_nodes, int64_t n_edges, int64_t* out,
+                     void* stream);
+
 /* ---------------------------------------------------------------------- */
 /* Filter network (radial basis -> cutoff -> MLP([K, F, F]) -> x cutoff)  */
 /* ---------------------------------------------------------------------- */

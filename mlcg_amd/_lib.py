@@ -59,6 +59,7 @@ _SIGNATURES = {
     "mlcg_exclusive_scan2_i32_noalloc": [_P, _P, _I64, _P, _P, _P],
     "mlcg_radius_fill": [_P, _P, _P, _I64, _F64, _I32, _I64, _P, _P, _P, _P, _I64, _I64, _P,
                          _P, _I64, _I64, _P, _P, _P, _P],
+    "mlcg_edge_values": [_P, _P, _I64, _I64, _P, _P],
     "mlcg_pair_reverse_map": [_P, _I64, _P, _I64, _P, _P, _P, _P],
     "mlcg_filter_fwd": [_P, _P, _I64, _P, _I64, _I32, _P, _P, _F32, _I32, _I32, _F32, _F32,
                         _I32, _F32, _F32, _I32, _P, _P, _P, _I32, _I32, _P, _P, _P, _P],

@@ -983,6 +983,32 @@ __global__ void radius_empty(int32_t* rowptr, int32_t* pairptr, int32_t* overflo
   if (overflow) *overflow = 0;
 }
 
+// out[e] = values[i] for the edges e of every row i: the frames of the edges
+// from the offsets, 8 bytes written an edge, instead of an index lookup that
+// reads the edge list as well (2048 x 100 beads, 7.6 M edges: 28 -> 13 us).
+// One wave takes kEdgeRows rows, whose offsets it reads together.
+constexpr int kEdgeRows = 8;
+
+__global__ __launch_bounds__(256) void edge_values_kernel(const int32_t* __restrict__ rowptr,
+                                                          const int64_t* __restrict__ values,
+                                                          int64_t n, int64_t n_edges,
+                                                          int64_t* __restrict__ out) {
+  const int lane = mlcg_lane();
+  const int64_t r0 = ((int64_t)blockIdx.x * 4 + threadIdx.x / MLCG_WAVE) * kEdgeRows;
+  if (r0 >= n) return;
+  const int64_t row = r0 + (lane < kEdgeRows ? lane : 0);
+  const int32_t off = rowptr[r0 + (lane <= kEdgeRows && r0 + lane <= n ? lane : 0)];
+  const int64_t val = values[row < n ? row : n - 1];
+  const int rows = (int)(n - r0 < kEdgeRows ? n - r0 : kEdgeRows);
+  for (int r = 0; r < rows; ++r) {
+    const int64_t b = __shfl(off, r, MLCG_WAVE);
+    int64_t e = __shfl(off, r + 1, MLCG_WAVE);
+    if (e > n_edges) e = n_edges;
+    const int64_t v = __shfl(val, r, MLCG_WAVE);
+    for (int64_t x = b + lane; x < e; x += MLCG_WAVE) out[x] = v;
+  }
+}
+
 // eid2pair for the lower copy (j, i) of every pair (i < j): binary search of i
 // in the sorted row j.
 __global__ void pair_reverse_kernel(const int32_t* __restrict__ pi,
@@ -1515,6 +1541,16 @@ extern "C" int mlcg_exclusion_pair_to_ptr(const int64_t* exc_pair_index, int64_t
     y_ptr[node + 1] = k;
   }
   return MLCG_OK;
+}
+
+extern "C" int mlcg_edge_values(const int32_t* rowptr, const int64_t* values, int64_t n_nodes,
+                                int64_t n_edges, int64_t* out, void* stream) {
+  MLCG_REQUIRE(n_nodes >= 0 && n_edges >= 0);
+  if (n_nodes == 0 || n_edges == 0) return MLCG_OK;
+  MLCG_REQUIRE(rowptr && values && out);
+  hipLaunchKernelGGL(edge_values_kernel, dim3(mlcg_div_up(n_nodes, 4 * kEdgeRows)), dim3(256), 0,
+                     mlcg_stream(stream), rowptr, values, n_nodes, n_edges, out);
+  return mlcg_launch_status();
 }
 
 extern "C" int mlcg_pair_reverse_map(const int32_t* pair_ij, int64_t pair_stride,

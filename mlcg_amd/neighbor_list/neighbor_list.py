@@ -17,18 +17,25 @@ from .. import ops
 _BACKENDS = ("torch", "custom_kernel", "hip")
 
 
-def hip_neighbor_list(data, rcut: float, self_interaction: bool = False,
-                      max_num_neighbors: int = 1000):
-    """(idx_i, idx_j, cell_shifts, mask) in the backend signature of
-    neighbor_list.py:73-78 (torch_neighbor_list for non-periodic data)."""
+def _graph(data, rcut: float, self_interaction: bool, max_num_neighbors: int):
+    """(radius graph, batch [N], cell shifts [E, 3] of non-periodic data)."""
     n = data.pos.shape[0]
     batch = data.batch if "batch" in data else torch.zeros(
         n, dtype=torch.long, device=data.pos.device)
     n_frames = int(data.n_atoms.numel()) if "n_atoms" in data else None
     g = ops.radius_graph(data.pos.detach(), rcut, batch=batch, loop=self_interaction,
                          max_num_neighbors=max_num_neighbors, n_frames=n_frames)
+    cell_shifts = torch.zeros((g.edge_index.shape[1], 3), dtype=data.pos.dtype,
+                              device=data.pos.device)
+    return g, batch, cell_shifts
+
+
+def hip_neighbor_list(data, rcut: float, self_interaction: bool = False,
+                      max_num_neighbors: int = 1000):
+    """(idx_i, idx_j, cell_shifts, mask) in the backend signature of
+    neighbor_list.py:73-78 (torch_neighbor_list for non-periodic data)."""
+    g, _, cell_shifts = _graph(data, rcut, self_interaction, max_num_neighbors)
     ei = g.edge_index
-    cell_shifts = torch.zeros((ei.shape[1], 3), dtype=data.pos.dtype, device=data.pos.device)
     return ei[0], ei[1], cell_shifts, ei[0] != ei[1]
 
 
@@ -41,15 +48,18 @@ def atomic_data2neighbor_list(data, rcut: float, self_interaction: bool = False,
             f"Method {nls_distance_method} not supported for nls-distance computation ")
     if "pbc" in data and bool(torch.as_tensor(data.pbc).any()):
         raise NotImplementedError("periodic systems are not supported by the HIP radius graph")
-    idx_i, idx_j, cell_shifts, _ = hip_neighbor_list(
-        data, rcut, self_interaction=self_interaction, max_num_neighbors=max_num_neighbors)
-    mapping = torch.stack([idx_i, idx_j], dim=0)
+    # the graph's own [2, E] edge list, and the frames of its edges from the row
+    # offsets (2048 x 100 beads: 177 -> 113 us without the copy, the unused mask
+    # and the index lookup)
+    g, batch, cell_shifts = _graph(data, rcut, self_interaction, max_num_neighbors)
+    mapping = g.edge_index
     order = mapping.shape[0]
-    batch = data.batch if "batch" in data else torch.zeros(
-        data.pos.shape[0], dtype=torch.long, device=data.pos.device)
     # every edge stays inside its frame by construction (the reference asserts
     # it, neighbor_list.py:89-91)
-    mapping_batch = batch[mapping[0]]
+    if batch.dtype == torch.int64:
+        mapping_batch = ops.edge_values(g, batch)
+    else:
+        mapping_batch = batch[mapping[0]]
     return make_neighbor_list(tag=f"nonbounded rc:{rcut} order:{order}", order=order,
                               index_mapping=mapping, mapping_batch=mapping_batch,
                               cell_shifts=cell_shifts, rcut=rcut,

@@ -378,6 +378,20 @@ def radius_graph(
                      flags=flags)
 
 
+def edge_values(graph: PairGraph, values: torch.Tensor) -> torch.Tensor:
+    """values[edge_index[0]] of an exactly sized graph ([N] int64 node values),
+    from the row offsets alone."""
+    n, e = graph.num_nodes, graph.num_edges
+    require_device(values)
+    _check(values.dtype == torch.int64 and tuple(values.shape) == (n,) and e >= 0,
+           "edge_values takes [N] int64 values and an exactly sized graph")
+    values = values.contiguous()
+    out = torch.empty(e, dtype=torch.int64, device=values.device)
+    call("mlcg_edge_values", ptr(graph.rowptr), ptr(values), n, e, ptr(out),
+         stream_handle(values.device))
+    return out
+
+
 # --------------------------------------------------------------------------
 # Reductions over long row dimensions
 
