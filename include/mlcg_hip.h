@@ -351,13 +351,13 @@ int mlcg_filter_bwd(const float* pos, const int32_t* pair_ij,
  * spacing from the others errs by less than 4e-6 of the largest value (1.6e-5
  * for derivatives; the interpolation used errs by 2^-4 of that), and no
  * pre-activation changes by more than 1/4 between nodes; non-finite values and
- * weights of magnitude 65504 or more never pass.  The *_gated entry points do
- * their work only if the table of `gate` serves (gate_want 1) or does not (0),
- * decided on the device; with gate == NULL they are the plain ones. */
+ * weights of magnitude 65504 or more never pass.  Entry points
+ * with a gate do their work only if the block's table serves (gate_want 1) or
+ * does not (0), decided on the device. */
 enum { MLCG_GATE_WORDS = 12 };
 int mlcg_filter_table(const void* const* weights, int num_blocks, int nodes,
                       float h, float rc, int basis, const float* centers,
-                      const float* widths, float alpha, int num_rbf, int
+                      const float* widths, double alpha, int num_rbf, int
                       rbf_cut_kind, float rbf_lo, float rbf_hi, int
                       conv_cut_kind, float conv_lo, float conv_hi, int act,
                       int num_filters, float* tables, uint32_t* gates, void*
@@ -367,81 +367,79 @@ int mlcg_filter_table_check(const float* tables, int num_blocks, int nodes,
                             stream);
 
 /* The pairs ordered by interpolation stencil: records [max_pairs, 4] = {pair,
- * i, j, distance bits}, stable in the pair index within a stencil; start and
+ * i, j, d / h in 2^-18 (all ones at or past `cut`, where the filter is zero)},
+ * stable in the pair index within a stencil; start and
  * run_start [nodes - 2] = first record and first run (of at most 64 records)
  * of every stencil; dist [max_pairs] in pair order.  Stencil s covers nodes
  * s .. s + 3. */
 int64_t mlcg_pair_bins_workspace_ints(int64_t max_pairs, int nodes);
 int mlcg_pair_bins(const float* pos, const int32_t* pair_ij, int64_t
                    pair_stride, const int32_t* n_pairs_dev, int64_t max_pairs,
-                   float h, int nodes, float* dist, int32_t* start,
+                   float h, int nodes, float cut, float* dist, int32_t* start,
                    int32_t* run_start, int32_t* records, int32_t* workspace,
                    int64_t workspace_ints, void* stream);
 
-/* W, dW/dd [max_pairs, F] (fp32, or fp16 when f16) by cubic Lagrange
- * interpolation in `table` (one block's [4, nodes + 1, F]); exactly zero from
- * distance `cut` on.  Nothing is written if the table does not serve. */
+/* W, dW/dd [max_pairs, F] of every block (fp32, or fp16 when f16) by cubic
+ * Lagrange interpolation in `tables`, written to outputs[2 k], outputs[2 k + 1]
+ * (host array of device pointers).
+ * Nothing is written for a block whose table does not serve. */
 int mlcg_filter_table_rows(const int32_t* records, const int32_t* n_pairs_dev,
-                           int64_t max_pairs, float h, int nodes, float
-                           cut, const float* table, const uint32_t* gate, int
-                           f16, void* W, void* Wd, void* stream);
+                           int64_t max_pairs, int nodes, const float* tables,
+                           const uint32_t* gates, int num_blocks, int f16,
+                           void* const* outputs, void* stream);
 
-/* Adjoints wbar, wdbar [nodes, F] of a block's table values: the pair adjoints
- * of mlcg_filter_bwd_cfconv times the interpolation weights, summed in a fixed
- * order.  mlcg_filter_bwd on the nodes then gives the weight gradients. */
+/* Adjoints of a block's table values: the pair adjoints of
+ * mlcg_filter_bwd_cfconv times the interpolation weights, summed per run into
+ * `slots` (mlcg_filter_table_reverse, one launch per block, slots of
+ * mlcg_filter_table_reverse_workspace_floats floats), then per node into wbar,
+ * wdbar [num_blocks, nodes, F] (mlcg_filter_table_combine, all blocks, whose
+ * slots follow each other); tangent as gagg1 != NULL.  Every sum has a fixed
+ * order.  mlcg_filter_bwd_blocks on the nodes then gives the weight
+ * gradients. */
 int64_t mlcg_filter_table_reverse_workspace_floats(int64_t max_pairs, int
     nodes);
 int mlcg_filter_table_reverse(const int32_t* records, const int32_t* start,
-                              const int32_t* run_start, int64_t max_pairs,
-                              float h, int nodes, float cut, const float*
-                              gagg2, const float* y, const float* gagg1, const
-                              float* ydot, const float* ddot, const uint32_t*
-                              gate, float* wbar, float* wdbar, float*
-                              workspace, int64_t workspace_floats, void*
-                              stream);
+                              const int32_t* run_start, int64_t max_pairs, int
+                              nodes, const float* gagg2, const float* y, const
+                              float* gagg1, const float* ydot, const float*
+                              ddot, const uint32_t* gate, float* slots,
+                              int64_t slot_floats, void* stream);
+int mlcg_filter_table_combine(const int32_t* run_start, int64_t max_pairs, int
+                              nodes, int tangent, const float* slots, int
+                              num_blocks, const uint32_t* gates, float* wbar,
+                              float* wdbar, void* stream);
 
-/* Gated forms (see mlcg_filter_table). */
-int mlcg_filter_fwd_gated(const float* pos, const int32_t* pair_ij, int64_t
-                          pair_stride, const int32_t* n_pairs_dev, int64_t
-                          max_pairs, int basis, const float* centers, const
-                          float* widths, float alpha, int num_rbf, int
-                          rbf_cut_kind, float rbf_lo, float rbf_hi, int
-                          conv_cut_kind, float conv_lo, float conv_hi, int
-                          act, const float* W1, const float* b1, const float*
-                          W2, int num_filters, int f16, void* W_out, void*
-                          Wd_out, float* dist_out, const uint32_t* gate, int
-                          gate_want, void* stream);
-int mlcg_filter_bwd_gated(const float* pos, const int32_t* pair_ij, int64_t
-                          pair_stride, const int32_t* n_pairs_dev, int64_t
-                          max_pairs, int basis, const float* centers, const
-                          float* widths, float alpha, int num_rbf, int
-                          rbf_cut_kind, float rbf_lo, float rbf_hi, int
-                          conv_cut_kind, float conv_lo, float conv_hi, int
-                          act, const float* W1, const float* b1, const float*
-                          W2, int num_filters, const float* Wbar, const float*
-                          Wdbar, float* dW1, float* db1, float* dW2, float*
-                          abar_out, float* adbar_out, float* workspace,
-                          int64_t workspace_floats, int fp32_strict, const
-                          uint32_t* gate, int gate_want, void* stream);
-int mlcg_filter_bwd_cfconv_gated(const float* pos, const int32_t* pair_ij,
-                                 int64_t pair_stride, const int32_t*
-                                 n_pairs_dev, int64_t max_pairs, int basis,
-                                 const float* centers, const float* widths,
-                                 float alpha, int num_rbf, int rbf_cut_kind,
-                                 float rbf_lo, float rbf_hi, int
-                                 conv_cut_kind, float conv_lo, float conv_hi,
-                                 int act, const float* W1, const float* b1,
-                                 const float* W2, int num_filters, const
-                                 float* gagg2, const float* y, const float*
-                                 gagg1, const float* ydot, const float* ddot,
-                                 float* dW1, float* db1, float* dW2, float*
-                                 abar_out, float* adbar_out, float* workspace,
-                                 int64_t workspace_floats, int fp32_strict,
-                                 const uint32_t* gate, int gate_want, void*
-                                 stream);
+/* Several blocks in one launch, gated (gates may be NULL).
+ * mlcg_filter_fwd_blocks: weights and outputs as above, no distances.
+ * mlcg_filter_bwd_blocks: 15 pointers a block -- W1, b1, W2, then the pair
+ * adjoints Wbar, Wdbar (mlcg_filter_bwd) or the node arrays gagg2, y, gagg1,
+ * ydot, ddot (mlcg_filter_bwd_cfconv), then dW1, db1, dW2, abar_out,
+ * adbar_out; every block takes its adjoints in the same form. */
+int mlcg_filter_fwd_blocks(const float* pos, const int32_t* pair_ij, int64_t
+                           pair_stride, const int32_t* n_pairs_dev, int64_t
+                           max_pairs, int basis, const float* centers, const
+                           float* widths, double alpha, int num_rbf, int
+                           rbf_cut_kind, float rbf_lo, float rbf_hi, int
+                           conv_cut_kind, float conv_lo, float conv_hi, int
+                           act, const void* const* weights, void* const*
+                           outputs, int num_blocks, int num_filters, int f16,
+                           const uint32_t* gates, int gate_want, void*
+                           stream);
+int64_t mlcg_filter_bwd_blocks_workspace_floats(int64_t max_pairs, int
+    num_rbf, int num_blocks);
+int mlcg_filter_bwd_blocks(const float* pos, const int32_t* pair_ij, int64_t
+                           pair_stride, const int32_t* n_pairs_dev, int64_t
+                           max_pairs, int basis, const float* centers, const
+                           float* widths, double alpha, int num_rbf, int
+                           rbf_cut_kind, float rbf_lo, float rbf_hi, int
+                           conv_cut_kind, float conv_lo, float conv_hi, int
+                           act, void* const* blocks, int num_blocks, int
+                           num_filters, const uint32_t* gates, int gate_want,
+                           float* workspace, int64_t workspace_floats, void*
+                           stream);
 int mlcg_rbf_param_grad_gated(const float* dist, const int32_t* n_pairs_dev,
                               int64_t max_pairs, int basis, const float*
-                              centers, const float* widths, float alpha, int
+                              centers, const float* widths, double alpha, int
                               num_rbf, int rbf_cut_kind, float rbf_lo, float
                               rbf_hi, const float* W1, int num_filters, const
                               float* abar, const float* adbar, int accumulate,

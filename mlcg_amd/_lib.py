@@ -63,35 +63,32 @@ _SIGNATURES = {
     "mlcg_pair_reverse_map": [_P, _I64, _P, _I64, _P, _P, _P, _P],
     "mlcg_filter_fwd": [_P, _P, _I64, _P, _I64, _I32, _P, _P, _F32, _I32, _I32, _F32, _F32,
                         _I32, _F32, _F32, _I32, _P, _P, _P, _I32, _I32, _P, _P, _P, _P],
-    "mlcg_filter_fwd_gated": [_P, _P, _I64, _P, _I64, _I32, _P, _P, _F32, _I32, _I32, _F32,
-        _F32, _I32, _F32, _F32, _I32, _P, _P, _P, _I32, _I32, _P, _P, _P, _P, _I32, _P],
     "mlcg_filter_bwd_workspace_floats": [_I64, _I32],
     "mlcg_filter_bwd": [_P, _P, _I64, _P, _I64, _I32, _P, _P, _F32, _I32, _I32, _F32, _F32,
                         _I32, _F32, _F32, _I32, _P, _P, _P, _I32, _P, _P, _P, _P, _P, _P, _P,
                         _P, _I64, _I32, _P],
-    "mlcg_filter_bwd_gated": [_P, _P, _I64, _P, _I64, _I32, _P, _P, _F32, _I32, _I32, _F32,
-        _F32, _I32, _F32, _F32, _I32, _P, _P, _P, _I32, _P, _P, _P, _P, _P, _P, _P, _P,
-        _I64, _I32, _P, _I32, _P],
     "mlcg_filter_bwd_cfconv": [_P, _P, _I64, _P, _I64, _I32, _P, _P, _F32, _I32, _I32, _F32,
                                _F32, _I32, _F32, _F32, _I32, _P, _P, _P, _I32, _P, _P, _P, _P,
                                _P, _P, _P, _P, _P, _P, _P, _I64, _I32, _P],
-    "mlcg_filter_bwd_cfconv_gated": [_P, _P, _I64, _P, _I64, _I32, _P, _P, _F32, _I32, _I32,
-        _F32, _F32, _I32, _F32, _F32, _I32, _P, _P, _P, _I32, _P, _P, _P, _P, _P, _P, _P,
-        _P, _P, _P, _P, _I64, _I32, _P, _I32, _P],
     "mlcg_rbf_param_grad_workspace_floats": [_I64, _I32],
     "mlcg_rbf_param_grad": [_P, _P, _I64, _I32, _P, _P, _F32, _I32, _I32, _F32, _F32, _P, _I32,
                             _P, _P, _I32, _P, _P, _P, _I64, _P],
-    "mlcg_rbf_param_grad_gated": [_P, _P, _I64, _I32, _P, _P, _F32, _I32, _I32, _F32, _F32,
-        _P, _I32, _P, _P, _I32, _P, _P, _P, _I64, _P, _I32, _P],
-    "mlcg_filter_table": [_P, _I32, _I32, _F32, _F32, _I32, _P, _P, _F32, _I32, _I32, _F32,
-                          _F32, _I32, _F32, _F32, _I32, _I32, _P, _P, _P],
+    "mlcg_rbf_param_grad_gated": [_P, _P, _I64, _I32, _P, _P, _F64, _I32, _I32, _F32, _F32, _P,
+        _I32, _P, _P, _I32, _P, _P, _P, _I64, _P, _I32, _P],
+    "mlcg_filter_table": [_P, _I32, _I32, _F32, _F32, _I32, _P, _P, _F64, _I32, _I32, _F32,
+        _F32, _I32, _F32, _F32, _I32, _I32, _P, _P, _P],
     "mlcg_filter_table_check": [_P, _I32, _I32, _F32, _F32, _P, _P],
     "mlcg_pair_bins_workspace_ints": [_I64, _I32],
-    "mlcg_pair_bins": [_P, _P, _I64, _P, _I64, _F32, _I32, _P, _P, _P, _P, _P, _I64, _P],
-    "mlcg_filter_table_rows": [_P, _P, _I64, _F32, _I32, _F32, _P, _P, _I32, _P, _P, _P],
+    "mlcg_pair_bins": [_P, _P, _I64, _P, _I64, _F32, _I32, _F32, _P, _P, _P, _P, _P, _I64, _P],
     "mlcg_filter_table_reverse_workspace_floats": [_I64, _I32],
-    "mlcg_filter_table_reverse": [_P, _P, _P, _I64, _F32, _I32, _F32, _P, _P, _P, _P, _P, _P,
-                                  _P, _P, _P, _I64, _P],
+    "mlcg_filter_fwd_blocks": [_P, _P, _I64, _P, _I64, _I32, _P, _P, _F64, _I32, _I32, _F32,
+        _F32, _I32, _F32, _F32, _I32, _P, _P, _I32, _I32, _I32, _P, _I32, _P],
+    "mlcg_filter_bwd_blocks": [_P, _P, _I64, _P, _I64, _I32, _P, _P, _F64, _I32, _I32, _F32,
+        _F32, _I32, _F32, _F32, _I32, _P, _I32, _I32, _P, _I32, _P, _I64, _P],
+    "mlcg_filter_table_rows": [_P, _P, _I64, _I32, _P, _P, _I32, _I32, _P, _P],
+    "mlcg_filter_table_reverse": [_P, _P, _P, _I64, _I32, _P, _P, _P, _P, _P, _P, _P, _I64, _P],
+    "mlcg_filter_table_combine": [_P, _I64, _I32, _I32, _P, _I32, _P, _P, _P, _P],
+    "mlcg_filter_bwd_blocks_workspace_floats": [_I64, _I32, _I32],
     "mlcg_cfconv_gather": [_P, _P, _I32, _P, _P, _P, _I64, _I32, _P, _P],
     "mlcg_cfconv_gather_bwd": [_P, _P, _P, _P, _I32, _P, _P, _P, _I64, _I32, _P, _P, _I32,
                                _P],
@@ -150,6 +147,7 @@ _SIGNATURES = {
 _RESTYPES = {"mlcg_version": _c.c_char_p, "mlcg_scan_workspace_ints": _I64,
              "mlcg_radius_workspace_bytes": _I64,
              "mlcg_pair_bins_workspace_ints": _I64,
+             "mlcg_filter_bwd_blocks_workspace_floats": _I64,
              "mlcg_filter_table_reverse_workspace_floats": _I64,
              "mlcg_filter_bwd_workspace_floats": _I64, "mlcg_node_tmm_workspace_floats": _I64,
              "mlcg_node_tmm_batch_workspace_floats": _I64,

@@ -106,6 +106,8 @@ struct RbfParams {
   const float* centers;
   const float* widths;
   float alpha;
+  double alpha64;  // the node kernels': a float's rounding of alpha alone moves
+                   // the basis' gradients by 1e-6
   int basis;
   int K;
   int rbf_kind;
@@ -115,6 +117,19 @@ struct RbfParams {
   int act;
   int same_cut;  // the CFConv envelope is the RBF envelope: evaluated once
   Cut rcut, ccut;  // the two envelopes in branch-free form
+};
+
+// Blocks of one launch (blockIdx.y): weights, outputs, and the gate that says
+// whether the block's pairs are evaluated here or through its table.
+constexpr int kMaxBlocks = 8;
+struct FwdBlock {
+  const float *W1, *b1, *W2;
+  void *W, *Wd;
+  float* dist;
+  FilterGate gate;
+};
+struct FwdBatch {
+  FwdBlock b[kMaxBlocks];
 };
 
 // Activation value and first derivative for a compile-time activation id.
@@ -185,11 +200,59 @@ __device__ __forceinline__ void rbf_eval(const RbfParams& rp, bool on, float cen
 __device__ __forceinline__ void rbf_expnormal_fine(const RbfParams& rp, float cen, float wid,
                                                    float d, float crbf, float dcrbf, float& g,
                                                    float& gd) {
-  const double ex = exp((double)rp.alpha * ((double)rp.rbf_lo - (double)d));
+  const double ex = exp(rp.alpha64 * ((double)rp.rbf_lo - (double)d));
   const float u = (float)(ex - (double)cen);
   const float e = __expf(-wid * (u * u));
   g = e * crbf;
   gd = e * (dcrbf + 2.0f * rp.alpha * wid * u * (float)ex * crbf);
+}
+
+// The elementwise functions of the filter in double, for the nodes of a table:
+// a node's rounding is shared by every pair near it (bonded pairs, a tenth of a
+// chain's, all lie in one cell) and does not average out over the pairs as in
+// the pair-by-pair kernels.  In float the gradients of an exponential-normal
+// basis, which depend on exp(-alpha d) - centre with a factor of some 45, were
+// 4e-6 off.  Envelope: identity, or cosine with lower bound 0.
+__device__ __forceinline__ void cutoff_f64(int kind, float hi, double d, double& c, double& dc) {
+  c = 1.0;
+  dc = 0.0;
+  if (kind == MLCG_CUT_COSINE) {
+    const double ih = 1.0 / (double)hi;
+    double sn, cs;
+    sincospi(d * ih, &sn, &cs);
+    const double m = d < (double)hi ? 1.0 : 0.0;
+    c = 0.5 * (cs + 1.0) * m;
+    dc = -0.5 * sn * (3.14159265358979323846 * ih) * m;
+  }
+}
+
+__device__ __forceinline__ void rbf_f64(const RbfParams& rp, double cen, double wid, double d,
+                                        double crbf, double dcrbf, double& g, double& gd) {
+  if (rp.basis == 0) {
+    const double diff = d - cen;
+    const double e = exp(wid * diff * diff);
+    g = e * crbf;
+    gd = e * (2.0 * wid * diff * crbf + dcrbf);
+  } else {
+    const double alpha = rp.alpha64;
+    const double ex = exp(alpha * ((double)rp.rbf_lo - d)), u = ex - cen;
+    const double e = exp(-wid * u * u);
+    g = e * crbf;
+    gd = e * (dcrbf + 2.0 * alpha * wid * u * ex * crbf);
+  }
+}
+
+__device__ __forceinline__ void act_f64(int act, double x, double& s, double& d1, double& d2) {
+  if (act == MLCG_ACT_TANH) {
+    s = tanh(x);
+    d1 = 1.0 - s * s;
+    d2 = -2.0 * s * d1;
+  } else {
+    const double sp = x > 20.0 ? x : fmax(x, 0.0) + log1p(exp(-fabs(x)));
+    d1 = 1.0 / (1.0 + exp(-x));
+    s = sp - 0.69314718055994530942;
+    d2 = d1 * (1.0 - d1);
+  }
 }
 
 // rbf_eval for a compile-time basis kind (no branch on rp.basis).
@@ -359,10 +422,15 @@ __device__ __forceinline__ void gemm2_f32(const float* w2s, const floatx4* bx,
 __global__ __launch_bounds__(kThreads) void filter_fwd_f32_kernel(
     const float* __restrict__ pos, const int32_t* __restrict__ pi,
     const int32_t* __restrict__ pj, const int32_t* __restrict__ n_pairs_dev,
-    int64_t max_pairs, RbfParams rp, const float* __restrict__ W1,
-    const float* __restrict__ b1, const float* __restrict__ W2, float* __restrict__ Wout,
-    float* __restrict__ Wdout, float* __restrict__ dist_out, FilterGate gate) {
-  if (gate_closed(gate)) return;
+    int64_t max_pairs, RbfParams rp, FwdBatch batch) {
+  const FwdBlock& blk = batch.b[blockIdx.y];
+  if (gate_closed(blk.gate)) return;
+  const float* __restrict__ W1 = blk.W1;
+  const float* __restrict__ b1 = blk.b1;
+  const float* __restrict__ W2 = blk.W2;
+  float* __restrict__ Wout = static_cast<float*>(blk.W);
+  float* __restrict__ Wdout = static_cast<float*>(blk.Wd);
+  float* __restrict__ dist_out = blk.dist;
   extern __shared__ float lds[];
   const int KS = (rp.K + 3) / 4;
   float* w1s = lds;
@@ -442,7 +510,7 @@ __global__ __launch_bounds__(kThreads) void filter_fwd_f32_kernel(
 // wave w of 8 owns feature tile w of both products: its slices of W1 and W2
 // (13 + 32 registers) are read straight into the A fragments, the activations
 // pass through LDS once, and a workgroup takes two node tiles.
-constexpr int kTableBlocks = 8;
+constexpr int kTableBlocks = kMaxBlocks;
 constexpr int kTableTiles = 2;
 constexpr int kTableStride = kF + 4;  // floats per node row in LDS (bank spread)
 struct FilterTableBatch {
@@ -450,37 +518,6 @@ struct FilterTableBatch {
   const float* b1[kTableBlocks];
   const float* W2[kTableBlocks];
 };
-
-// Envelope (identity, or cosine with lower bound 0) and basis function in double.
-__device__ __forceinline__ void cutoff_f64(int kind, float hi, double d, double& c, double& dc) {
-  c = 1.0;
-  dc = 0.0;
-  if (kind == MLCG_CUT_COSINE) {
-    const double ih = 1.0 / (double)hi;
-    double sn, cs;
-    sincospi(d * ih, &sn, &cs);
-    const double m = d < (double)hi ? 1.0 : 0.0;
-    c = 0.5 * (cs + 1.0) * m;
-    dc = -0.5 * sn * (3.14159265358979323846 * ih) * m;
-  }
-}
-
-__device__ __forceinline__ void rbf_f64(const RbfParams& rp, int k, double d, double crbf,
-                                        double dcrbf, double& g, double& gd) {
-  const double cen = rp.centers[k];
-  if (rp.basis == 0) {
-    const double wid = rp.widths[0], diff = d - cen;
-    const double e = exp(wid * diff * diff);
-    g = e * crbf;
-    gd = e * (2.0 * wid * diff * crbf + dcrbf);
-  } else {
-    const double wid = rp.widths[k], alpha = rp.alpha;
-    const double ex = exp(alpha * ((double)rp.rbf_lo - d)), u = ex - cen;
-    const double e = exp(-wid * u * u);
-    g = e * crbf;
-    gd = e * (dcrbf + 2.0 * alpha * wid * u * ex * crbf);
-  }
-}
 
 template <int KSMAX>
 __global__ __launch_bounds__(kThreads) void filter_table_kernel(
@@ -503,10 +540,7 @@ __global__ __launch_bounds__(kThreads) void filter_table_kernel(
   for (int u = 0; u < kFT; ++u) a2[u] = *reinterpret_cast<const float4*>(W2 + 16 * u);
   const float4 bias = *reinterpret_cast<const float4*>(fb.b1[blk] + 16 * w + 4 * q);
   const float bv[4] = {bias.x, bias.y, bias.z, bias.w};
-  // the basis at the nodes, each wave its k steps: in double, since a node's
-  // rounding is shared by every pair near it and does not average out over the
-  // pairs (exponential-normal basis in fp32: the forces' parameter gradients
-  // 4e-6 off instead of 6e-7)
+  // the basis at the nodes, each wave its k steps
 #pragma unroll
   for (int t = 0; t < kTableTiles; ++t) {
     const int k = (blockIdx.x * kTableTiles + t) * 16 + n;
@@ -515,7 +549,9 @@ __global__ __launch_bounds__(kThreads) void filter_table_kernel(
     cutoff_f64(rp.rbf_kind, rp.rbf_hi, d, crbf, dcrbf);
     for (int s = w; s < KSMAX; s += kWaves) {
       double g = 0.0, gd = 0.0;
-      if (4 * s + q < K) rbf_f64(rp, 4 * s + q, d, crbf, dcrbf, g, gd);
+      if (4 * s + q < K)
+        rbf_f64(rp, rp.centers[4 * s + q], rp.widths[rp.basis == 0 ? 0 : 4 * s + q], d, crbf,
+                dcrbf, g, gd);
       gs[t][0][4 * s + q][n] = (float)g;
       gs[t][1][4 * s + q][n] = (float)gd;
     }
@@ -555,8 +591,9 @@ __global__ __launch_bounds__(kThreads) void filter_table_kernel(
     float* pdc = &hdc.x;
 #pragma unroll
     for (int i = 0; i < 4; ++i) {
-      float s, d1, d2;
-      mlcg_act(rp.act, a[i] + bv[i], s, d1, d2);
+      double s64, e64, unused;
+      act_f64(rp.act, (double)a[i] + bv[i], s64, e64, unused);
+      const float s = (float)s64, d1 = (float)e64;
       const unsigned u = __float_as_uint(fabsf(ad[i]) * h);
       steep = steep > u ? steep : u;
       pv[i] = s;
@@ -679,10 +716,15 @@ template <int KS32, int BASIS, int ACT>
 __global__ __launch_bounds__(kThreads16, kWaves16 * MLCG_F16_GROUPS_PER_CU / 4) void filter_fwd_f16_kernel(
     const float* __restrict__ pos, const int32_t* __restrict__ pi,
     const int32_t* __restrict__ pj, const int32_t* __restrict__ n_pairs_dev,
-    int64_t max_pairs, RbfParams rp, const float* __restrict__ W1,
-    const float* __restrict__ b1, const float* __restrict__ W2, __half* __restrict__ Wout,
-    __half* __restrict__ Wdout, float* __restrict__ dist_out, FilterGate gate) {
-  if (gate_closed(gate)) return;
+    int64_t max_pairs, RbfParams rp, FwdBatch batch) {
+  const FwdBlock& blk = batch.b[blockIdx.y];
+  if (gate_closed(blk.gate)) return;
+  const float* __restrict__ W1 = blk.W1;
+  const float* __restrict__ b1 = blk.b1;
+  const float* __restrict__ W2 = blk.W2;
+  __half* __restrict__ Wout = static_cast<__half*>(blk.W);
+  __half* __restrict__ Wdout = static_cast<__half*>(blk.Wd);
+  float* __restrict__ dist_out = blk.dist;
   extern __shared__ float lds[];
   _Float16* w1h = reinterpret_cast<_Float16*>(lds);
   _Float16* w2h = w1h + kFT * KS32 * MLCG_WAVE * 8;
@@ -913,10 +955,15 @@ template <int BASIS, int ACT>
 __global__ __launch_bounds__(kThreadsX3) void filter_fwd_x3_kernel(
     const float* __restrict__ pos, const int32_t* __restrict__ pi,
     const int32_t* __restrict__ pj, const int32_t* __restrict__ n_pairs_dev,
-    int64_t max_pairs, RbfParams rp, const float* __restrict__ W1,
-    const float* __restrict__ b1, const float* __restrict__ W2, float* __restrict__ Wout,
-    float* __restrict__ Wdout, float* __restrict__ dist_out, FilterGate gate) {
-  if (gate_closed(gate)) return;
+    int64_t max_pairs, RbfParams rp, FwdBatch batch) {
+  const FwdBlock& blk = batch.b[blockIdx.y];
+  if (gate_closed(blk.gate)) return;
+  const float* __restrict__ W1 = blk.W1;
+  const float* __restrict__ b1 = blk.b1;
+  const float* __restrict__ W2 = blk.W2;
+  float* __restrict__ Wout = static_cast<float*>(blk.W);
+  float* __restrict__ Wdout = static_cast<float*>(blk.Wd);
+  float* __restrict__ dist_out = blk.dist;
   extern __shared__ float lds[];
   const int K = rp.K;
   constexpr int KS32 = kX3Blocks;
@@ -1321,6 +1368,18 @@ struct PairAdjoint {
   const float* dd;    //            ddot [P] (with g1)
 };
 
+// Blocks of one launch (blockIdx.y).
+struct BwdBlock {
+  const float *W1, *b1, *W2;
+  PairAdjoint adj;
+  float *abar, *adbar;
+  float *dW1, *db1, *dW2;
+  FilterGate gate;
+};
+struct BwdBatch {
+  BwdBlock b[kMaxBlocks];
+};
+
 __device__ __forceinline__ float4 ld4(const float* __restrict__ p, int64_t row, int col) {
   return *reinterpret_cast<const float4*>(p + row * kF + col);
 }
@@ -1403,11 +1462,18 @@ template <int KSMAX, bool kNodes, int BASIS, int ACT>
 __global__ __launch_bounds__(kBwdThreads) void filter_bwd_fused_kernel(
     const float* __restrict__ pos, const int32_t* __restrict__ pi,
     const int32_t* __restrict__ pj, const int32_t* __restrict__ n_pairs_dev,
-    int64_t max_pairs, RbfParams rp, const float* __restrict__ W1,
-    const float* __restrict__ b1, const float* __restrict__ W2, PairAdjoint adj,
-    float* __restrict__ abar_out, float* __restrict__ adbar_out, float* __restrict__ partial,
-    FilterGate gate) {
+    int64_t max_pairs, RbfParams rp, BwdBatch batch, float* __restrict__ partials) {
+  const BwdBlock& blk = batch.b[blockIdx.y];
+  const FilterGate gate = blk.gate;
   if (gate_closed(gate)) return;
+  const float* __restrict__ W1 = blk.W1;
+  const float* __restrict__ b1 = blk.b1;
+  const float* __restrict__ W2 = blk.W2;
+  const PairAdjoint adj = blk.adj;
+  float* __restrict__ abar_out = blk.abar;
+  float* __restrict__ adbar_out = blk.adbar;
+  float* __restrict__ partial =
+      partials + (int64_t)blockIdx.y * gridDim.x * bwd_partial_floats(rp.K);
   constexpr int KTMAX = (4 * KSMAX + 15) / 16;
   // basis rows span the compile-time maximum width (rows k >= K hold zeros),
   // so the k loops below run without data-dependent branches
@@ -1572,7 +1638,7 @@ __global__ __launch_bounds__(kBwdThreads) void filter_bwd_fused_kernel(
   float ra = 1.0f, arun = 0.0f;  // the same for ab in step 6 (no beta: |g| <= 1)
 
   // on the nodes of a table the exponential-normal basis takes its inner
-  // exponential in double: a node's rounding is shared by every pair near it
+  // exponential in double
   const bool fine_basis = !kNodes && BASIS != 0 && gate.words != nullptr && rp.basis == 1;
   const bool tangent = kNodes && adj.g1 != nullptr;
   const bool has_yd = tangent && adj.yd != nullptr;
@@ -2131,9 +2197,14 @@ __global__ __launch_bounds__(kBwdThreads) void filter_bwd_fused_kernel(
 constexpr int kRedOut = 64;
 
 __global__ __launch_bounds__(256) void filter_bwd_reduce_kernel(
-    const float* __restrict__ partial, int groups, int K, float* __restrict__ dW1,
-    float* __restrict__ db1, float* __restrict__ dW2, FilterGate gate) {
-  if (gate_closed(gate)) return;
+    const float* __restrict__ partials, int groups, int K, BwdBatch batch) {
+  const BwdBlock& blk = batch.b[blockIdx.y];
+  if (gate_closed(blk.gate)) return;
+  float* __restrict__ dW1 = blk.dW1;
+  float* __restrict__ db1 = blk.db1;
+  float* __restrict__ dW2 = blk.dW2;
+  const float* __restrict__ partial =
+      partials + (int64_t)blockIdx.y * groups * bwd_partial_floats(K);
   __shared__ float part[4][kRedOut];
   const int Kp16 = bwd_kp16(K);
   const int stride = bwd_partial_floats(K);
@@ -2169,9 +2240,12 @@ __global__ __launch_bounds__(256) void filter_bwd_reduce_kernel(
   if (slice == 0 && dst) *dst = (part[0][o] + part[1][o]) + (part[2][o] + part[3][o]);
 }
 
-int bwd_groups(int64_t max_pairs) {
+// Workgroups of one of n blocks: one per CU in all (a workgroup's 144 KiB of LDS
+// leave no room for a second), so that a batch's weights are staged once.
+int bwd_groups(int64_t max_pairs, int n) {
   const int64_t tiles = (max_pairs + 15) / 16;
-  return (int)(tiles < 256 ? (tiles < 1 ? 1 : tiles) : 256);
+  const int64_t most = 256 / n;
+  return (int)(tiles < most ? (tiles < 1 ? 1 : tiles) : most);
 }
 
 // Kernels here use more than 64 KiB of dynamic LDS; raise their limit to the
@@ -2219,13 +2293,14 @@ void allow_lds_once() {
   done[dev] = true;
 }
 
-RbfParams make_params(int basis, const float* centers, const float* widths, float alpha, int K,
+RbfParams make_params(int basis, const float* centers, const float* widths, double alpha, int K,
                       int rk, float rlo, float rhi, int ck, float clo, float chi, int act) {
   RbfParams rp;
   rp.basis = basis;
   rp.centers = centers;
   rp.widths = widths;
-  rp.alpha = alpha;
+  rp.alpha = (float)alpha;
+  rp.alpha64 = alpha;
   rp.K = K;
   rp.rbf_kind = rk;
   rp.rbf_lo = rlo;
@@ -2272,20 +2347,20 @@ extern "C" int mlcg_numerics_flags(int* out, int clear, void* stream) {
 
 namespace {
 
+// The filter forward of n <= kMaxBlocks blocks.
 int filter_fwd_impl(const float* pos, const int32_t* pair_ij, int64_t pair_stride,
-                               const int32_t* n_pairs_dev, int64_t max_pairs, int basis,
-                               const float* centers, const float* widths, float alpha,
-                               int num_rbf, int rbf_cut_kind, float rbf_lo, float rbf_hi,
-                               int conv_cut_kind, float conv_lo, float conv_hi, int act,
-                               const float* W1, const float* b1, const float* W2,
-                               int num_filters, int f16, void* W_out, void* Wd_out,
-                               float* dist_out, const FilterGate& gate, void* stream) {
+                    const int32_t* n_pairs_dev, int64_t max_pairs, int basis,
+                    const float* centers, const float* widths, double alpha, int num_rbf,
+                    int rbf_cut_kind, float rbf_lo, float rbf_hi, int conv_cut_kind,
+                    float conv_lo, float conv_hi, int act, int num_filters, int f16,
+                    const FwdBatch& fb, int n, void* stream) {
   if (!valid_params(basis, num_rbf, rbf_cut_kind, conv_cut_kind, act, num_filters))
     return MLCG_ERR_UNSUPPORTED;
   MLCG_REQUIRE(max_pairs >= 0 && pair_stride >= max_pairs);
   if (max_pairs == 0) return MLCG_OK;
-  MLCG_REQUIRE(pos && pair_ij && n_pairs_dev && centers && widths && W1 && b1 && W2 && W_out &&
-               Wd_out);
+  MLCG_REQUIRE(pos && pair_ij && n_pairs_dev && centers && widths);
+  for (int k = 0; k < n; ++k)
+    MLCG_REQUIRE(fb.b[k].W1 && fb.b[k].b1 && fb.b[k].W2 && fb.b[k].W && fb.b[k].Wd);
   RbfParams rp = make_params(basis, centers, widths, alpha, num_rbf, rbf_cut_kind, rbf_lo,
                              rbf_hi, conv_cut_kind, conv_lo, conv_hi, act);
   const unsigned groups = mlcg_persistent_groups(mlcg_div_up(max_pairs, 16 * kWaves), 1);
@@ -2298,9 +2373,8 @@ int filter_fwd_impl(const float* pos, const int32_t* pair_ij, int64_t pair_strid
     allow_lds_once();
     const unsigned gx = mlcg_persistent_groups(mlcg_div_up(max_pairs, 16 * kWavesX3), 1);
 #define MLCG_X3_LAUNCH(B, A)                                                               \
-  hipLaunchKernelGGL((filter_fwd_x3_kernel<B, A>), dim3(gx), dim3(kThreadsX3), lds, s, pos,  \
-                     pair_ij, pair_ij + pair_stride, n_pairs_dev, max_pairs, rp, W1, b1, W2, \
-                     static_cast<float*>(W_out), static_cast<float*>(Wd_out), dist_out, gate)
+  hipLaunchKernelGGL((filter_fwd_x3_kernel<B, A>), dim3(gx, n), dim3(kThreadsX3), lds, s, pos, \
+                     pair_ij, pair_ij + pair_stride, n_pairs_dev, max_pairs, rp, fb)
     if (basis == 0 && act == 0) MLCG_X3_LAUNCH(0, 0);
     else if (basis == 0) MLCG_X3_LAUNCH(0, 1);
     else if (act == 0) MLCG_X3_LAUNCH(1, 0);
@@ -2311,9 +2385,8 @@ int filter_fwd_impl(const float* pos, const int32_t* pair_ij, int64_t pair_strid
     const size_t lds =
         sizeof(float) * (kFT * KS * MLCG_WAVE + kFT * kFT * MLCG_WAVE * 4 + 2 * kMaxK);
     allow_lds_once();
-    hipLaunchKernelGGL(filter_fwd_f32_kernel, dim3(groups), dim3(kThreads), lds, s, pos,
-                       pair_ij, pair_ij + pair_stride, n_pairs_dev, max_pairs, rp, W1, b1, W2,
-                       static_cast<float*>(W_out), static_cast<float*>(Wd_out), dist_out, gate);
+    hipLaunchKernelGGL(filter_fwd_f32_kernel, dim3(groups, n), dim3(kThreads), lds, s, pos,
+                       pair_ij, pair_ij + pair_stride, n_pairs_dev, max_pairs, rp, fb);
   } else {
     // K padded to 64 or 128 (two or four 32-wide k blocks)
     const int KS32 = num_rbf <= 64 ? 2 : 4;
@@ -2323,11 +2396,9 @@ int filter_fwd_impl(const float* pos, const int32_t* pair_ij, int64_t pair_strid
     allow_lds_once();
     const unsigned groups16 =
         mlcg_persistent_groups(mlcg_div_up(max_pairs, 16 * kWaves16), MLCG_F16_GROUPS_PER_CU);
-#define MLCG_F16_LAUNCH(KB, B, A)                                                             \
-  hipLaunchKernelGGL((filter_fwd_f16_kernel<KB, B, A>), dim3(groups16), dim3(kThreads16), lds, \
-                     s, pos, pair_ij, pair_ij + pair_stride, n_pairs_dev, max_pairs, rp, W1,   \
-                     b1, W2, static_cast<__half*>(W_out), static_cast<__half*>(Wd_out),       \
-                     dist_out, gate)
+#define MLCG_F16_LAUNCH(KB, B, A)                                                          \
+  hipLaunchKernelGGL((filter_fwd_f16_kernel<KB, B, A>), dim3(groups16, n), dim3(kThreads16), \
+                     lds, s, pos, pair_ij, pair_ij + pair_stride, n_pairs_dev, max_pairs, rp, fb)
 #define MLCG_F16_KB(KB)                                       \
   if (basis == 0 && act == 0) MLCG_F16_LAUNCH(KB, 0, 0);      \
   else if (basis == 0) MLCG_F16_LAUNCH(KB, 0, 1);             \
@@ -2354,23 +2425,46 @@ extern "C" int mlcg_filter_fwd(const float* pos, const int32_t* pair_ij, int64_t
                                const float* W1, const float* b1, const float* W2,
                                int num_filters, int f16, void* W_out, void* Wd_out,
                                float* dist_out, void* stream) {
-  return filter_fwd_impl(pos, pair_ij, pair_stride, n_pairs_dev, max_pairs, basis, centers, widths, alpha, num_rbf, rbf_cut_kind, rbf_lo, rbf_hi, conv_cut_kind, conv_lo, conv_hi, act, W1, b1, W2, num_filters, f16, W_out, Wd_out, dist_out, FilterGate{nullptr, 0}, stream);
+  FwdBatch fb = {};
+  fb.b[0] = FwdBlock{W1, b1, W2, W_out, Wd_out, dist_out, FilterGate{nullptr, 0}};
+  return filter_fwd_impl(pos, pair_ij, pair_stride, n_pairs_dev, max_pairs, basis, centers,
+                         widths, alpha, num_rbf, rbf_cut_kind, rbf_lo, rbf_hi, conv_cut_kind,
+                         conv_lo, conv_hi, act, num_filters, f16, fb, 1, stream);
 }
 
-extern "C" int mlcg_filter_fwd_gated(const float* pos, const int32_t* pair_ij, int64_t pair_stride,
-                               const int32_t* n_pairs_dev, int64_t max_pairs, int basis,
-                               const float* centers, const float* widths, float alpha,
-                               int num_rbf, int rbf_cut_kind, float rbf_lo, float rbf_hi,
-                               int conv_cut_kind, float conv_lo, float conv_hi, int act,
-                               const float* W1, const float* b1, const float* W2,
-                               int num_filters, int f16, void* W_out, void* Wd_out,
-                               float* dist_out, const uint32_t* gate, int gate_want, void* stream) {
-  return filter_fwd_impl(pos, pair_ij, pair_stride, n_pairs_dev, max_pairs, basis, centers, widths, alpha, num_rbf, rbf_cut_kind, rbf_lo, rbf_hi, conv_cut_kind, conv_lo, conv_hi, act, W1, b1, W2, num_filters, f16, W_out, Wd_out, dist_out, FilterGate{gate, gate_want}, stream);
+extern "C" int mlcg_filter_fwd_blocks(const float* pos, const int32_t* pair_ij,
+                                      int64_t pair_stride, const int32_t* n_pairs_dev,
+                                      int64_t max_pairs, int basis, const float* centers,
+                                      const float* widths, double alpha, int num_rbf,
+                                      int rbf_cut_kind, float rbf_lo, float rbf_hi,
+                                      int conv_cut_kind, float conv_lo, float conv_hi, int act,
+                                      const void* const* weights, void* const* outputs,
+                                      int num_blocks, int num_filters, int f16,
+                                      const uint32_t* gates, int gate_want, void* stream) {
+  MLCG_REQUIRE(weights && outputs && num_blocks >= 1);
+  for (int first = 0; first < num_blocks; first += kMaxBlocks) {
+    const int n = num_blocks - first < kMaxBlocks ? num_blocks - first : kMaxBlocks;
+    FwdBatch fb = {};
+    for (int k = 0; k < n; ++k) {
+      const void* const* w = weights + 3 * (first + k);
+      void* const* o = outputs + 2 * (first + k);
+      fb.b[k] = FwdBlock{static_cast<const float*>(w[0]), static_cast<const float*>(w[1]),
+                         static_cast<const float*>(w[2]), o[0], o[1], nullptr,
+                         FilterGate{gates ? gates + (first + k) * kGateWords : nullptr,
+                                    gate_want}};
+    }
+    const int st = filter_fwd_impl(pos, pair_ij, pair_stride, n_pairs_dev, max_pairs, basis,
+                                   centers, widths, alpha, num_rbf, rbf_cut_kind, rbf_lo, rbf_hi,
+                                   conv_cut_kind, conv_lo, conv_hi, act, num_filters, f16, fb, n,
+                                   stream);
+    if (st != MLCG_OK) return st;
+  }
+  return MLCG_OK;
 }
 
 extern "C" int mlcg_filter_table(const void* const* weights, int num_blocks, int nodes, float h,
                                  float rc, int basis, const float* centers, const float* widths,
-                                 float alpha, int num_rbf, int rbf_cut_kind, float rbf_lo,
+                                 double alpha, int num_rbf, int rbf_cut_kind, float rbf_lo,
                                  float rbf_hi, int conv_cut_kind, float conv_lo, float conv_hi,
                                  int act, int num_filters, float* tables, uint32_t* gates,
                                  void* stream) {
@@ -2405,28 +2499,31 @@ extern "C" int mlcg_filter_table(const void* const* weights, int num_blocks, int
 
 extern "C" int64_t mlcg_filter_bwd_workspace_floats(int64_t max_pairs, int num_rbf) {
   if (max_pairs < 0 || num_rbf < 1 || num_rbf > kMaxK) return -1;
-  return (int64_t)bwd_groups(max_pairs) * bwd_partial_floats(num_rbf);
+  return (int64_t)bwd_groups(max_pairs, 1) * bwd_partial_floats(num_rbf);
 }
 
 namespace {
 
+// n <= kMaxBlocks blocks, all from explicit pair adjoints or all from nodes.
 int launch_filter_bwd(const float* pos, const int32_t* pair_ij, int64_t pair_stride,
                       const int32_t* n_pairs_dev, int64_t max_pairs, int basis,
-                      const float* centers, const float* widths, float alpha, int num_rbf,
+                      const float* centers, const float* widths, double alpha, int num_rbf,
                       int rbf_cut_kind, float rbf_lo, float rbf_hi, int conv_cut_kind,
-                      float conv_lo, float conv_hi, int act, const float* W1, const float* b1,
-                      const float* W2, int num_filters, const PairAdjoint& adj, bool nodes,
-                      float* dW1, float* db1, float* dW2, float* abar_out, float* adbar_out,
-                      float* workspace, int64_t workspace_floats, bool fp32_strict,
-                      const FilterGate& gate, void* stream) {
+                      float conv_lo, float conv_hi, int act, int num_filters,
+                      const BwdBatch& batch, int n, bool nodes, float* workspace,
+                      int64_t workspace_floats, bool fp32_strict, void* stream) {
   if (!valid_params(basis, num_rbf, rbf_cut_kind, conv_cut_kind, act, num_filters))
     return MLCG_ERR_UNSUPPORTED;
   MLCG_REQUIRE(max_pairs >= 0 && pair_stride >= max_pairs);
-  MLCG_REQUIRE(centers && widths && W1 && b1 && W2 && dW1 && db1 && dW2 && workspace);
+  MLCG_REQUIRE(centers && widths && workspace);
   MLCG_REQUIRE(max_pairs == 0 || (pos && pair_ij && n_pairs_dev));
-  MLCG_REQUIRE((abar_out == nullptr) == (adbar_out == nullptr));
-  const int groups = bwd_groups(max_pairs);
-  MLCG_REQUIRE(workspace_floats >= (int64_t)groups * bwd_partial_floats(num_rbf));
+  for (int k = 0; k < n; ++k) {
+    const BwdBlock& b = batch.b[k];
+    MLCG_REQUIRE(b.W1 && b.b1 && b.W2 && b.dW1 && b.db1 && b.dW2);
+    MLCG_REQUIRE((b.abar == nullptr) == (b.adbar == nullptr));
+  }
+  const int groups = bwd_groups(max_pairs, n);
+  MLCG_REQUIRE(workspace_floats >= (int64_t)n * groups * bwd_partial_floats(num_rbf));
   RbfParams rp = make_params(basis, centers, widths, alpha, num_rbf, rbf_cut_kind, rbf_lo,
                              rbf_hi, conv_cut_kind, conv_lo, conv_hi, act);
   hipStream_t s = mlcg_stream(stream);
@@ -2437,10 +2534,9 @@ int launch_filter_bwd(const float* pos, const int32_t* pair_ij, int64_t pair_str
   allow_lds_once();
   const int grid = max_pairs == 0 ? 1 : groups;
 #define MLCG_BWD_LAUNCH(KS, NODES, B, A)                                                      \
-  hipLaunchKernelGGL((filter_bwd_fused_kernel<KS, NODES, B, A>), dim3(grid),                 \
+  hipLaunchKernelGGL((filter_bwd_fused_kernel<KS, NODES, B, A>), dim3(grid, n),              \
                      dim3(kBwdThreads), lds, s, pos, pair_ij, pair_ij + pair_stride,         \
-                     n_pairs_dev, max_pairs, rp, W1, b1, W2, adj, abar_out, adbar_out,       \
-                     workspace, gate)
+                     n_pairs_dev, max_pairs, rp, batch, workspace)
 #define MLCG_BWD_SMALL(NODES)                                   \
   if (basis == 0 && act == 0) MLCG_BWD_LAUNCH(16, NODES, 0, 0); \
   else if (basis == 0) MLCG_BWD_LAUNCH(16, NODES, 0, 1);        \
@@ -2458,31 +2554,12 @@ int launch_filter_bwd(const float* pos, const int32_t* pair_ij, int64_t pair_str
 #undef MLCG_BWD_SMALL
 #undef MLCG_BWD_LAUNCH
   const int total = kF * kF + kF * num_rbf + kF;
-  hipLaunchKernelGGL(filter_bwd_reduce_kernel, dim3((total + kRedOut - 1) / kRedOut), dim3(256),
-                     0, s, workspace, groups, num_rbf, dW1, db1, dW2, gate);
+  hipLaunchKernelGGL(filter_bwd_reduce_kernel, dim3((total + kRedOut - 1) / kRedOut, n),
+                     dim3(256), 0, s, workspace, groups, num_rbf, batch);
   return mlcg_launch_status();
 }
 
 }  // namespace
-
-static int filter_bwd_impl(const float* pos, const int32_t* pair_ij, int64_t pair_stride,
-                               const int32_t* n_pairs_dev, int64_t max_pairs, int basis,
-                               const float* centers, const float* widths, float alpha,
-                               int num_rbf, int rbf_cut_kind, float rbf_lo, float rbf_hi,
-                               int conv_cut_kind, float conv_lo, float conv_hi, int act,
-                               const float* W1, const float* b1, const float* W2,
-                               int num_filters, const float* Wbar, const float* Wdbar,
-                               float* dW1, float* db1, float* dW2, float* abar_out,
-                               float* adbar_out, float* workspace, int64_t workspace_floats,
-                               int fp32_strict, const FilterGate& gate, void* stream) {
-  MLCG_REQUIRE(max_pairs == 0 || (Wbar && Wdbar));
-  PairAdjoint adj{Wbar, Wdbar, nullptr, nullptr, nullptr, nullptr, nullptr};
-  return launch_filter_bwd(pos, pair_ij, pair_stride, n_pairs_dev, max_pairs, basis, centers,
-                           widths, alpha, num_rbf, rbf_cut_kind, rbf_lo, rbf_hi, conv_cut_kind,
-                           conv_lo, conv_hi, act, W1, b1, W2, num_filters, adj, false, dW1, db1,
-                           dW2, abar_out, adbar_out, workspace, workspace_floats,
-                           fp32_strict != 0, gate, stream);
-}
 
 extern "C" int mlcg_filter_bwd(const float* pos, const int32_t* pair_ij, int64_t pair_stride,
                                const int32_t* n_pairs_dev, int64_t max_pairs, int basis,
@@ -2494,42 +2571,14 @@ extern "C" int mlcg_filter_bwd(const float* pos, const int32_t* pair_ij, int64_t
                                float* dW1, float* db1, float* dW2, float* abar_out,
                                float* adbar_out, float* workspace, int64_t workspace_floats,
                                int fp32_strict, void* stream) {
-  return filter_bwd_impl(pos, pair_ij, pair_stride, n_pairs_dev, max_pairs, basis, centers, widths, alpha, num_rbf, rbf_cut_kind, rbf_lo, rbf_hi, conv_cut_kind, conv_lo, conv_hi, act, W1, b1, W2, num_filters, Wbar, Wdbar, dW1, db1, dW2, abar_out, adbar_out, workspace, workspace_floats, fp32_strict, FilterGate{nullptr, 0}, stream);
-}
-
-extern "C" int mlcg_filter_bwd_gated(const float* pos, const int32_t* pair_ij, int64_t pair_stride,
-                               const int32_t* n_pairs_dev, int64_t max_pairs, int basis,
-                               const float* centers, const float* widths, float alpha,
-                               int num_rbf, int rbf_cut_kind, float rbf_lo, float rbf_hi,
-                               int conv_cut_kind, float conv_lo, float conv_hi, int act,
-                               const float* W1, const float* b1, const float* W2,
-                               int num_filters, const float* Wbar, const float* Wdbar,
-                               float* dW1, float* db1, float* dW2, float* abar_out,
-                               float* adbar_out, float* workspace, int64_t workspace_floats,
-                               int fp32_strict, const uint32_t* gate, int gate_want, void* stream) {
-  return filter_bwd_impl(pos, pair_ij, pair_stride, n_pairs_dev, max_pairs, basis, centers, widths, alpha, num_rbf, rbf_cut_kind, rbf_lo, rbf_hi, conv_cut_kind, conv_lo, conv_hi, act, W1, b1, W2, num_filters, Wbar, Wdbar, dW1, db1, dW2, abar_out, adbar_out, workspace, workspace_floats, fp32_strict, FilterGate{gate, gate_want}, stream);
-}
-
-static int filter_bwd_cfconv_impl(const float* pos, const int32_t* pair_ij,
-                                      int64_t pair_stride, const int32_t* n_pairs_dev,
-                                      int64_t max_pairs, int basis, const float* centers,
-                                      const float* widths, float alpha, int num_rbf,
-                                      int rbf_cut_kind, float rbf_lo, float rbf_hi,
-                                      int conv_cut_kind, float conv_lo, float conv_hi, int act,
-                                      const float* W1, const float* b1, const float* W2,
-                                      int num_filters, const float* gagg2, const float* y,
-                                      const float* gagg1, const float* ydot,
-                                      const float* ddot, float* dW1, float* db1, float* dW2,
-                                      float* abar_out, float* adbar_out, float* workspace,
-                                      int64_t workspace_floats, int fp32_strict, const FilterGate& gate, void* stream) {
-  MLCG_REQUIRE(max_pairs == 0 || (gagg2 && y));
-  MLCG_REQUIRE(!gagg1 || ddot);
-  PairAdjoint adj{nullptr, nullptr, gagg2, y, gagg1, gagg1 ? ydot : nullptr, ddot};
+  MLCG_REQUIRE(max_pairs == 0 || (Wbar && Wdbar));
+  BwdBatch batch = {};
+  batch.b[0] = BwdBlock{W1, b1, W2, {Wbar, Wdbar, nullptr, nullptr, nullptr, nullptr, nullptr},
+                        abar_out, adbar_out, dW1, db1, dW2, {nullptr, 0}};
   return launch_filter_bwd(pos, pair_ij, pair_stride, n_pairs_dev, max_pairs, basis, centers,
                            widths, alpha, num_rbf, rbf_cut_kind, rbf_lo, rbf_hi, conv_cut_kind,
-                           conv_lo, conv_hi, act, W1, b1, W2, num_filters, adj, true, dW1, db1,
-                           dW2, abar_out, adbar_out, workspace, workspace_floats,
-                           fp32_strict != 0, gate, stream);
+                           conv_lo, conv_hi, act, num_filters, batch, 1, false, workspace,
+                           workspace_floats, fp32_strict != 0, stream);
 }
 
 extern "C" int mlcg_filter_bwd_cfconv(const float* pos, const int32_t* pair_ij,
@@ -2544,22 +2593,58 @@ extern "C" int mlcg_filter_bwd_cfconv(const float* pos, const int32_t* pair_ij,
                                       const float* ddot, float* dW1, float* db1, float* dW2,
                                       float* abar_out, float* adbar_out, float* workspace,
                                       int64_t workspace_floats, int fp32_strict, void* stream) {
-  return filter_bwd_cfconv_impl(pos, pair_ij, pair_stride, n_pairs_dev, max_pairs, basis, centers, widths, alpha, num_rbf, rbf_cut_kind, rbf_lo, rbf_hi, conv_cut_kind, conv_lo, conv_hi, act, W1, b1, W2, num_filters, gagg2, y, gagg1, ydot, ddot, dW1, db1, dW2, abar_out, adbar_out, workspace, workspace_floats, fp32_strict, FilterGate{nullptr, 0}, stream);
+  MLCG_REQUIRE(max_pairs == 0 || (gagg2 && y));
+  MLCG_REQUIRE(!gagg1 || ddot);
+  BwdBatch batch = {};
+  batch.b[0] = BwdBlock{W1, b1, W2,
+                        {nullptr, nullptr, gagg2, y, gagg1, gagg1 ? ydot : nullptr, ddot},
+                        abar_out, adbar_out, dW1, db1, dW2, {nullptr, 0}};
+  return launch_filter_bwd(pos, pair_ij, pair_stride, n_pairs_dev, max_pairs, basis, centers,
+                           widths, alpha, num_rbf, rbf_cut_kind, rbf_lo, rbf_hi, conv_cut_kind,
+                           conv_lo, conv_hi, act, num_filters, batch, 1, true, workspace,
+                           workspace_floats, fp32_strict != 0, stream);
 }
 
-extern "C" int mlcg_filter_bwd_cfconv_gated(const float* pos, const int32_t* pair_ij,
+extern "C" int64_t mlcg_filter_bwd_blocks_workspace_floats(int64_t max_pairs, int num_rbf,
+                                                           int num_blocks) {
+  if (max_pairs < 0 || num_rbf < 1 || num_rbf > kMaxK || num_blocks < 1) return -1;
+  const int n = num_blocks < kMaxBlocks ? num_blocks : kMaxBlocks;
+  return (int64_t)n * bwd_groups(max_pairs, n) * bwd_partial_floats(num_rbf);
+}
+
+extern "C" int mlcg_filter_bwd_blocks(const float* pos, const int32_t* pair_ij,
                                       int64_t pair_stride, const int32_t* n_pairs_dev,
                                       int64_t max_pairs, int basis, const float* centers,
-                                      const float* widths, float alpha, int num_rbf,
+                                      const float* widths, double alpha, int num_rbf,
                                       int rbf_cut_kind, float rbf_lo, float rbf_hi,
                                       int conv_cut_kind, float conv_lo, float conv_hi, int act,
-                                      const float* W1, const float* b1, const float* W2,
-                                      int num_filters, const float* gagg2, const float* y,
-                                      const float* gagg1, const float* ydot,
-                                      const float* ddot, float* dW1, float* db1, float* dW2,
-                                      float* abar_out, float* adbar_out, float* workspace,
-                                      int64_t workspace_floats, int fp32_strict, const uint32_t* gate, int gate_want, void* stream) {
-  return filter_bwd_cfconv_impl(pos, pair_ij, pair_stride, n_pairs_dev, max_pairs, basis, centers, widths, alpha, num_rbf, rbf_cut_kind, rbf_lo, rbf_hi, conv_cut_kind, conv_lo, conv_hi, act, W1, b1, W2, num_filters, gagg2, y, gagg1, ydot, ddot, dW1, db1, dW2, abar_out, adbar_out, workspace, workspace_floats, fp32_strict, FilterGate{gate, gate_want}, stream);
+                                      void* const* blocks, int num_blocks, int num_filters,
+                                      const uint32_t* gates, int gate_want, float* workspace,
+                                      int64_t workspace_floats, void* stream) {
+  MLCG_REQUIRE(blocks && num_blocks >= 1);
+  for (int first = 0; first < num_blocks; first += kMaxBlocks) {
+    const int n = num_blocks - first < kMaxBlocks ? num_blocks - first : kMaxBlocks;
+    BwdBatch batch = {};
+    bool nodes = false;
+    for (int k = 0; k < n; ++k) {
+      auto at = [&](int x) { return static_cast<float*>(blocks[15 * (first + k) + x]); };
+      BwdBlock& b = batch.b[k];
+      b = BwdBlock{at(0), at(1), at(2),
+                   {at(3), at(4), at(5), at(6), at(7), at(7) ? at(8) : nullptr, at(9)},
+                   at(13), at(14), at(10), at(11), at(12),
+                   {gates ? gates + (first + k) * kGateWords : nullptr, gate_want}};
+      const bool node_form = b.adj.g2 != nullptr;
+      MLCG_REQUIRE(k == 0 || node_form == nodes);
+      nodes = node_form;
+      MLCG_REQUIRE(nodes ? b.adj.y && (!b.adj.g1 || b.adj.dd) : b.adj.Wbar && b.adj.Wdbar);
+    }
+    const int st = launch_filter_bwd(pos, pair_ij, pair_stride, n_pairs_dev, max_pairs, basis,
+                                     centers, widths, alpha, num_rbf, rbf_cut_kind, rbf_lo,
+                                     rbf_hi, conv_cut_kind, conv_lo, conv_hi, act, num_filters,
+                                     batch, n, nodes, workspace, workspace_floats, false, stream);
+    if (st != MLCG_OK) return st;
+  }
+  return MLCG_OK;
 }
 
 // ---------------------------------------------------------------------------
@@ -2584,7 +2669,7 @@ constexpr int kRgMaxGroups = 512;
 __device__ __forceinline__ float exp_of(float x) { return __expf(x); }
 __device__ __forceinline__ double exp_of(double x) { return exp(x); }
 
-// T: double on the nodes of a table (see rbf_expnormal_fine), else float.
+// T: double on the nodes of a table, else float.
 template <typename T>
 __device__ __forceinline__ void basis_param_derivs(const RbfParams& rp, T cen, T wid, T d, T C,
                                                    T dC, T& g_c, T& g_w, T& gd_c, T& gd_w) {
@@ -2598,7 +2683,7 @@ __device__ __forceinline__ void basis_param_derivs(const RbfParams& rp, T cen, T
     gd_c = -e * (T(2) * c * x * q + T(2) * c * C);  // dg'/dcenter
     gd_w = e * (x * x * q + T(2) * x * C);         // dg'/dc
   } else {
-    const T alpha = rp.alpha;
+    const T alpha = (T)(sizeof(T) == 8 ? rp.alpha64 : (double)rp.alpha);
     const T ex = exp_of(alpha * (T(rp.rbf_lo) - d));
     const T u = ex - cen;
     const T b = wid;
@@ -2725,6 +2810,7 @@ __global__ void rbf_grad_reduce_kernel(const float* __restrict__ partial, int gr
   const int which = x / kp, k = x % kp;
   if (k >= K) return;
   float v = 0.f;
+#pragma unroll 16  // loads in flight; the order of the sum stays
   for (int g = 0; g < groups; ++g) v += partial[(int64_t)g * 2 * kp + x];
   float* dst = which == 0 ? dcenters + k : dwidths + k;
   *dst = accumulate ? *dst + v : v;
@@ -2745,7 +2831,7 @@ extern "C" int64_t mlcg_rbf_param_grad_workspace_floats(int64_t max_pairs, int n
 
 static int rbf_param_grad_impl(const float* dist, const int32_t* n_pairs_dev,
                                    int64_t max_pairs, int basis, const float* centers,
-                                   const float* widths, float alpha, int num_rbf,
+                                   const float* widths, double alpha, int num_rbf,
                                    int rbf_cut_kind, float rbf_lo, float rbf_hi,
                                    const float* W1, int num_filters, const float* abar,
                                    const float* adbar, int accumulate, float* dcenters,
@@ -2797,7 +2883,7 @@ extern "C" int mlcg_rbf_param_grad(const float* dist, const int32_t* n_pairs_dev
 
 extern "C" int mlcg_rbf_param_grad_gated(const float* dist, const int32_t* n_pairs_dev,
                                    int64_t max_pairs, int basis, const float* centers,
-                                   const float* widths, float alpha, int num_rbf,
+                                   const float* widths, double alpha, int num_rbf,
                                    int rbf_cut_kind, float rbf_lo, float rbf_hi,
                                    const float* W1, int num_filters, const float* abar,
                                    const float* adbar, int accumulate, float* dcenters,

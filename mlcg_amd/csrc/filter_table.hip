@@ -7,8 +7,9 @@
 // interpolated from four nodes (cubic Lagrange, values and derivatives each
 // from their own table), and the reverse of that interpolation gives the
 // adjoints of the nodes, on which the filter backward then runs.  The grid
-// spacing has 11 significant bits and the grid below 2^13 nodes, so the node
-// distances are exact in fp32, and so is a pair's distance from its node.
+// spacing has 11 significant bits and the grid at most 2^13 nodes, so the node
+// distances are exact in fp32; a pair's place between them comes from its
+// distance in double.
 //
 // The pairs are ordered by their interpolation stencil once per call (a
 // stable counting sort: mlcg_pair_bins), so that a wave reads a stencil's
@@ -30,20 +31,30 @@ constexpr int kMaxKeys = 8192;
 constexpr int kRev = 64;      // records of a run (table_reverse_kernel)
 constexpr int kRevWaves = 8;  // runs of a workgroup
 
-// Stencil of a distance: nodes key .. key + 3, clamped to the grid.
-__device__ __forceinline__ int stencil_key(float d, float inv_h, int nkeys) {
-  const int b = (int)(d * inv_h) - 1;
+// Position of a pair in the grid, in cells: 14 integer and 18 fraction bits,
+// from the distance in double.  A float distance is off by up to 1e-6 A at 20
+// A, the largest single error of the pairwise filters (5.4e-7 of the weight
+// gradients); the fraction here resolves 3e-8 A.  kPastCut: at or past the
+// cutoff of a cosine envelope, where the filter is zero.
+constexpr int kFracBits = 18;
+constexpr uint32_t kPastCut = 0xffffffffu;
+
+__device__ __forceinline__ uint32_t grid_position(double d, double inv_h) {
+  const double u = d * inv_h * (double)(1 << kFracBits);
+  return u < 4294967294.0 ? (uint32_t)u : 0xfffffffeu;
+}
+
+// Stencil of a position: nodes key .. key + 3, clamped to the grid.
+__device__ __forceinline__ int stencil_key(uint32_t u, int nkeys) {
+  const int b = (int)(u >> kFracBits) - 1;
   return b < 0 ? 0 : (b > nkeys - 1 ? nkeys - 1 : b);
 }
 
-// Cubic Lagrange weights at position t (in cells) from the stencil's first
-// node; zero past the cutoff distance of a cosine envelope (cut), where the
-// filter is zero.
-__device__ __forceinline__ void stencil_weights(float d, float h, float inv_h, int key, float cut,
-                                                float w[4]) {
-  const float t0 = fmaf(-(float)key, h, d) * inv_h;
+// Cubic Lagrange weights from the stencil's first node; zero past the cutoff.
+__device__ __forceinline__ void stencil_weights(uint32_t u, int key, float w[4]) {
+  const float t0 = (float)(u - ((uint32_t)key << kFracBits)) * (1.0f / (1 << kFracBits));
   const float t1 = t0 - 1.0f, t2 = t0 - 2.0f, t3 = t0 - 3.0f;
-  const float m = d < cut ? 1.0f : 0.0f;
+  const float m = u != kPastCut ? 1.0f : 0.0f;
   const float a = t0 * t1 * m, b = t2 * t3 * m;
   w[0] = t1 * b * (-1.0f / 6.0f);
   w[1] = t0 * b * 0.5f;
@@ -68,8 +79,9 @@ __device__ __forceinline__ void wave_range(int64_t np, int blk, int groups, int 
 // Counts of every key among the block's pairs, and the pair distances.
 __global__ __launch_bounds__(kSortThreads) void pair_key_count_kernel(
     const float* __restrict__ pos, const int32_t* __restrict__ pi,
-    const int32_t* __restrict__ pj, const int32_t* __restrict__ n_dev, int64_t cap, float inv_h,
-    int nkeys, float* __restrict__ dist, uint32_t* __restrict__ hist) {
+    const int32_t* __restrict__ pj, const int32_t* __restrict__ n_dev, int64_t cap, double inv_h,
+    int nkeys, float cut, float* __restrict__ dist, uint32_t* __restrict__ where,
+    uint32_t* __restrict__ hist) {
   extern __shared__ uint32_t cnt[];  // [nkeys]
   for (int b = threadIdx.x; b < nkeys; b += kSortThreads) cnt[b] = 0u;
   __syncthreads();
@@ -80,13 +92,17 @@ __global__ __launch_bounds__(kSortThreads) void pair_key_count_kernel(
 #pragma unroll 4
   for (int64_t p = lo + mlcg_lane(); p < hi; p += MLCG_WAVE) {
     const int64_t i = pi[p], j = pj[p];
-    const float dx = pos[3 * j + 0] - pos[3 * i + 0];
-    const float dy = pos[3 * j + 1] - pos[3 * i + 1];
-    const float dz = pos[3 * j + 2] - pos[3 * i + 2];
+    const float xi = pos[3 * i], yi = pos[3 * i + 1], zi = pos[3 * i + 2];
+    const float xj = pos[3 * j], yj = pos[3 * j + 1], zj = pos[3 * j + 2];
+    const float dx = xj - xi, dy = yj - yi, dz = zj - zi;
     // the filter forward's own fma order, so both routes have the same distances
     const float d = sqrtf(fmaf(dz, dz, fmaf(dy, dy, dx * dx)));
     dist[p] = d;
-    atomicAdd(&cnt[stencil_key(d, inv_h, nkeys)], 1u);
+    const double ex = (double)xj - xi, ey = (double)yj - yi, ez = (double)zj - zi;
+    const uint32_t u =
+        d < cut ? grid_position(sqrt(ex * ex + ey * ey + ez * ez), inv_h) : kPastCut;
+    where[p] = u;
+    atomicAdd(&cnt[stencil_key(u, nkeys)], 1u);
   }
   __syncthreads();
   uint32_t* h = hist + (int64_t)blockIdx.x * nkeys;
@@ -121,12 +137,12 @@ __global__ __launch_bounds__(256) void pair_key_offsets_kernel(uint32_t* __restr
   if (s == 3 && b < nkeys) totals[b] = run;
 }
 
-// Writes the records {pair, i, j, distance bits} in key order, stable in the
+// Writes the records {pair, i, j, grid position} in key order, stable in the
 // pair index, and the keys' first positions.
 __global__ __launch_bounds__(kSortThreads) void pair_key_scatter_kernel(
     const int32_t* __restrict__ pi, const int32_t* __restrict__ pj,
-    const int32_t* __restrict__ n_dev, int64_t cap, float inv_h, int nkeys,
-    const float* __restrict__ dist, const uint32_t* __restrict__ hist,
+    const int32_t* __restrict__ n_dev, int64_t cap, int nkeys,
+    const uint32_t* __restrict__ where, const uint32_t* __restrict__ hist,
     const uint32_t* __restrict__ totals, int32_t* __restrict__ start,
     int32_t* __restrict__ run_start, int4* __restrict__ recs) {
   extern __shared__ uint32_t off[];  // [kSortWaves][nkeys]
@@ -141,7 +157,7 @@ __global__ __launch_bounds__(kSortThreads) void pair_key_scatter_kernel(
   uint32_t* mine = off + (w < kSortWaves ? w : 0) * nkeys;
 #pragma unroll 4
   for (int64_t p = lo + l; p < hi; p += MLCG_WAVE)
-    atomicAdd(&mine[stencil_key(dist[p], inv_h, nkeys)], 1u);
+    atomicAdd(&mine[stencil_key(where[p], nkeys)], 1u);
   // first record and first run of every key: exclusive scans of the totals and
   // of the runs (of at most kRev records) they make, each thread over its own
   // stretch of consecutive keys
@@ -196,8 +212,8 @@ __global__ __launch_bounds__(kSortThreads) void pair_key_scatter_kernel(
   for (int64_t p0 = lo; p0 < hi; p0 += MLCG_WAVE) {
     const int64_t p = p0 + l;
     const bool on = p < hi;
-    const float d = on ? dist[p] : 0.0f;
-    const int key = stencil_key(d, inv_h, nkeys);
+    const uint32_t u = on ? where[p] : 0u;
+    const int key = stencil_key(u, nkeys);
     // lanes of this wave with the same key
     unsigned long long same = __ballot(on);
 #pragma unroll
@@ -209,7 +225,7 @@ __global__ __launch_bounds__(kSortThreads) void pair_key_scatter_kernel(
     if (on) {
       const int rank = __popcll(same & ((1ull << l) - 1ull));
       const uint32_t base = *(volatile uint32_t*)&mine[key];
-      const int4 r = int4{(int)p, pi[p], pj[p], __float_as_int(d)};
+      const int4 r = int4{(int)p, pi[p], pj[p], (int)u};
       recs[base + rank] = r;
       // the first lane of the group moves the counter past it, after every
       // lane of the group has read it (one wave: LDS operations in program
@@ -315,12 +331,21 @@ __device__ __forceinline__ float4 lerp4(const float4* r, const float w[4]) {
                 r[0].w * w[0] + r[1].w * w[1] + r[2].w * w[2] + r[3].w * w[3]};
 }
 
+constexpr int kMaxBlocks = 8;  // blocks of a launch (blockIdx.y)
+struct RowsBatch {
+  void *W[kMaxBlocks], *Wd[kMaxBlocks];
+};
+
 template <typename T>
 __global__ __launch_bounds__(256) void table_rows_kernel(
-    const int4* __restrict__ recs, const int32_t* __restrict__ n_dev, int64_t cap, float h,
-    float inv_h, int nkeys, float cut, const float* __restrict__ table, int64_t plane, FilterGate gate,
-    T* __restrict__ W, T* __restrict__ Wd) {
-  if (gate_closed(gate)) return;
+    const int4* __restrict__ recs, const int32_t* __restrict__ n_dev, int64_t cap, int nkeys,
+    const float* __restrict__ tables, int64_t plane,
+    const unsigned* __restrict__ gates, RowsBatch batch) {
+  const int blk = blockIdx.y;
+  if (!filter_table_serves(gates + blk * kGateWords)) return;
+  const float* __restrict__ table = tables + (int64_t)blk * 4 * plane;
+  T* __restrict__ W = static_cast<T*>(batch.W[blk]);
+  T* __restrict__ Wd = static_cast<T*>(batch.Wd[blk]);
   const int64_t np = live_pairs(n_dev, cap);
   const int l = mlcg_lane(), hl = l & 31, hb = l & 32;
   const int64_t s0 = ((int64_t)blockIdx.x * 8 + (threadIdx.x >> 5)) * kSeg;
@@ -332,8 +357,8 @@ __global__ __launch_bounds__(256) void table_rows_kernel(
   int cur = -1;
   for (int k = 0; k < n; ++k) {
     const int p = __shfl(r.x, hb | k, MLCG_WAVE);
-    const float d = __int_as_float(__shfl(r.w, hb | k, MLCG_WAVE));
-    const int key = stencil_key(d, inv_h, nkeys);
+    const uint32_t u = (uint32_t)__shfl(r.w, hb | k, MLCG_WAVE);
+    const int key = stencil_key(u, nkeys);
     if (key != cur) {
       const float* c = table + (int64_t)key * kF + f;
 #pragma unroll
@@ -344,7 +369,7 @@ __global__ __launch_bounds__(256) void table_rows_kernel(
       cur = key;
     }
     float w[4];
-    stencil_weights(d, h, inv_h, key, cut, w);
+    stencil_weights(u, key, w);
     store_row4(W + (int64_t)p * kF, f, lerp4(tw, w));
     store_row4(Wd + (int64_t)p * kF, f, lerp4(td, w));
   }
@@ -397,8 +422,7 @@ __device__ __forceinline__ int run_key(const int32_t* __restrict__ run_start, in
 template <bool kTan, bool kYd>
 __global__ __launch_bounds__(kRevWaves * MLCG_WAVE) void table_reverse_kernel(
     const int4* __restrict__ recs, const int32_t* __restrict__ start,
-    const int32_t* __restrict__ run_start, float h, float inv_h, int nkeys, float cut,
-    const float* __restrict__ g2, const float* __restrict__ y, const float* __restrict__ g1,
+    const int32_t* __restrict__ run_start, int nkeys, const float* __restrict__ g2, const float* __restrict__ y, const float* __restrict__ g1,
     const float* __restrict__ yd, const float* __restrict__ dd, FilterGate gate,
     float* __restrict__ slots) {
   if (gate_closed(gate)) return;
@@ -418,7 +442,7 @@ __global__ __launch_bounds__(kRevWaves * MLCG_WAVE) void table_reverse_kernel(
   const int4 r = recs[s0 + (l < n ? l : n - 1) * parts];
   const float ddl = kTan ? dd[r.x] : 0.0f;
   float w_l[4];
-  stencil_weights(__int_as_float(r.w), h, inv_h, key, cut, w_l);
+  stencil_weights((uint32_t)r.w, key, w_l);
   const int f = 2 * l;
   float2 aw[4], ad[4];
 #pragma unroll
@@ -529,9 +553,14 @@ __device__ __forceinline__ void add_slots(const float* __restrict__ o, int first
 
 template <bool kTan>
 __global__ __launch_bounds__(256) void table_combine_kernel(
-    const int32_t* __restrict__ run_start, int nkeys, const float* __restrict__ slots, int nodes,
-    FilterGate gate, float* __restrict__ wbar, float* __restrict__ wdbar) {
-  if (gate_closed(gate)) return;
+    const int32_t* __restrict__ run_start, int nkeys, const float* __restrict__ block_slots,
+    int64_t slot_stride, int nodes, const unsigned* __restrict__ gates,
+    float* __restrict__ block_wbar, float* __restrict__ block_wdbar) {
+  const int blk = blockIdx.y;
+  if (!filter_table_serves(gates + blk * kGateWords)) return;
+  const float* __restrict__ slots = block_slots + blk * slot_stride;
+  float* __restrict__ wbar = block_wbar + (int64_t)blk * nodes * kF;
+  float* __restrict__ wdbar = block_wdbar + (int64_t)blk * nodes * kF;
   __shared__ float2 part[4][2][MLCG_WAVE];
   const int m = blockIdx.x, l = mlcg_lane();
   const int x = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
@@ -580,40 +609,41 @@ void allow_sort_lds_once() {
   done[dev] = true;
 }
 
-bool table_shape_ok(int nodes) { return nodes >= 16 && nodes - 3 <= kMaxKeys; }
+bool table_shape_ok(int nodes) { return nodes >= 16 && nodes <= kMaxKeys; }
 
 }  // namespace
 
 extern "C" int64_t mlcg_pair_bins_workspace_ints(int64_t max_pairs, int nodes) {
   if (max_pairs < 0 || !table_shape_ok(nodes)) return -1;
-  return (int64_t)(sort_groups(max_pairs) + 1) * (nodes - 3);
+  return (int64_t)(sort_groups(max_pairs) + 1) * (nodes - 3) + max_pairs;
 }
 
 extern "C" int mlcg_pair_bins(const float* pos, const int32_t* pair_ij, int64_t pair_stride,
                               const int32_t* n_pairs_dev, int64_t max_pairs, float h,
-                              int nodes, float* dist, int32_t* start, int32_t* run_start,
+                              int nodes, float cut, float* dist, int32_t* start, int32_t* run_start,
                               int32_t* records,
                               int32_t* workspace, int64_t workspace_ints, void* stream) {
   MLCG_REQUIRE(max_pairs >= 0 && max_pairs < (1LL << 31) && pair_stride >= max_pairs);
   MLCG_REQUIRE(table_shape_ok(nodes) && h > 0.0f);
-  const float inv_h = 1.0f / h;
+  const double inv_h = 1.0 / (double)h;
   MLCG_REQUIRE(pos && pair_ij && n_pairs_dev && dist && start && run_start && records &&
                workspace);
   const int nkeys = nodes - 3;
   const int groups = sort_groups(max_pairs);
-  MLCG_REQUIRE(workspace_ints >= (int64_t)(groups + 1) * nkeys);
+  MLCG_REQUIRE(workspace_ints >= (int64_t)(groups + 1) * nkeys + max_pairs);
   uint32_t* totals = reinterpret_cast<uint32_t*>(workspace);
   uint32_t* hist = totals + nkeys;
+  uint32_t* where = hist + (int64_t)groups * nkeys;
   hipStream_t s = mlcg_stream(stream);
   allow_sort_lds_once();
   hipLaunchKernelGGL(pair_key_count_kernel, dim3(groups), dim3(kSortThreads),
                      sizeof(uint32_t) * nkeys, s, pos, pair_ij, pair_ij + pair_stride,
-                     n_pairs_dev, max_pairs, inv_h, nkeys, dist, hist);
+                     n_pairs_dev, max_pairs, inv_h, nkeys, cut, dist, where, hist);
   hipLaunchKernelGGL(pair_key_offsets_kernel, dim3(mlcg_div_up(nkeys, MLCG_WAVE)), dim3(256), 0,
                      s, hist, groups, nkeys, totals);
   hipLaunchKernelGGL(pair_key_scatter_kernel, dim3(groups), dim3(kSortThreads),
                      sizeof(uint32_t) * kSortWaves * nkeys, s, pair_ij, pair_ij + pair_stride,
-                     n_pairs_dev, max_pairs, inv_h, nkeys, dist, hist, totals, start, run_start,
+                     n_pairs_dev, max_pairs, nkeys, where, hist, totals, start, run_start,
                      reinterpret_cast<int4*>(records));
   return mlcg_launch_status();
 }
@@ -628,24 +658,33 @@ extern "C" int mlcg_filter_table_check(const float* tables, int num_blocks, int 
 }
 
 extern "C" int mlcg_filter_table_rows(const int32_t* records, const int32_t* n_pairs_dev,
-                                      int64_t max_pairs, float h, int nodes, float cut,
-                                      const float* table, const uint32_t* gate, int f16, void* W,
-                                      void* Wd, void* stream) {
-  MLCG_REQUIRE(table_shape_ok(nodes) && max_pairs >= 0);
+                                      int64_t max_pairs, int nodes, const float* tables, const uint32_t* gates, int num_blocks,
+                                      int f16, void* const* outputs, void* stream) {
+  MLCG_REQUIRE(table_shape_ok(nodes) && max_pairs >= 0 && num_blocks >= 1);
   if (max_pairs == 0) return MLCG_OK;
-  MLCG_REQUIRE(records && n_pairs_dev && table && gate && W && Wd);
+  MLCG_REQUIRE(records && n_pairs_dev && tables && gates && outputs);
   const int64_t plane = (int64_t)(nodes + 1) * kF;
-  const FilterGate g{gate, 1};
-  const dim3 grid(mlcg_div_up(max_pairs, 8 * kSeg));
   const int4* recs = reinterpret_cast<const int4*>(records);
-  if (f16)
-    hipLaunchKernelGGL((table_rows_kernel<__half>), grid, dim3(256), 0, mlcg_stream(stream),
-                       recs, n_pairs_dev, max_pairs, h, 1.0f / h, nodes - 3, cut, table, plane, g,
-                       static_cast<__half*>(W), static_cast<__half*>(Wd));
-  else
-    hipLaunchKernelGGL((table_rows_kernel<float>), grid, dim3(256), 0, mlcg_stream(stream),
-                       recs, n_pairs_dev, max_pairs, h, 1.0f / h, nodes - 3, cut, table, plane, g,
-                       static_cast<float*>(W), static_cast<float*>(Wd));
+  for (int first = 0; first < num_blocks; first += kMaxBlocks) {
+    const int n = num_blocks - first < kMaxBlocks ? num_blocks - first : kMaxBlocks;
+    RowsBatch batch = {};
+    for (int k = 0; k < n; ++k) {
+      batch.W[k] = outputs[2 * (first + k)];
+      batch.Wd[k] = outputs[2 * (first + k) + 1];
+      MLCG_REQUIRE(batch.W[k] && batch.Wd[k]);
+    }
+    const dim3 grid(mlcg_div_up(max_pairs, 8 * kSeg), n);
+    const float* t = tables + (int64_t)first * 4 * plane;
+    const uint32_t* g = gates + first * kGateWords;
+    if (f16)
+      hipLaunchKernelGGL((table_rows_kernel<__half>), grid, dim3(256), 0, mlcg_stream(stream),
+                         recs, n_pairs_dev, max_pairs, nodes - 3, t, plane, g,
+                         batch);
+    else
+      hipLaunchKernelGGL((table_rows_kernel<float>), grid, dim3(256), 0, mlcg_stream(stream),
+                         recs, n_pairs_dev, max_pairs, nodes - 3, t, plane, g,
+                         batch);
+  }
   return mlcg_launch_status();
 }
 
@@ -655,17 +694,15 @@ extern "C" int64_t mlcg_filter_table_reverse_workspace_floats(int64_t max_pairs,
 }
 
 extern "C" int mlcg_filter_table_reverse(const int32_t* records, const int32_t* start,
-                                         const int32_t* run_start, int64_t max_pairs, float h,
-                                         int nodes, float cut, const float* gagg2,
+                                         const int32_t* run_start, int64_t max_pairs, int nodes,
+                                         const float* gagg2,
                                          const float* y, const float* gagg1, const float* ydot,
-                                         const float* ddot, const uint32_t* gate, float* wbar,
-                                         float* wdbar, float* workspace,
-                                         int64_t workspace_floats, void* stream) {
+                                         const float* ddot, const uint32_t* gate, float* slots,
+                                         int64_t slot_floats, void* stream) {
   MLCG_REQUIRE(table_shape_ok(nodes) && max_pairs >= 0);
-  MLCG_REQUIRE(records && start && run_start && gagg2 && y && gate && wbar && wdbar &&
-               workspace);
+  MLCG_REQUIRE(records && start && run_start && gagg2 && y && gate && slots);
   MLCG_REQUIRE(!gagg1 || ddot);
-  MLCG_REQUIRE(workspace_floats >= mlcg_filter_table_reverse_workspace_floats(max_pairs, nodes));
+  MLCG_REQUIRE(slot_floats >= mlcg_filter_table_reverse_workspace_floats(max_pairs, nodes));
   const FilterGate g{gate, 1};
   const int nkeys = nodes - 3;
   const int4* recs = reinterpret_cast<const int4*>(records);
@@ -674,7 +711,7 @@ extern "C" int mlcg_filter_table_reverse(const int32_t* records, const int32_t* 
   const dim3 grid(mlcg_div_up((max_pairs + kRev - 1) / kRev + nkeys, kRevWaves));
 #define MLCG_REV(T, Y)                                                                        \
   hipLaunchKernelGGL((table_reverse_kernel<T, Y>), grid, dim3(kRevWaves * MLCG_WAVE), 0, s, recs, start,      \
-                     run_start, h, 1.0f / h, nkeys, cut, gagg2, y, gagg1, ydot, ddot, g, workspace)
+                     run_start, nkeys, gagg2, y, gagg1, ydot, ddot, g, slots)
   if (gagg1 && ydot)
     MLCG_REV(true, true);
   else if (gagg1)
@@ -682,12 +719,22 @@ extern "C" int mlcg_filter_table_reverse(const int32_t* records, const int32_t* 
   else
     MLCG_REV(false, false);
 #undef MLCG_REV
-  const dim3 cgrid(nodes);
-  if (gagg1)
-    hipLaunchKernelGGL((table_combine_kernel<true>), cgrid, dim3(256), 0, s, run_start,
-                       nkeys, workspace, nodes, g, wbar, wdbar);
+  return mlcg_launch_status();
+}
+
+extern "C" int mlcg_filter_table_combine(const int32_t* run_start, int64_t max_pairs, int nodes,
+                                         int tangent, const float* slots, int num_blocks,
+                                         const uint32_t* gates, float* wbar, float* wdbar,
+                                         void* stream) {
+  MLCG_REQUIRE(table_shape_ok(nodes) && max_pairs >= 0 && num_blocks >= 1);
+  MLCG_REQUIRE(run_start && slots && gates && wbar && wdbar);
+  const int64_t stride = mlcg_filter_table_reverse_workspace_floats(max_pairs, nodes);
+  const dim3 grid(nodes, num_blocks);
+  if (tangent)
+    hipLaunchKernelGGL((table_combine_kernel<true>), grid, dim3(256), 0, mlcg_stream(stream),
+                       run_start, nodes - 3, slots, stride, nodes, gates, wbar, wdbar);
   else
-    hipLaunchKernelGGL((table_combine_kernel<false>), cgrid, dim3(256), 0, s, run_start,
-                       nkeys, workspace, nodes, g, wbar, wdbar);
+    hipLaunchKernelGGL((table_combine_kernel<false>), grid, dim3(256), 0, mlcg_stream(stream),
+                       run_start, nodes - 3, slots, stride, nodes, gates, wbar, wdbar);
   return mlcg_launch_status();
 }

@@ -303,43 +303,28 @@ def _table_grid(spec: FusedSpec, filt, graph: ops.PairGraph, pos: torch.Tensor, 
     return grid
 
 
-def _start_tables(spec: FusedSpec, P: Params, st: "State", pos, graph) -> torch.Tensor:
-    """The blocks' filter tables (returned) and their gate words, on the side
-    stream while the caller's stream orders the pairs: the tables depend on the
-    weights alone.  Their buffers belong to the caller's stream, which waits for
-    the side stream before it goes on."""
+def _filter_weights(P: Params):
+    return [(bp.W1, bp.b1, bp.W2) for bp in P.blocks]
+
+
+def _table_filters(spec: FusedSpec, P: Params, st: "State", pos, graph) -> dict:
+    """{k: (W, Wd, None)} of every block through its table.  The tables, which
+    depend on the weights alone, are made on the side stream while the caller's
+    stream orders the pairs; their buffers belong to the caller's stream, which
+    waits for the side stream before it goes on."""
     main = torch.cuda.current_stream(pos.device)
     side = _side_stream(main)
-    out = ops.filter_table_buffers(st.grid, len(P.blocks))
+    weights = _filter_weights(P)
+    tables, st.gates = out = ops.filter_table_buffers(st.grid, len(P.blocks))
     side.wait_stream(main)
     with torch.cuda.stream(side):
-        ops.filter_tables(st.grid, st.filt, [(bp.W1, bp.b1, bp.W2) for bp in P.blocks], out=out)
+        ops.filter_tables(st.grid, st.filt, weights, out=out)
     st.bins = ops.pair_bins(pos, graph, st.grid)
     st.dist = st.bins.dist
     main.wait_stream(side)
-    st.gates = out[1]
-    return out[0]
-
-
-def _block_filters(spec: FusedSpec, P: Params, st: "State", pos, graph, tables, k: int,
-                   out=None):
-    """(W, Wd) of block k, from its table where that serves."""
-    bp = P.blocks[k]
-    if st.grid is None:
-        W, Wd, dist = ops.filter_fwd(pos, graph, st.filt, bp.W1, bp.b1, bp.W2, f16=spec.f16,
-                                     want_dist=(k == 0), strict_fp32=spec.strict_fp32, out=out)
-        if k == 0:
-            st.dist = dist
-        return W, Wd
-    if out is None:
-        dt = torch.float16 if spec.f16 else torch.float32
-        shape = (graph.pair_capacity, ops.NUM_FILTERS)
-        out = (torch.empty(shape, dtype=dt, device=pos.device),
-               torch.empty(shape, dtype=dt, device=pos.device))
-    ops.filter_table_rows(st.grid, st.bins, graph, tables[k], st.gates[k], out)
-    ops.filter_fwd(pos, graph, st.filt, bp.W1, bp.b1, bp.W2, f16=spec.f16, want_dist=False,
-                   out=out, gate=st.gates[k])
-    return out
+    rows = ops.filter_rows(st.grid, st.bins, pos, graph, st.filt, weights, tables, st.gates,
+                           f16=spec.f16)
+    return {k: (W, Wd, None) for k, (W, Wd) in enumerate(rows)}
 
 
 # Filter forwards of blocks 1.. on the side stream (MLCG_FILTER_AHEAD=0 keeps
@@ -347,9 +332,9 @@ def _block_filters(spec: FusedSpec, P: Params, st: "State", pos, graph, tables, 
 _FILTER_AHEAD = os.environ.get("MLCG_FILTER_AHEAD", "1") != "0"
 
 
-def _filters_ahead(spec: FusedSpec, P: Params, st: "State", pos: torch.Tensor,
-                   graph: ops.PairGraph, tables) -> dict:
-    """Issues the filter forwards of blocks 1.. on the side stream at the start
+def _filters_ahead(spec: FusedSpec, P: Params, pos: torch.Tensor, graph: ops.PairGraph,
+                   filt) -> dict:
+    """Issues the pair-by-pair filter forwards of blocks 1.. on the side stream at the start
     of the forward: they depend only on the pair distances and the block's
     filter weights, not on node features, so they run beside block 0's node
     linears and gathers (memory-bound work that leaves VGPRs and LDS free on
@@ -369,7 +354,10 @@ def _filters_ahead(spec: FusedSpec, P: Params, st: "State", pos: torch.Tensor,
     ahead = {}
     with torch.cuda.stream(side):
         for k in range(1, len(P.blocks)):
-            W, Wd = _block_filters(spec, P, st, pos, graph, tables, k, out=outs[k])
+            bp = P.blocks[k]
+            W, Wd, _ = ops.filter_fwd(pos, graph, filt, bp.W1, bp.b1, bp.W2, f16=spec.f16,
+                                      want_dist=False, strict_fp32=spec.strict_fp32,
+                                      out=outs[k])
             ev = torch.cuda.Event()
             ev.record(side)
             ahead[k] = (W, Wd, ev)
@@ -423,16 +411,20 @@ def forward(spec: FusedSpec, P: Params, pos: torch.Tensor, types: torch.Tensor,
     # otherwise hold every CU while this short launch waits for one
     st.wimg = _weight_images(P, x, transposed=save)
     st.grid = _table_grid(spec, st.filt, graph, pos, reverse)
-    tables = None
     if st.grid is not None:
-        tables = _start_tables(spec, P, st, pos, graph)
-    ahead = _filters_ahead(spec, P, st, pos, graph, tables)
+        ahead = _table_filters(spec, P, st, pos, graph)
+    else:
+        ahead = _filters_ahead(spec, P, pos, graph, st.filt)
     for k, bp in enumerate(P.blocks):
         if k in ahead:
             W, Wd, done = ahead[k]
         else:
-            W, Wd = _block_filters(spec, P, st, pos, graph, tables, k)
+            W, Wd, dist = ops.filter_fwd(pos, graph, st.filt, bp.W1, bp.b1, bp.W2,
+                                         f16=spec.f16, want_dist=(k == 0),
+                                         strict_fp32=spec.strict_fp32)
             done = None
+            if k == 0:
+                st.dist = dist
         y = ops.node_linear(x, bp.A1, w_image=_wi(st, k, "A1", False))
         if done is not None:
             torch.cuda.current_stream(pos.device).wait_event(done)
@@ -686,34 +678,62 @@ def _node_tmm_batch(probs, rows, device):
     return [ops.node_tmm(a1, b1, a2, b2, colsum=cs) for a1, b1, a2, b2, cs in probs]
 
 
-def _filter_reverse(spec, st, bp, k, gagg2, g1, yd, dd, g_basis):
-    """(gW1, gb1, gW2, g_basis) of block k's filter from the node adjoints; the
-    basis parameters are shared by all blocks, so g_basis accumulates."""
-    graph, filt, train_basis = st.graph, st.filt, spec.basis_trainable
-    if st.grid is None:
-        res = ops.filter_bwd_cfconv(st.pos, graph, filt, bp.W1, bp.b1, bp.W2, gagg2, st.y[k], g1,
-                                    yd, dd, pair_adjoints=train_basis,
+class _FilterReverse:
+    """Weight and basis gradients of the blocks' filters from their node
+    adjoints.  Pair by pair, add() computes a block's at once.  Through the
+    tables it reduces the pairs onto the block's nodes, and finish() takes the
+    nodes of all blocks through the filter backward in one launch (160 tiles a
+    block leave a third of the chip idle: 512 x 35 beads, 27 us a block alone,
+    30 us for three), beside one for the blocks whose table does not serve."""
+
+    def __init__(self, spec: FusedSpec, P: Params, st: "State"):
+        self.spec, self.P, self.st = spec, P, st
+        L = len(P.blocks)
+        self.grads, self.adjoints = [None] * L, [None] * L
+        self.basis = None  # shared by the blocks: accumulates
+        self.slots = None
+        if st.grid is not None:
+            self.slots = ops.filter_table_slots(st.grid, st.graph, L)
+
+    def add(self, k: int, gagg2, g1, yd, dd) -> None:
+        spec, st, bp = self.spec, self.st, self.P.blocks[k]
+        if self.slots is not None:
+            self.adjoints[k] = (gagg2, st.y[k], g1, yd, dd)
+            ops.filter_table_reverse(st.grid, st.bins, st.graph, *self.adjoints[k], st.gates[k],
+                                     self.slots[k])
+            return
+        res = ops.filter_bwd_cfconv(st.pos, st.graph, st.filt, bp.W1, bp.b1, bp.W2, gagg2,
+                                    st.y[k], g1, yd, dd, pair_adjoints=spec.basis_trainable,
                                     strict_fp32=spec.strict_fp32)
-        if train_basis:
-            g_basis = ops.rbf_param_grad(st.dist, graph, filt, bp.W1, res[3], res[4],
-                                         out=g_basis)
-        return (*res[:3], g_basis)
-    # through the table's nodes where it serves, else pair by pair: of each
-    # couple of launches one returns at once
-    grid, gate = st.grid, st.gates[k]
-    wbar, wdbar = ops.filter_table_reverse(grid, st.bins, graph, gagg2, st.y[k], g1, yd, dd, gate)
-    at_nodes = ops.filter_bwd(grid.pos, grid.graph, filt, bp.W1, bp.b1, bp.W2, wbar, wdbar,
-                              pair_adjoints=train_basis, gate=gate)
-    by_pair = ops.filter_bwd_cfconv(st.pos, graph, filt, bp.W1, bp.b1, bp.W2, gagg2, st.y[k], g1,
-                                    yd, dd, pair_adjoints=train_basis, gate=gate,
-                                    out=at_nodes[:3])
-    if train_basis:
-        first = g_basis is None
-        g_basis = ops.rbf_param_grad(grid.dist, grid.graph, filt, bp.W1, *at_nodes[3:],
-                                     out=g_basis, gate=gate, gate_want=1)
-        ops.rbf_param_grad(st.dist, graph, filt, bp.W1, *by_pair[3:], out=g_basis,
-                           accumulate=not first, gate=gate, gate_want=0)
-    return (*at_nodes[:3], g_basis)
+        self.grads[k] = res[:3]
+        if spec.basis_trainable:
+            self.basis = ops.rbf_param_grad(st.dist, st.graph, st.filt, bp.W1, res[3], res[4],
+                                            out=self.basis)
+
+    def finish(self):
+        """([(gW1, gb1, gW2)] of the blocks, basis gradients or None)."""
+        spec, st = self.spec, self.st
+        if self.slots is None or not self.grads:
+            return self.grads, self.basis
+        grid, L, train = st.grid, len(self.grads), spec.basis_trainable
+        weights = _filter_weights(self.P)
+        self.grads = [ops.filter_grads(st.filt, st.pos.device) for _ in range(L)]
+        wbar, wdbar = ops.filter_table_combine(grid, st.bins, st.graph,
+                                               self.adjoints[0][2] is not None, st.gates,
+                                               self.slots)
+        nodes = ops.filter_bwd_blocks(grid.pos, grid.graph, st.filt, weights,
+                                      list(zip(wbar, wdbar)), self.grads, st.gates, 1,
+                                      pair_adjoints=train)
+        pairs = ops.filter_bwd_blocks(st.pos, st.graph, st.filt, weights, self.adjoints,
+                                      self.grads, st.gates, 0, pair_adjoints=train)
+        if train:
+            for k in range(L - 1, -1, -1):
+                W1, gate, first = weights[k][0], st.gates[k], self.basis is None
+                self.basis = ops.rbf_param_grad(grid.dist, grid.graph, st.filt, W1, *nodes[k],
+                                                out=self.basis, gate=gate, gate_want=1)
+                ops.rbf_param_grad(st.dist, st.graph, st.filt, W1, *pairs[k], out=self.basis,
+                                   accumulate=not first, gate=gate, gate_want=0)
+        return self.grads, self.basis
 
 
 def _blocks_reverse2(spec, P, st, tw, xbar2, g_out_w, g_out_b):
@@ -723,7 +743,7 @@ def _blocks_reverse2(spec, P, st, tw, xbar2, g_out_w, g_out_b):
     graph = st.graph
     n_lin = len(P.out_w)
     g_blocks = [None] * len(P.blocks)
-    g_basis = None
+    filters = _FilterReverse(spec, P, st)
     side = _SideStream(st.pos.device)
     N = st.pos.shape[0]
 
@@ -757,8 +777,9 @@ def _blocks_reverse2(spec, P, st, tw, xbar2, g_out_w, g_out_b):
             lambda: _node_tmm_batch(probs, N, st.pos.device), *held)
         xbar2 = ops.node_linear(ybar2, bp.A1, transpose=True, residual=xbar2,
                                 w_image=_wi(st, k, "A1", True))
-        gW1, gb1, gW2, g_basis = _filter_reverse(spec, st, bp, k, gagg2, g1, yd, dd, g_basis)
-        g_blocks[k] = [gW1, gb1, gW2, gA1, gA2, gc2, gA3, gc3]
+        filters.add(k, gagg2, g1, yd, dd)
+        g_blocks[k] = [gA1, gA2, gc2, gA3, gc3]
+    g_filters, g_basis = filters.finish()
     if P.emb.shape[0] <= 128 and P.emb.shape[1] == 128 and st.types.dtype == torch.int64:
         # fixed summation order; an out-of-table type raises a numerics flag
         g_emb = ops.type_sum(xbar2, st.types, P.emb.shape[0], want_bad=False)[0]
@@ -766,8 +787,8 @@ def _blocks_reverse2(spec, P, st, tw, xbar2, g_out_w, g_out_b):
         g_emb = torch.zeros_like(P.emb).index_add_(0, st.types, xbar2)
     side.join()
     out = [g_emb]
-    for gb in g_blocks:
-        out += gb
+    for gf, gb in zip(g_filters, g_blocks):
+        out += [*gf, *gb]
     for k in range(n_lin):
         out.append(g_out_w[k])
         if P.out_b[k] is not None:

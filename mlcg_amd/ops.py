@@ -874,29 +874,17 @@ BASIS_GAUSSIAN, BASIS_EXPNORMAL = 0, 1
 FILTER_FP32, FILTER_FP16, FILTER_FP32_STRICT = 0, 1, 2
 
 
-def _call_gated(name: str, args: tuple, gate: Optional[torch.Tensor], want: int, dev) -> None:
-    """Entry point `name`, or with `gate` its gated form: the launch does its
-    work only if the table serves (want 1) or does not (want 0)."""
-    if gate is None:
-        call(name, *args, stream_handle(dev))
-    else:
-        call(name + "_gated", *args, ptr(gate), want, stream_handle(dev))
-
-
 def filter_fwd(pos: torch.Tensor, graph: PairGraph, spec: FilterSpec, W1: torch.Tensor,
                b1: torch.Tensor, W2: torch.Tensor, f16: bool = False,
                want_dist: bool = True, strict_fp32: bool = False,
                out: Optional[Tuple[torch.Tensor, torch.Tensor]] = None,
-               gate: Optional[torch.Tensor] = None,
                ) -> Tuple[torch.Tensor, torch.Tensor, Optional[torch.Tensor]]:
     """W [P, F], dW/dd [P, F] (fp32, or fp16 when f16) and distances [P].
     fp32 results come from split-fp16 products (about 22 significant bits
     per operand, fp32 accumulation) unless strict_fp32 asks for the fp32
     MFMA throughout (mlcg_filter_fwd's FP32_STRICT mode).  `out` = (W, Wd)
     written in place of new tensors (a caller that launches on another
-    stream allocates them on the stream that consumes them).  With `gate` (a
-    block's gate words, filter_tables) the kernel returns at once when the
-    block's table serves."""
+    stream allocates them on the stream that consumes them)."""
     pos = _validate_pos(pos)
     F = W1.shape[0]
     _check(F == NUM_FILTERS, lambda: f"num_filters must be {NUM_FILTERS} for the HIP filter kernel")
@@ -920,7 +908,7 @@ def filter_fwd(pos: torch.Tensor, graph: PairGraph, spec: FilterSpec, W1: torch.
             ptr(b1c), ptr(W2c), F,
             FILTER_FP16 if f16 else (FILTER_FP32_STRICT if strict_fp32 else FILTER_FP32),
             ptr(W), ptr(Wd), ptr(dist))
-    _call_gated("mlcg_filter_fwd", args, gate, 0, pos.device)
+    call("mlcg_filter_fwd", *args, stream_handle(pos.device))
     return W, Wd, dist
 
 
@@ -968,6 +956,11 @@ def _pair_adjoint_outputs(want: bool, cap: int, F: int, dev):
             torch.empty(cap, F, dtype=torch.float32, device=dev))
 
 
+def filter_grads(spec: FilterSpec, dev):
+    """Uninitialised (dW1, db1, dW2)."""
+    return _filter_grads(NUM_FILTERS, spec.num_rbf, dev)
+
+
 def _filter_grads(F: int, K: int, dev):
     return (torch.empty(F, K, dtype=torch.float32, device=dev),
             torch.empty(F, dtype=torch.float32, device=dev),
@@ -976,15 +969,12 @@ def _filter_grads(F: int, K: int, dev):
 
 def filter_bwd(pos: torch.Tensor, graph: PairGraph, spec: FilterSpec, W1: torch.Tensor,
                b1: torch.Tensor, W2: torch.Tensor, Wbar: torch.Tensor,
-               Wdbar: torch.Tensor, pair_adjoints: bool = False, strict_fp32: bool = False,
-               gate: Optional[torch.Tensor] = None, out=None):
+               Wdbar: torch.Tensor, pair_adjoints: bool = False, strict_fp32: bool = False):
     """Gradients (dW1 [F, K], db1 [F], dW2 [F, F]) of <Wbar, W> + <Wdbar, dW/dd>;
     with pair_adjoints also the first-layer pair adjoints (abar, adbar)
     [P, F] that rbf_param_grad consumes.  strict_fp32 runs every product on
     the fp32 MFMA instead of split-fp16 products (which hold activations and
-    derivatives below 2^19, see check_numerics).  With `gate` the launch writes
-    its results, into `out` = (dW1, db1, dW2) when given, only if the block's
-    table serves."""
+    derivatives below 2^19, see check_numerics)."""
     pos = _validate_pos(pos)
     F = W1.shape[0]
     K = spec.num_rbf
@@ -995,7 +985,7 @@ def filter_bwd(pos: torch.Tensor, graph: PairGraph, spec: FilterSpec, W1: torch.
     nws = int(_lib.load().mlcg_filter_bwd_workspace_floats(cap, K))
     _check(nws > 0, lambda: f"num_rbf={K} is not supported by the filter backward")
     ws = torch.empty(nws, dtype=torch.float32, device=dev)
-    dW1, db1, dW2 = _filter_grads(F, K, dev) if out is None else out
+    dW1, db1, dW2 = _filter_grads(F, K, dev)
     W1c, b1c, W2c = (t.detach().float().contiguous() for t in (W1, b1, W2))
     ab, adb = _pair_adjoint_outputs(pair_adjoints, cap, F, dev)
     args = (ptr(pos), ptr(graph.pair_ij), cap, ptr(graph.n_pairs_dev), cap,
@@ -1003,7 +993,7 @@ def filter_bwd(pos: torch.Tensor, graph: PairGraph, spec: FilterSpec, W1: torch.
             spec.conv_cut_kind, spec.conv_lo, spec.conv_hi, spec.act, ptr(W1c), ptr(b1c),
             ptr(W2c), F, ptr(Wbar.contiguous()), ptr(Wdbar.contiguous()), ptr(dW1), ptr(db1),
             ptr(dW2), ptr(ab), ptr(adb), ptr(ws), nws, int(strict_fp32))
-    _call_gated("mlcg_filter_bwd", args, gate, 1, dev)
+    call("mlcg_filter_bwd", *args, stream_handle(dev))
     if pair_adjoints:
         return dW1, db1, dW2, ab, adb
     return dW1, db1, dW2
@@ -1014,12 +1004,10 @@ def filter_bwd_cfconv(pos: torch.Tensor, graph: PairGraph, spec: FilterSpec,
                       gagg2: torch.Tensor, y: torch.Tensor, gagg1: Optional[torch.Tensor],
                       ydot: Optional[torch.Tensor],
                       ddot: Optional[torch.Tensor], pair_adjoints: bool = False,
-                      strict_fp32: bool = False, gate: Optional[torch.Tensor] = None,
-                      out=None):
+                      strict_fp32: bool = False):
     """filter_bwd with Wbar_p = g2_i y_j + g2_j y_i + g1_i yd_j + g1_j yd_i and
     Wdbar_p = dd_p (g1_i y_j + g1_j y_i) formed in the kernel from node arrays
-    (pair_adjoints, strict_fp32 and out as in filter_bwd).  With `gate` the launch
-    writes its results only if the block's table does not serve."""
+    (pair_adjoints and strict_fp32 as in filter_bwd)."""
     pos = _validate_pos(pos)
     F = W1.shape[0]
     K = spec.num_rbf
@@ -1028,7 +1016,7 @@ def filter_bwd_cfconv(pos: torch.Tensor, graph: PairGraph, spec: FilterSpec,
     nws = int(_lib.load().mlcg_filter_bwd_workspace_floats(cap, K))
     _check(nws > 0, lambda: f"num_rbf={K} is not supported by the filter backward")
     ws = torch.empty(nws, dtype=torch.float32, device=dev)
-    dW1, db1, dW2 = _filter_grads(F, K, dev) if out is None else out
+    dW1, db1, dW2 = _filter_grads(F, K, dev)
     W1c, b1c, W2c = (t.detach().float().contiguous() for t in (W1, b1, W2))
     c = lambda t: None if t is None else t.contiguous()  # noqa: E731
     ab, adb = _pair_adjoint_outputs(pair_adjoints, cap, F, dev)
@@ -1037,7 +1025,7 @@ def filter_bwd_cfconv(pos: torch.Tensor, graph: PairGraph, spec: FilterSpec,
             spec.conv_cut_kind, spec.conv_lo, spec.conv_hi, spec.act, ptr(W1c), ptr(b1c),
             ptr(W2c), F, ptr(c(gagg2)), ptr(c(y)), ptr(c(gagg1)), ptr(c(ydot)), ptr(ddot),
             ptr(dW1), ptr(db1), ptr(dW2), ptr(ab), ptr(adb), ptr(ws), nws, int(strict_fp32))
-    _call_gated("mlcg_filter_bwd_cfconv", args, gate, 0, dev)
+    call("mlcg_filter_bwd_cfconv", *args, stream_handle(dev))
     if pair_adjoints:
         return dW1, db1, dW2, ab, adb
     return dW1, db1, dW2
@@ -1070,7 +1058,10 @@ def rbf_param_grad(dist: torch.Tensor, graph: PairGraph, spec: FilterSpec, W1: t
             spec.rbf_cut_kind, spec.rbf_lo, spec.rbf_hi, ptr(W1c), NUM_FILTERS,
             ptr(abar.contiguous()), ptr(adbar.contiguous()), int(accumulate), ptr(out[0]),
             ptr(out[1]), ptr(ws), nws)
-    _call_gated("mlcg_rbf_param_grad", args, gate, gate_want, dev)
+    if gate is None:
+        call("mlcg_rbf_param_grad", *args, stream_handle(dev))
+    else:
+        call("mlcg_rbf_param_grad_gated", *args, ptr(gate), gate_want, stream_handle(dev))
     return out
 
 
@@ -1078,7 +1069,7 @@ def rbf_param_grad(dist: torch.Tensor, graph: PairGraph, spec: FilterSpec, W1: t
 # Filter through a table over the distance (csrc/filter_table.hip)
 
 GATE_WORDS = 12
-TABLE_MAX_NODES = 8192 + 3
+TABLE_MAX_NODES = 8192
 
 
 @dataclass
@@ -1152,7 +1143,7 @@ def filter_grid(spec: FilterSpec, device) -> Optional[FilterGrid]:
 class PairBins:
     """Pairs in the order of their interpolation stencil (pair_bins)."""
 
-    records: torch.Tensor  # [P, 4] int32: pair, i, j, distance bits
+    records: torch.Tensor  # [P, 4] int32: pair, i, j, d / h in 2^-18
     start: torch.Tensor    # [nodes - 2] int32: first record of every stencil
     runs: torch.Tensor     # [nodes - 2] int32: first run of every stencil
     dist: torch.Tensor     # [P] float32, in pair order
@@ -1169,7 +1160,7 @@ def pair_bins(pos: torch.Tensor, graph: PairGraph, grid: FilterGrid) -> PairBins
     start, runs = torch.empty(2, grid.nodes - 2, dtype=torch.int32, device=dev)
     records = torch.empty(cap, 4, dtype=torch.int32, device=dev)
     call("mlcg_pair_bins", ptr(pos), ptr(graph.pair_ij), cap, ptr(graph.n_pairs_dev), cap,
-         grid.h, grid.nodes, ptr(dist), ptr(start), ptr(runs), ptr(records), ptr(ws), nws,
+         grid.h, grid.nodes, grid.cut, ptr(dist), ptr(start), ptr(runs), ptr(records), ptr(ws), nws,
          stream_handle(dev))
     return PairBins(records, start, runs, dist)
 
@@ -1191,54 +1182,119 @@ def filter_tables(grid: FilterGrid, spec: FilterSpec, weights, out=None
     them)."""
     dev = grid.pos.device
     L = len(weights)
-    F = NUM_FILTERS
-    flat = [t.detach().float().contiguous() for w in weights for t in w]
-    for k in range(L):
-        W1, b1, W2 = flat[3 * k:3 * k + 3]
-        _check(tuple(W1.shape) == (F, spec.num_rbf) and tuple(W2.shape) == (F, F)
-               and tuple(b1.shape) == (F,), "filter weights have unexpected shapes")
-    require_device(*flat)
+    flat = _block_weights(spec, weights)
     tables, gates = filter_table_buffers(grid, L) if out is None else out
-    ptrs = (ctypes.c_void_p * len(flat))(*[ptr(t) for t in flat])
-    call("mlcg_filter_table", ptrs, L, grid.nodes, grid.h, grid.rc, *spec.basis_args(),
+    call("mlcg_filter_table", _pointers(flat), L, grid.nodes, grid.h, grid.rc, *spec.basis_args(),
          spec.num_rbf, spec.rbf_cut_kind, spec.rbf_lo, spec.rbf_hi, spec.conv_cut_kind,
-         spec.conv_lo, spec.conv_hi, spec.act, F, ptr(tables), ptr(gates), stream_handle(dev))
+         spec.conv_lo, spec.conv_hi, spec.act, NUM_FILTERS, ptr(tables), ptr(gates),
+         stream_handle(dev))
     call("mlcg_filter_table_check", ptr(tables), L, grid.nodes, grid.h, grid.rc, ptr(gates),
          stream_handle(dev))
     return tables, gates
 
 
-def filter_table_rows(grid: FilterGrid, bins: PairBins, graph: PairGraph, table: torch.Tensor,
-                      gate: torch.Tensor, out: Tuple[torch.Tensor, torch.Tensor]) -> None:
-    """W, dW/dd of the pairs interpolated from a block's table into `out`
-    (fp32 or fp16); nothing is written if the table does not serve."""
-    W, Wd = out
+def _pointers(tensors):
+    """Host array of device addresses (None -> NULL)."""
+    return (ctypes.c_void_p * len(tensors))(*[ptr(t) for t in tensors])
+
+
+def _block_weights(spec: FilterSpec, weights) -> list:
+    """[(W1, b1, W2)] as a flat list of contiguous fp32 tensors."""
+    F = NUM_FILTERS
+    flat = [t.detach().float().contiguous() for w in weights for t in w]
+    for k in range(0, len(flat), 3):
+        _check(tuple(flat[k].shape) == (F, spec.num_rbf) and tuple(flat[k + 1].shape) == (F,)
+               and tuple(flat[k + 2].shape) == (F, F), "filter weights have unexpected shapes")
+    require_device(*flat)
+    return flat
+
+
+def filter_rows(grid: FilterGrid, bins: PairBins, pos: torch.Tensor, graph: PairGraph,
+                spec: FilterSpec, weights, tables: torch.Tensor, gates: torch.Tensor,
+                f16: bool = False) -> list:
+    """[(W, dW/dd)] [P, F] (fp32 or fp16) of the blocks' pairs: interpolated from
+    the tables, or evaluated pair by pair for a block whose table does not
+    serve; one launch each for all blocks."""
+    pos = _validate_pos(pos)
     cap = graph.pair_capacity
-    _check(W.dtype == Wd.dtype and tuple(W.shape) == tuple(Wd.shape) == (cap, NUM_FILTERS)
-           and W.is_contiguous() and Wd.is_contiguous(),
-           "filter_table_rows out tensors must be contiguous [pair_capacity, 128]")
-    call("mlcg_filter_table_rows", ptr(bins.records), ptr(graph.n_pairs_dev), cap, grid.h,
-         grid.nodes, grid.cut, ptr(table), ptr(gate), int(W.dtype == torch.float16), ptr(W),
-         ptr(Wd), stream_handle(W.device))
+    dev = pos.device
+    L = len(weights)
+    _check(tuple(tables.shape) == (L, 4, grid.nodes + 1, NUM_FILTERS)
+           and tuple(gates.shape) == (L, GATE_WORDS) and tables.is_contiguous()
+           and gates.is_contiguous(), "tables / gates have unexpected shapes")
+    flat = _block_weights(spec, weights)
+    dt = torch.float16 if f16 else torch.float32
+    out = [torch.empty(cap, NUM_FILTERS, dtype=dt, device=dev) for _ in range(2 * L)]
+    outs = _pointers(out)
+    call("mlcg_filter_table_rows", ptr(bins.records), ptr(graph.n_pairs_dev), cap, grid.nodes,
+         ptr(tables), ptr(gates), L, int(f16), outs, stream_handle(dev))
+    call("mlcg_filter_fwd_blocks", ptr(pos), ptr(graph.pair_ij), cap, ptr(graph.n_pairs_dev), cap,
+         *spec.basis_args(), spec.num_rbf, spec.rbf_cut_kind, spec.rbf_lo, spec.rbf_hi,
+         spec.conv_cut_kind, spec.conv_lo, spec.conv_hi, spec.act, _pointers(flat), outs, L,
+         NUM_FILTERS, FILTER_FP16 if f16 else FILTER_FP32, ptr(gates), 0, stream_handle(dev))
+    return [(out[2 * k], out[2 * k + 1]) for k in range(L)]
+
+
+def filter_table_slots(grid: FilterGrid, graph: PairGraph, blocks: int) -> torch.Tensor:
+    """[blocks, floats] partial sums of filter_table_reverse."""
+    n = int(_lib.load().mlcg_filter_table_reverse_workspace_floats(graph.pair_capacity,
+                                                                   grid.nodes))
+    return torch.empty(blocks, n, dtype=torch.float32, device=grid.pos.device)
 
 
 def filter_table_reverse(grid: FilterGrid, bins: PairBins, graph: PairGraph,
                          gagg2: torch.Tensor, y: torch.Tensor, gagg1: Optional[torch.Tensor],
                          ydot: Optional[torch.Tensor], ddot: Optional[torch.Tensor],
-                         gate: torch.Tensor) -> Tuple[torch.Tensor, torch.Tensor]:
-    """Adjoints (Wbar, Wdbar) [nodes, F] of a block's table values from the
-    node arrays of filter_bwd_cfconv."""
-    dev = y.device
+                         gate: torch.Tensor, slots: torch.Tensor) -> None:
+    """First part of the adjoints of a block's table values, into the block's
+    slots, from the node arrays of filter_bwd_cfconv."""
     cap = graph.pair_capacity
-    nws = int(_lib.load().mlcg_filter_table_reverse_workspace_floats(cap, grid.nodes))
-    ws = torch.empty(nws, dtype=torch.float32, device=dev)
-    wbar = torch.empty(grid.nodes, NUM_FILTERS, dtype=torch.float32, device=dev)
-    wdbar = torch.empty(grid.nodes, NUM_FILTERS, dtype=torch.float32, device=dev)
     g2, yc, g1, yd = (None if t is None else t.contiguous() for t in (gagg2, y, gagg1, ydot))
     call("mlcg_filter_table_reverse", ptr(bins.records), ptr(bins.start), ptr(bins.runs), cap,
-         grid.h, grid.nodes, grid.cut, ptr(g2), ptr(yc), ptr(g1), ptr(yd), ptr(ddot),
-         ptr(gate), ptr(wbar), ptr(wdbar), ptr(ws), nws, stream_handle(dev))
+         grid.nodes, ptr(g2), ptr(yc), ptr(g1), ptr(yd), ptr(ddot),
+         ptr(gate), ptr(slots), slots.numel(), stream_handle(y.device))
+
+
+def filter_table_combine(grid: FilterGrid, bins: PairBins, graph: PairGraph, tangent: bool,
+                         gates: torch.Tensor, slots: torch.Tensor
+                         ) -> Tuple[torch.Tensor, torch.Tensor]:
+    """Adjoints (Wbar, Wdbar) [blocks, nodes, F] of the blocks' table values."""
+    L = slots.shape[0]
+    wbar, wdbar = torch.empty(2, L, grid.nodes, NUM_FILTERS, dtype=torch.float32,
+                              device=slots.device)
+    call("mlcg_filter_table_combine", ptr(bins.runs), graph.pair_capacity, grid.nodes,
+         int(tangent), ptr(slots), L, ptr(gates), ptr(wbar), ptr(wdbar),
+         stream_handle(slots.device))
     return wbar, wdbar
+
+
+def filter_bwd_blocks(pos: torch.Tensor, graph: PairGraph, spec: FilterSpec, weights, adjoints,
+                      grads, gates: torch.Tensor, gate_want: int, pair_adjoints: bool = False):
+    """filter_bwd (adjoints [(Wbar, Wdbar)]) or filter_bwd_cfconv (adjoints
+    [(gagg2, y, gagg1, ydot, ddot)]) of several blocks in one launch, into
+    grads [(dW1, db1, dW2)]; a block's work is done only if its table serves
+    (gate_want 1) or does not (0).  With pair_adjoints, the list of the blocks'
+    first-layer pair adjoints (abar, adbar)."""
+    pos = _validate_pos(pos)
+    cap = graph.pair_capacity
+    dev = pos.device
+    K, F, L = spec.num_rbf, NUM_FILTERS, len(weights)
+    nws = int(_lib.load().mlcg_filter_bwd_blocks_workspace_floats(cap, K, L))
+    _check(nws > 0, lambda: f"num_rbf={K} is not supported by the filter backward")
+    ws = torch.empty(nws, dtype=torch.float32, device=dev)
+    flat = _block_weights(spec, weights)
+    abars, args = [], []
+    for k, adj in enumerate(adjoints):
+        adj = [None if t is None else t.contiguous() for t in adj]
+        adj = adj + [None] * 5 if len(adj) == 2 else [None, None] + adj
+        ab = _pair_adjoint_outputs(pair_adjoints, cap, F, dev)
+        abars.append(ab)
+        args += flat[3 * k:3 * k + 3] + adj + list(grads[k]) + list(ab)
+    call("mlcg_filter_bwd_blocks", ptr(pos), ptr(graph.pair_ij), cap, ptr(graph.n_pairs_dev), cap,
+         *spec.basis_args(), K, spec.rbf_cut_kind, spec.rbf_lo, spec.rbf_hi, spec.conv_cut_kind,
+         spec.conv_lo, spec.conv_hi, spec.act, _pointers(args), L, F, ptr(gates), gate_want,
+         ptr(ws), nws, stream_handle(dev))
+    return abars
 
 
 # --------------------------------------------------------------------------
