@@ -410,7 +410,8 @@ int mlcg_filter_table_combine(const int32_t* run_start, int64_t max_pairs, int
                               float* wdbar, void* stream);
 
 /* Several blocks in one launch, gated (gates may be NULL).
- * mlcg_filter_fwd_blocks: weights and outputs as above, no distances.
+ * mlcg_filter_fwd_blocks: weights and outputs as above; dist_out [P]: the
+ * distances, from the first block (NULL = not wanted; needs gates == NULL).
  * mlcg_filter_bwd_blocks: 15 pointers a block -- W1, b1, W2, then the pair
  * adjoints Wbar, Wdbar (mlcg_filter_bwd) or the node arrays gagg2, y, gagg1,
  * ydot, ddot (mlcg_filter_bwd_cfconv), then dW1, db1, dW2, abar_out,
@@ -422,8 +423,8 @@ int mlcg_filter_fwd_blocks(const float* pos, const int32_t* pair_ij, int64_t
                            rbf_cut_kind, float rbf_lo, float rbf_hi, int
                            conv_cut_kind, float conv_lo, float conv_hi, int
                            act, const void* const* weights, void* const*
-                           outputs, int num_blocks, int num_filters, int f16,
-                           const uint32_t* gates, int gate_want, void*
+                           outputs, float* dist_out, int num_blocks, int
+                           num_filters, int f16, const uint32_t* gates, int gate_want, void*
                            stream);
 int64_t mlcg_filter_bwd_blocks_workspace_floats(int64_t max_pairs, int
     num_rbf, int num_blocks);
@@ -559,6 +560,62 @@ int mlcg_pair_forces(const float* pos, const float* dist, const float* dbar,
                      const int32_t* rowptr, const int32_t* col,
                      const int32_t* eid2pair, int64_t n_nodes, int accumulate,
                      float* forces, void* stream);
+
+/* Energies [n_frames] and forces [n_nodes, 3] of the SchNet whose filter values
+ * and distances are already there: embedding lookup, node sweep, output network
+ * and reverse sweep, issued one after the other on the stream with the launches
+ * of the separate entry points.  filters: W, Wd of each block.  weights:
+ * embedding table [num_types, 128]; lin1 [128, 128], lin2, its bias, lin, its
+ * bias of each block; output network W0 [out_hidden, 128], b0 (may be NULL), w1,
+ * b1 (may be NULL).  seed [n_nodes]: adjoint of the node energies.
+ * arrays: mlcg_energy_forces_arrays() arrays of [n_nodes, 128].  With keep they
+ * hold, in this order, x (num_blocks + 1), then num_blocks each of y, s, z (only
+ * with an activation other than tanh), agg, gagg, xbar, ybar (the first not
+ * written), sbar, zbar, for the second reverse sweep; without it they are
+ * scratch.  images: 6 * num_blocks split weight images (64 KiB each; with keep
+ * they stay valid: lin1, lin2, lin of each block, each as it is and transposed).
+ * out_rows: with keep the output network's activations [n_nodes, out_hidden]
+ * and, with an activation other than tanh, its pre-activations; then, with and
+ * without keep, the node energies [n_nodes].  dbar [P]:
+ * distance adjoints. */
+int64_t mlcg_energy_forces_arrays(int num_blocks, int block_act, int keep);
+int mlcg_energy_forces(const float* pos, const float* dist, const int64_t*
+                       types, int64_t n_nodes, const int64_t* frame_ptr,
+                       int64_t n_frames, const int32_t* rowptr, const int32_t*
+                       col, const int32_t* eid2pair, const void* const*
+                       filters, int w_f16, const void* const* weights, int
+                       num_blocks, int num_types, int out_hidden, int
+                       block_act, int out_act, int keep, const float* seed,
+                       float* arrays, int64_t num_arrays, void* images, float*
+                       out_rows, float* dbar, float* energies, float* forces,
+                       void* stream);
+
+/* Parameter gradients of <pw, o> + <tw, odot>, odot the derivative of the node
+ * energies o along positions + scale * u, after mlcg_energy_forces with keep and
+ * seed = tw: tangent sweep, output network, second reverse sweep, with the
+ * launches of the separate entry points; the filters' gradients are left to the
+ * caller.  arrays, images, out_rows: as kept; filters fp32; pw may be NULL.
+ * arrays2: mlcg_energy_forces_grad_arrays() arrays of [n_nodes, 128]: after
+ * num_blocks of xdot, num_blocks each of ydot (the first not written), aggdot,
+ * zdot, sdot, gagg2, then scratch; with ddot [P] that is what the filters'
+ * gradients read.  grads: one per weight, shaped like it (the output
+ * network's biases NULL as there).  At most 128 types. */
+int64_t mlcg_energy_forces_grad_arrays(int num_blocks);
+int64_t mlcg_energy_forces_grad_workspace_floats(int64_t n_nodes, int num_types,
+                                                 int out_hidden);
+int mlcg_energy_forces_grad(const float* pos, const float* dist, const int64_t*
+                            types, int64_t n_nodes, const int32_t* rowptr,
+                            const int32_t* col, const int32_t* eid2pair, const
+                            int32_t* pair_ij, int64_t pair_capacity, const
+                            int32_t* n_pairs_dev, const void* const* filters,
+                            const void* const* weights, int num_blocks, int
+                            num_types, int out_hidden, int block_act, int
+                            out_act, const float* u, float scale, const float*
+                            tw, const float* pw, const float* arrays, const
+                            void* images, const float* out_rows, float* ddot,
+                            float* arrays2, int64_t num_arrays2, float*
+                            workspace, int64_t workspace_floats, void* const*
+                            grads, void* stream);
 
 /* E[b] = sum_{n in frame b} values[n * stride] (ascending n).  Replaces
  * torch_geometric.utils.scatter(..., reduce="sum") of schnet.py:158. */

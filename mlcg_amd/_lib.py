@@ -82,7 +82,14 @@ _SIGNATURES = {
     "mlcg_pair_bins": [_P, _P, _I64, _P, _I64, _F32, _I32, _F32, _P, _P, _P, _P, _P, _I64, _P],
     "mlcg_filter_table_reverse_workspace_floats": [_I64, _I32],
     "mlcg_filter_fwd_blocks": [_P, _P, _I64, _P, _I64, _I32, _P, _P, _F64, _I32, _I32, _F32,
-        _F32, _I32, _F32, _F32, _I32, _P, _P, _I32, _I32, _I32, _P, _I32, _P],
+        _F32, _I32, _F32, _F32, _I32, _P, _P, _P, _I32, _I32, _I32, _P, _I32, _P],
+    "mlcg_energy_forces_arrays": [_I32, _I32, _I32],
+    "mlcg_energy_forces_grad_arrays": [_I32],
+    "mlcg_energy_forces_grad_workspace_floats": [_I64, _I32, _I32],
+    "mlcg_energy_forces_grad": [_P, _P, _P, _I64, _P, _P, _P, _P, _I64, _P, _P, _P, _I32, _I32,
+        _I32, _I32, _I32, _P, _F32, _P, _P, _P, _P, _P, _P, _P, _I64, _P, _I64, _P, _P],
+    "mlcg_energy_forces": [_P, _P, _P, _I64, _P, _I64, _P, _P, _P, _P, _I32, _P, _I32, _I32, _I32,
+        _I32, _I32, _I32, _P, _P, _I64, _P, _P, _P, _P, _P, _P],
     "mlcg_filter_bwd_blocks": [_P, _P, _I64, _P, _I64, _I32, _P, _P, _F64, _I32, _I32, _F32,
         _F32, _I32, _F32, _F32, _I32, _P, _I32, _I32, _P, _I32, _P, _I64, _P],
     "mlcg_filter_table_rows": [_P, _P, _I64, _I32, _P, _P, _I32, _I32, _P, _P],
@@ -146,7 +153,9 @@ _SIGNATURES = {
 }
 _RESTYPES = {"mlcg_version": _c.c_char_p, "mlcg_scan_workspace_ints": _I64,
              "mlcg_radius_workspace_bytes": _I64,
-             "mlcg_pair_bins_workspace_ints": _I64,
+             "mlcg_pair_bins_workspace_ints": _I64, "mlcg_energy_forces_arrays": _I64,
+             "mlcg_energy_forces_grad_arrays": _I64,
+             "mlcg_energy_forces_grad_workspace_floats": _I64,
              "mlcg_filter_bwd_blocks_workspace_floats": _I64,
              "mlcg_filter_table_reverse_workspace_floats": _I64,
              "mlcg_filter_bwd_workspace_floats": _I64, "mlcg_node_tmm_workspace_floats": _I64,
@@ -247,6 +256,11 @@ def set_timer(timer: Optional[LaunchTimer]) -> Optional[LaunchTimer]:
     global _timer
     old, _timer = _timer, timer
     return old
+
+
+def timed(names) -> bool:
+    """Whether a launch timer watches one of these entry points."""
+    return _timer is not None and any(_timer.wants(n) for n in names)
 
 
 def call(name: str, *args, work=None) -> None:

@@ -2439,9 +2439,9 @@ extern "C" int mlcg_filter_fwd_blocks(const float* pos, const int32_t* pair_ij,
                                       int rbf_cut_kind, float rbf_lo, float rbf_hi,
                                       int conv_cut_kind, float conv_lo, float conv_hi, int act,
                                       const void* const* weights, void* const* outputs,
-                                      int num_blocks, int num_filters, int f16,
+                                      float* dist_out, int num_blocks, int num_filters, int f16,
                                       const uint32_t* gates, int gate_want, void* stream) {
-  MLCG_REQUIRE(weights && outputs && num_blocks >= 1);
+  MLCG_REQUIRE(weights && outputs && num_blocks >= 1 && !(dist_out && gates));
   for (int first = 0; first < num_blocks; first += kMaxBlocks) {
     const int n = num_blocks - first < kMaxBlocks ? num_blocks - first : kMaxBlocks;
     FwdBatch fb = {};
@@ -2449,7 +2449,8 @@ extern "C" int mlcg_filter_fwd_blocks(const float* pos, const int32_t* pair_ij,
       const void* const* w = weights + 3 * (first + k);
       void* const* o = outputs + 2 * (first + k);
       fb.b[k] = FwdBlock{static_cast<const float*>(w[0]), static_cast<const float*>(w[1]),
-                         static_cast<const float*>(w[2]), o[0], o[1], nullptr,
+                         static_cast<const float*>(w[2]), o[0], o[1],
+                         first + k == 0 ? dist_out : nullptr,
                          FilterGate{gates ? gates + (first + k) * kGateWords : nullptr,
                                     gate_want}};
     }

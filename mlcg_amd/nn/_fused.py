@@ -37,7 +37,7 @@ import os
 
 import torch
 
-from .. import ops
+from .. import _lib, ops
 from .activations import ACT_TANH, act_derivs, act_value
 
 
@@ -166,6 +166,7 @@ class State:
     xdotL: Optional[torch.Tensor] = None      # tangent of the last block output
     out_seed: Optional[torch.Tensor] = None   # reverse seed the forward already applied
     out_xbar: Optional[torch.Tensor] = None   # ... and the adjoint it produced
+    kept: Optional["Kept"] = None             # a native sweep's arrays instead of the lists
 
 
 def _out_fused(P: "Params") -> bool:
@@ -303,12 +304,17 @@ def _table_grid(spec: FusedSpec, filt, graph: ops.PairGraph, pos: torch.Tensor, 
     return grid
 
 
+# The filters' tables on the side stream (MLCG_FILTER_AHEAD=0 makes them in order
+# on the caller's stream).
+_FILTER_AHEAD = os.environ.get("MLCG_FILTER_AHEAD", "1") != "0"
+
+
 def _filter_weights(P: Params):
     return [(bp.W1, bp.b1, bp.W2) for bp in P.blocks]
 
 
-def _table_filters(spec: FusedSpec, P: Params, st: "State", pos, graph) -> dict:
-    """{k: (W, Wd, None)} of every block through its table.  The tables, which
+def _table_filters(spec: FusedSpec, P: Params, st: "State", pos, graph) -> list:
+    """[(W, dW/dd)] of every block through its table.  The tables, which
     depend on the weights alone, are made on the side stream while the caller's
     stream orders the pairs; their buffers belong to the caller's stream, which
     waits for the side stream before it goes on."""
@@ -316,52 +322,31 @@ def _table_filters(spec: FusedSpec, P: Params, st: "State", pos, graph) -> dict:
     side = _side_stream(main)
     weights = _filter_weights(P)
     tables, st.gates = out = ops.filter_table_buffers(st.grid, len(P.blocks))
-    side.wait_stream(main)
-    with torch.cuda.stream(side):
+    if _FILTER_AHEAD:
+        side.wait_stream(main)
+    with torch.cuda.stream(side if _FILTER_AHEAD else main):
         ops.filter_tables(st.grid, st.filt, weights, out=out)
     st.bins = ops.pair_bins(pos, graph, st.grid)
     st.dist = st.bins.dist
-    main.wait_stream(side)
-    rows = ops.filter_rows(st.grid, st.bins, pos, graph, st.filt, weights, tables, st.gates,
+    if _FILTER_AHEAD:
+        main.wait_stream(side)
+    return ops.filter_rows(st.grid, st.bins, pos, graph, st.filt, weights, tables, st.gates,
                            f16=spec.f16)
-    return {k: (W, Wd, None) for k, (W, Wd) in enumerate(rows)}
 
 
-# Filter forwards of blocks 1.. on the side stream (MLCG_FILTER_AHEAD=0 keeps
-# them in block order on the caller's stream).
-_FILTER_AHEAD = os.environ.get("MLCG_FILTER_AHEAD", "1") != "0"
-
-
-def _filters_ahead(spec: FusedSpec, P: Params, pos: torch.Tensor, graph: ops.PairGraph,
-                   filt) -> dict:
-    """Issues the pair-by-pair filter forwards of blocks 1.. on the side stream at the start
-    of the forward: they depend only on the pair distances and the block's
-    filter weights, not on node features, so they run beside block 0's node
-    linears and gathers (memory-bound work that leaves VGPRs and LDS free on
-    each CU).  Returns {k: (W, Wd, event)}; the caller's stream waits on the
-    event before block k's gather.  The outputs are allocated on the caller's
-    stream, which alone uses them afterwards."""
-    if not (_FILTER_AHEAD and pos.is_cuda and len(P.blocks) > 1):
-        return {}
-    main = torch.cuda.current_stream(pos.device)
-    side = _side_stream(main)
-    cap = graph.pair_capacity
-    dt = torch.float16 if spec.f16 else torch.float32
-    outs = {k: (torch.empty(cap, ops.NUM_FILTERS, dtype=dt, device=pos.device),
-                torch.empty(cap, ops.NUM_FILTERS, dtype=dt, device=pos.device))
-            for k in range(1, len(P.blocks))}
-    side.wait_stream(main)
-    ahead = {}
-    with torch.cuda.stream(side):
-        for k in range(1, len(P.blocks)):
-            bp = P.blocks[k]
-            W, Wd, _ = ops.filter_fwd(pos, graph, filt, bp.W1, bp.b1, bp.W2, f16=spec.f16,
-                                      want_dist=False, strict_fp32=spec.strict_fp32,
-                                      out=outs[k])
-            ev = torch.cuda.Event()
-            ev.record(side)
-            ahead[k] = (W, Wd, ev)
-    return ahead
+def _filters(spec: FusedSpec, P: Params, st: "State", pos, graph) -> list:
+    """[(W, dW/dd)] of the blocks, and the pair distances in st.dist: through
+    their tables where st has a grid, else pair by pair, all blocks in one launch
+    (512 x 35 beads, energies and forces: 756 us of device time against 763 with
+    the blocks' launches on a second stream beside the node sweep; 24 x 35 beads
+    173 against 203)."""
+    if st.grid is not None:
+        return _table_filters(spec, P, st, pos, graph)
+    if not P.blocks:
+        return []
+    rows, st.dist = ops.filter_fwd_blocks(pos, graph, st.filt, _filter_weights(P), f16=spec.f16,
+                                          strict_fp32=spec.strict_fp32)
+    return rows
 
 
 # Split images of the block weights made once per forward (MLCG_NODE_IMAGES=0
@@ -400,34 +385,15 @@ def forward(spec: FusedSpec, P: Params, pos: torch.Tensor, types: torch.Tensor,
     kernel also forms the adjoint a following reverse1(seed=rev_seed) starts
     from."""
     st = State(pos=pos, types=types, graph=graph, filt=filter_spec(spec, P))
-    # the lookup goes first: the side stream's filter forwards then start
-    # with the first block's node products already queued behind it
     if (P.emb.dim() == 2 and P.emb.shape[1] == ops.NUM_FILTERS
             and P.emb.dtype == torch.float32 and types.dtype == torch.int64):
         x = ops.embedding_gather(P.emb.detach(), types)
     else:
         x = P.emb.index_select(0, types)
-    # the weight images before the side stream's filter forwards, which would
-    # otherwise hold every CU while this short launch waits for one
     st.wimg = _weight_images(P, x, transposed=save)
     st.grid = _table_grid(spec, st.filt, graph, pos, reverse)
-    if st.grid is not None:
-        ahead = _table_filters(spec, P, st, pos, graph)
-    else:
-        ahead = _filters_ahead(spec, P, pos, graph, st.filt)
-    for k, bp in enumerate(P.blocks):
-        if k in ahead:
-            W, Wd, done = ahead[k]
-        else:
-            W, Wd, dist = ops.filter_fwd(pos, graph, st.filt, bp.W1, bp.b1, bp.W2,
-                                         f16=spec.f16, want_dist=(k == 0),
-                                         strict_fp32=spec.strict_fp32)
-            done = None
-            if k == 0:
-                st.dist = dist
+    for (W, Wd), (k, bp) in zip(_filters(spec, P, st, pos, graph), enumerate(P.blocks)):
         y = ops.node_linear(x, bp.A1, w_image=_wi(st, k, "A1", False))
-        if done is not None:
-            torch.cuda.current_stream(pos.device).wait_event(done)
         agg = ops.cfconv_gather(y, W, graph)
         # z itself is only read back by the shifted-softplus derivatives;
         # x_next = x + lin(act(z))
@@ -524,6 +490,115 @@ def reverse1(spec: FusedSpec, P: Params, st: State, seed: torch.Tensor,
     if not need_forces:
         return None
     return ops.pair_forces(st.pos, st.dist, dbar, graph)
+
+
+# What the native sweeps launch without passing through these wrappers.
+_SWEEP = ("mlcg_embedding_gather", "mlcg_node_weight_images", "mlcg_node_gemm",
+          "mlcg_node_gemm2", "mlcg_cfconv_gather", "mlcg_out_forward", "mlcg_segment_sum",
+          "mlcg_cfconv_gather_bwd", "mlcg_pair_forces")
+_SWEEP2 = ("mlcg_pair_ddot", "mlcg_node_gemm", "mlcg_node_gemm2", "mlcg_cfconv_gather_tangent",
+           "mlcg_out_rev2", "mlcg_cfconv_gather_rev2", "mlcg_node_tmm_batch", "mlcg_type_sum")
+
+
+@dataclass
+class Kept:
+    """A native sweep's state: its weights and filters, and what
+    ops.energy_forces kept."""
+
+    weights: list
+    filters: list
+    arrays: tuple
+
+
+def energy_forces(spec: FusedSpec, P: Params, pos: torch.Tensor, types: torch.Tensor,
+                  graph: ops.PairGraph, seed: torch.Tensor, training: bool
+                  ) -> Tuple[torch.Tensor, torch.Tensor, State]:
+    """(E, F, state) of forward and reverse1(seed).  Where the kernels tile the
+    model's widths and no launch of the sweep is timed by itself, one native call
+    issues the node sweep (ops.energy_forces): the same launches with the same
+    results, without their cost in Python."""
+    weights = [P.emb]
+    for b in P.blocks:
+        weights += (b.A1, b.A2, b.c2, b.A3, b.c3)
+    for w, b in zip(P.out_w, P.out_b):
+        weights += (w, b)
+    if not (P.blocks and _out_fused(P) and _NODE_IMAGES and not _lib.timed(_SWEEP)
+            and ops.energy_forces_ok(pos, types, graph, weights, P.out_w[0].shape[0])):
+        E, st = forward(spec, P, pos, types, graph, save=True, rev_seed=seed, reverse=training)
+        return E, reverse1(spec, P, st, seed, keep_adjoints=training), st
+    st = State(pos=pos, types=types, graph=graph, filt=filter_spec(spec, P))
+    st.grid = _table_grid(spec, st.filt, graph, pos, training)
+    filters = _filters(spec, P, st, pos, graph)
+    E, F, arrays = ops.energy_forces(pos, types, graph, st.dist, filters, weights,
+                                     P.out_w[0].shape[0], spec.block_act, spec.out_act, seed,
+                                     training)
+    if training:
+        st.kept = Kept(weights, filters, arrays)
+    return E, F, st
+
+
+def _unpack(spec: FusedSpec, P: Params, st: State) -> None:
+    """The lists of st that tangent and reverse2 read, from a native sweep's
+    arrays."""
+    kept, st.kept = st.kept, None
+    L, (arrays, images, rows) = len(P.blocks), kept.arrays
+    n, hidden = st.pos.shape[0], P.out_w[0].shape[0]
+    it = iter(arrays.unbind(0))
+    take = lambda m: [next(it) for _ in range(m)]  # noqa: E731
+    st.W, st.Wd = [list(t) for t in zip(*kept.filters)]
+    *st.x, st.xL = take(L + 1)
+    st.y, st.s = take(L), take(L)
+    st.z = take(L) if spec.block_act != ACT_TANH else [None] * L
+    st.agg, st.gagg1, st.xbar_out, st.ybar1 = take(L), take(L), take(L), take(L)
+    st.ybar1[0] = None
+    st.sbar1, st.zbar1 = take(L), take(L)
+    st.os_ = [rows[:n * hidden].view(n, hidden)]
+    st.oz = [rows[n * hidden:2 * n * hidden].view(n, hidden)
+             if spec.out_act != ACT_TANH else None]
+    st.wimg = {(k, m, t): images[(3 * k + i) * 2 + t] for k in range(L)
+               for i, m in enumerate(_IMAGE_NAMES) for t in (False, True)}
+
+
+def force_gradients(spec: FusedSpec, P: Params, st: State, u: Optional[torch.Tensor],
+                    scale: float, tw: Optional[torch.Tensor], pw: Optional[torch.Tensor]
+                    ) -> List[torch.Tensor]:
+    """tangent(u, scale) and reverse2(tw, pw) after energy_forces(seed=tw): by one
+    native call and the filters' gradients where energy_forces was one, too."""
+    if st.kept is None or u is None or P.emb.shape[0] > 128 or _TMM_SIDE or _lib.timed(_SWEEP2):
+        if st.kept is not None:
+            _unpack(spec, P, st)
+        if u is not None:
+            tangent(spec, P, st, u, scale)
+        return reverse2(spec, P, st, tw, pw)
+    kept, L = st.kept, len(P.blocks)
+    grads, ddot, st.y, gagg1, ydot, gagg2 = ops.energy_forces_grad(
+        st.pos, st.types, st.graph, st.dist, kept.filters, kept.weights, P.out_w[0].shape[0],
+        spec.block_act, spec.out_act, kept.arrays, u, scale, tw, pw)
+    filters = _FilterReverse(spec, P, st)
+    for k in range(L - 1, -1, -1):
+        filters.add(k, gagg2[k], gagg1[k], ydot[k], ddot)
+    g_filters, g_basis = filters.finish()
+    blocks = [grads[1 + 5 * k:6 + 5 * k] for k in range(L)]
+    return _flat_gradients(spec, P, grads[0], g_filters, blocks, grads[-4::2], grads[-3::2],
+                           g_basis)
+
+
+def _flat_gradients(spec, P, g_emb, g_filters, g_blocks, g_out_w, g_out_b, g_basis):
+    """The gradients in Params.flat() order."""
+    out = [g_emb]
+    for gf, gb in zip(g_filters, g_blocks):
+        out += [*gf, *gb]
+    for k in range(len(P.out_w)):
+        out.append(g_out_w[k])
+        if P.out_b[k] is not None:
+            out.append(g_out_b[k])
+    if spec.basis_trainable:
+        gc, gw = g_basis
+        if P.basis[1].numel() != gw.numel():  # one shared Gaussian coefficient
+            gw = gw.sum()
+        out += [gc.reshape(P.basis[0].shape).to(P.basis[0].dtype),
+                gw.reshape(P.basis[1].shape).to(P.basis[1].dtype)]
+    return out
 
 
 def tangent(spec: FusedSpec, P: Params, st: State, u: torch.Tensor,
@@ -741,7 +816,6 @@ def _blocks_reverse2(spec, P, st, tw, xbar2, g_out_w, g_out_b):
     adjoint xbar2; assembles the gradients in Params.flat() order."""
     tangent_on = tw is not None
     graph = st.graph
-    n_lin = len(P.out_w)
     g_blocks = [None] * len(P.blocks)
     filters = _FilterReverse(spec, P, st)
     side = _SideStream(st.pos.device)
@@ -786,20 +860,7 @@ def _blocks_reverse2(spec, P, st, tw, xbar2, g_out_w, g_out_b):
     else:
         g_emb = torch.zeros_like(P.emb).index_add_(0, st.types, xbar2)
     side.join()
-    out = [g_emb]
-    for gf, gb in zip(g_filters, g_blocks):
-        out += [*gf, *gb]
-    for k in range(n_lin):
-        out.append(g_out_w[k])
-        if P.out_b[k] is not None:
-            out.append(g_out_b[k])
-    if spec.basis_trainable:
-        gc, gw = g_basis
-        if P.basis[1].numel() != gw.numel():  # one shared Gaussian coefficient
-            gw = gw.sum()
-        out += [gc.reshape(P.basis[0].shape).to(P.basis[0].dtype),
-                gw.reshape(P.basis[1].shape).to(P.basis[1].dtype)]
-    return out
+    return _flat_gradients(spec, P, g_emb, g_filters, g_blocks, g_out_w, g_out_b, g_basis)
 
 
 _ONES: dict = {}
@@ -839,9 +900,7 @@ class EnergyForces(torch.autograd.Function):
     def forward(ctx, spec, pos, types, batch, graph, training, *flat):
         P = Params.unflat(spec, list(flat))
         ones = _ones(pos.shape[0], pos.device)
-        E, st = forward(spec, P, pos, types, graph, save=True, rev_seed=ones,
-                        reverse=bool(training))
-        F = reverse1(spec, P, st, ones, keep_adjoints=bool(training))
+        E, F, st = energy_forces(spec, P, pos, types, graph, ones, bool(training))
         if training:
             ctx.spec, ctx.P, ctx.st, ctx.batch = spec, P, st, batch
         ctx.set_materialize_grads(False)
@@ -857,14 +916,13 @@ class EnergyForces(torch.autograd.Function):
         tw = pw = None
         if Fbar is not None:
             # <Fbar, F> = <Fbar, -grad sum E> : tangent along u = -Fbar, seed 1
-            tangent(spec, P, st, Fbar, scale=-1.0)
             tw = _ones(st.pos.shape[0], st.pos.device)
         if Ebar is not None:
             pw = node_seed(Ebar, batch)
         if tw is None and pw is None:
             grads = [None] * len(P.flat())
         else:
-            grads = reverse2(spec, P, st, tw, pw)
+            grads = force_gradients(spec, P, st, Fbar, -1.0, tw, pw)
         ctx.st = None
         return (None, None, None, None, None, None, *grads)
 

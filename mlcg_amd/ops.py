@@ -1230,9 +1230,132 @@ def filter_rows(grid: FilterGrid, bins: PairBins, pos: torch.Tensor, graph: Pair
          ptr(tables), ptr(gates), L, int(f16), outs, stream_handle(dev))
     call("mlcg_filter_fwd_blocks", ptr(pos), ptr(graph.pair_ij), cap, ptr(graph.n_pairs_dev), cap,
          *spec.basis_args(), spec.num_rbf, spec.rbf_cut_kind, spec.rbf_lo, spec.rbf_hi,
-         spec.conv_cut_kind, spec.conv_lo, spec.conv_hi, spec.act, _pointers(flat), outs, L,
-         NUM_FILTERS, FILTER_FP16 if f16 else FILTER_FP32, ptr(gates), 0, stream_handle(dev))
+         spec.conv_cut_kind, spec.conv_lo, spec.conv_hi, spec.act, _pointers(flat), outs,
+         None, L, NUM_FILTERS, FILTER_FP16 if f16 else FILTER_FP32, ptr(gates), 0,
+         stream_handle(dev))
     return [(out[2 * k], out[2 * k + 1]) for k in range(L)]
+
+
+def filter_fwd_blocks(pos: torch.Tensor, graph: PairGraph, spec: FilterSpec, weights,
+                      f16: bool = False, strict_fp32: bool = False) -> Tuple[list, torch.Tensor]:
+    """([(W, dW/dd)] of the blocks, distances [P]): filter_fwd of every block's
+    (W1, b1, W2), one launch for all."""
+    pos = _validate_pos(pos)
+    cap, dev, L = graph.pair_capacity, pos.device, len(weights)
+    flat = _block_weights(spec, weights)
+    dt = torch.float16 if f16 else torch.float32
+    out = [torch.empty(cap, NUM_FILTERS, dtype=dt, device=dev) for _ in range(2 * L)]
+    dist = torch.empty(cap, dtype=torch.float32, device=dev)
+    mode = FILTER_FP16 if f16 else (FILTER_FP32_STRICT if strict_fp32 else FILTER_FP32)
+    call("mlcg_filter_fwd_blocks", ptr(pos), ptr(graph.pair_ij), cap, ptr(graph.n_pairs_dev), cap,
+         *spec.basis_args(), spec.num_rbf, spec.rbf_cut_kind, spec.rbf_lo, spec.rbf_hi,
+         spec.conv_cut_kind, spec.conv_lo, spec.conv_hi, spec.act, _pointers(flat),
+         _pointers(out), ptr(dist), L, NUM_FILTERS, mode, None, 0, stream_handle(dev))
+    return list(zip(out[::2], out[1::2])), dist
+
+
+def energy_forces_ok(pos: torch.Tensor, types: torch.Tensor, graph: PairGraph, weights,
+                     hidden: int) -> bool:
+    """Whether energy_forces takes these (see there)."""
+    shape, dev = (NUM_FILTERS, NUM_FILTERS), pos.device
+    if not (pos.is_cuda and graph.pair_capacity and graph.num_nodes and types.is_contiguous()
+            and types.dtype == torch.int64 and types.device == dev
+            and types.shape == pos.shape[:1] and graph.num_nodes == pos.shape[0]
+            and graph.frame_ptr.numel() > 1):
+        return False
+    for t in weights:
+        if t is not None and not (t.dtype == torch.float32 and t.is_contiguous()
+                                  and t.device == dev):
+            return False
+    n = (len(weights) - 5) // 5
+    square, width = weights[1:1 + 5 * n], NUM_FILTERS
+    return (n >= 1 and weights[0].dim() == 2 and weights[0].shape[1] == width
+            and all(square[5 * k + i].shape == shape for k in range(n) for i in (0, 1, 3))
+            and all(square[5 * k + i].numel() == width for k in range(n) for i in (2, 4))
+            and hidden in OUT_HIDDEN and weights[-4].shape == (hidden, width)
+            and weights[-2].numel() == hidden)
+
+
+def energy_forces(pos: torch.Tensor, types: torch.Tensor, graph: PairGraph, dist: torch.Tensor,
+                  filters, weights, hidden: int, block_act: int, out_act: int,
+                  seed: torch.Tensor, keep: bool):
+    """(E [B], F [N, 3], kept) of the node sweep and its reverse in one call
+    (mlcg_energy_forces) from the blocks' filters [(W, dW/dd)].  weights:
+    embedding table; A1, A2, c2, A3, c3 of each block; W0, b0 | None, w1,
+    b1 | None of the output network.  The caller has asked energy_forces_ok about
+    these arguments.  With keep, kept = (arrays, images, rows) as
+    mlcg_energy_forces documents them, for energy_forces_grad."""
+    pos = _validate_pos(pos)
+    n, dev, L = pos.shape[0], pos.device, len(filters)
+    cap, dt = graph.pair_capacity, filters[0][0].dtype
+    flat = [t for f in filters for t in f]
+    _check(len(weights) == 5 + 5 * L and all(
+        t.shape == (cap, NUM_FILTERS) and t.dtype == dt and t.is_contiguous() and t.device == dev
+        for t in flat) and dt in (torch.float32, torch.float16),
+        "filters must be contiguous [P, 128] tensors of one type")
+    for t, m in ((dist, cap), (seed, n)):
+        _check(t.shape == (m,) and t.dtype == torch.float32 and t.is_contiguous()
+               and t.device == dev, "dist / seed must be contiguous float32 vectors")
+    count = int(_lib.load().mlcg_energy_forces_arrays(L, block_act, int(keep)))
+    arrays = torch.empty(count, n, NUM_FILTERS, dtype=torch.float32, device=dev)
+    images = torch.empty(6 * L, NODE_W_IMAGE_HALFS, dtype=torch.float16, device=dev)
+    per = 1 + ((1 + (out_act != 0)) * hidden if keep else 0)
+    rows = torch.empty(n * per, dtype=torch.float32, device=dev)
+    dbar = torch.empty(cap, dtype=torch.float32, device=dev)
+    B = graph.frame_ptr.numel() - 1
+    E = torch.empty(B, dtype=torch.float32, device=dev)
+    F = torch.empty_like(pos)
+    call("mlcg_energy_forces", ptr(pos), ptr(dist), ptr(types), n, ptr(graph.frame_ptr), B,
+         ptr(graph.rowptr), ptr(graph.col), ptr(graph.eid2pair), _pointers(flat),
+         int(dt == torch.float16), _pointers(weights), L, weights[0].shape[0], hidden,
+         int(block_act), int(out_act), int(keep), ptr(seed), ptr(arrays), count, ptr(images),
+         ptr(rows), ptr(dbar), ptr(E), ptr(F), stream_handle(dev))
+    return E, F, (arrays, images, rows) if keep else None
+
+
+def energy_forces_grad(pos: torch.Tensor, types: torch.Tensor, graph: PairGraph,
+                       dist: torch.Tensor, filters, weights, hidden: int, block_act: int,
+                       out_act: int, kept, u: torch.Tensor, scale: float, tw: torch.Tensor,
+                       pw: Optional[torch.Tensor]):
+    """(grads, ddot, y, gagg1, ydot, gagg2) after energy_forces(keep=True) with
+    seed = tw: the gradients of <pw, o> + <tw, odot> by every entry of weights
+    (None for a None), odot along scale * u, and what the gradients of the
+    filters read, per block (mlcg_energy_forces_grad)."""
+    _check(energy_forces_ok(pos, types, graph, weights, hidden) and weights[0].shape[0] <= 128,
+           "energy_forces_grad: unsupported shapes, types or layouts")
+    pos, (arrays, images, rows) = _validate_pos(pos), kept
+    n, dev, L, cap = pos.shape[0], pos.device, len(filters), graph.pair_capacity
+    flat = [t for f in filters for t in f]
+    ssp = int(block_act != 0)
+    _check(len(weights) == 5 + 5 * L and all(
+        t.shape == (cap, NUM_FILTERS) and t.dtype == torch.float32 and t.is_contiguous()
+        and t.device == dev for t in flat), "filters must be contiguous [P, 128] float32 tensors")
+    _check(arrays.shape == (1 + (9 + ssp) * L, n, NUM_FILTERS)
+           and images.shape == (6 * L, NODE_W_IMAGE_HALFS)
+           and rows.numel() == n * (1 + (1 + (out_act != 0)) * hidden),
+           "kept arrays do not match the call")
+    u = u.contiguous()
+    for t, shape in ((dist, (cap,)), (tw, (n,)), (pw, (n,)), (u, (n, 3))):
+        _check(t is None or t.shape == shape and t.dtype == torch.float32 and t.is_contiguous()
+               and t.device == dev, "dist, u, tw, pw must be float32 tensors matching pos")
+    lib = _lib.load()
+    count = int(lib.mlcg_energy_forces_grad_arrays(L))
+    arrays2 = torch.empty(count, n, NUM_FILTERS, dtype=torch.float32, device=dev)
+    ddot = torch.empty(cap, dtype=torch.float32, device=dev)
+    types_n = weights[0].shape[0]
+    nws = int(lib.mlcg_energy_forces_grad_workspace_floats(n, types_n, hidden))
+    ws = torch.empty(nws, dtype=torch.float32, device=dev)
+    grads = [None if t is None else torch.empty(t.shape, dtype=torch.float32, device=dev)
+             for t in weights]
+    call("mlcg_energy_forces_grad", ptr(pos), ptr(dist), ptr(types), n, ptr(graph.rowptr),
+         ptr(graph.col), ptr(graph.eid2pair), ptr(graph.pair_ij), cap, ptr(graph.n_pairs_dev),
+         _pointers(flat), _pointers(weights), L, types_n, hidden, int(block_act), int(out_act),
+         ptr(u), float(scale), ptr(tw), ptr(pw), ptr(arrays), ptr(images), ptr(rows), ptr(ddot),
+         ptr(arrays2), count, ptr(ws), nws, _pointers(grads), stream_handle(dev))
+    at = lambda a, k: a[k:k + L].unbind(0)  # noqa: E731
+    r0 = 1 + (3 + ssp) * L
+    return (grads, ddot, at(arrays, L + 1), at(arrays, r0 + L),
+            (None, *at(arrays2, L)[1:]), at(arrays2, 5 * L))
 
 
 def filter_table_slots(grid: FilterGrid, graph: PairGraph, blocks: int) -> torch.Tensor:
