@@ -33,7 +33,7 @@ Besides the JSON contract fields the line carries
                    forces per call, and the fp16 filter kernel's MFMA fraction;
   eager_step    -- the same config-2 step launched kernel by kernel: wall
                    time, host issue time, device time, and the device time
-                   with the filter forwards issued in block order;
+                   with the filters' tables made on a second stream;
   md_config5    -- config 5 (100 x 268-bead Langevin replicas, SchNet +
                    priors, captured step): MD steps/s;
   cpu_baseline  -- the CPU restatement (oracle/schnet_ref.py) of the same
@@ -115,6 +115,19 @@ def algorithmic_work(name: str, E: int, P: int, N: int, B: int, f16: bool = Fals
     if name == "mlcg_filter_fwd":
         # value and distance-tangent through both linears
         return "mfma", 2 * 2 * kf_ff * P, "flop"
+    if name == "mlcg_filter_fwd_blocks":
+        # the same, all blocks in one launch (gated: blocks whose table does
+        # not serve, so usually none; see kernel_report)
+        return "mfma", N_BLOCKS * 2 * 2 * kf_ff * P, "flop"
+    if name == "mlcg_filter_table_rows":
+        # value and slope rows of every pair and block written, records read
+        return "hbm", N_BLOCKS * 2 * sw * F * P + 16 * P, "byte"
+    if name == "mlcg_filter_table_reverse":
+        # records and ddot per pair; gagg2, y, gagg1, ydot in (the rows each
+        # pair gathers come from the caches and are not counted)
+        return "hbm", 20 * P + 4 * 4 * F * N, "byte"
+    if name == "mlcg_pair_bins":
+        return "hbm", 8 * P + 12 * N + 4 * P + 16 * P, "byte"
     if name in ("mlcg_filter_bwd", "mlcg_filter_bwd_cfconv"):
         # two reverse products through W2^T plus the pair reductions of the
         # weight gradients dW2 (two streams) and dW1 (two streams); the
@@ -169,12 +182,21 @@ def algorithmic_work(name: str, E: int, P: int, N: int, B: int, f16: bool = Fals
 # products of split operands: their MFMA ceiling, in fp32-equivalent FLOP/s,
 # is a third of the fp16 peak.  (The filter backward's recomputation of the
 # first layer stays on the fp32 MFMA but is not counted as algorithmic work.)
-SPLIT_FP16 = {"mlcg_filter_fwd", "mlcg_filter_bwd", "mlcg_filter_bwd_cfconv"}
+SPLIT_FP16 = {"mlcg_filter_fwd", "mlcg_filter_fwd_blocks", "mlcg_filter_bwd",
+              "mlcg_filter_bwd_cfconv"}
 SPLIT_FP16_PEAK_TFLOPS = FP16_MFMA_PEAK_TFLOPS / 3
 
 # entry point -> kernel symbol(s) it launches (as rocprofv3 names them)
 KERNEL_SYMBOL = {
     "mlcg_filter_fwd": "filter_fwd_x3_kernel",
+    "mlcg_filter_fwd_blocks": "filter_fwd_x3_kernel",
+    "mlcg_filter_table": "filter_table_kernel",
+    "mlcg_filter_table_check": "table_check_kernel",
+    "mlcg_filter_table_rows": "table_rows_kernel",
+    "mlcg_filter_table_reverse": "table_reverse_kernel",
+    "mlcg_filter_table_combine": "table_combine_kernel",
+    "mlcg_filter_bwd_blocks": "filter_bwd_fused_kernel",
+    "mlcg_pair_bins": "pair_key_scatter_kernel",
     "mlcg_filter_bwd": "filter_bwd_fused_kernel",
     "mlcg_filter_bwd_cfconv": "filter_bwd_fused_kernel",
     "mlcg_node_tmm": "node_tmm_kernel",
@@ -202,8 +224,12 @@ def kernel_report(summary, E, P, N, B, work=None):
     on the epilogue); the other entry points use algorithmic_work."""
     work = work or {}
     rows = {}
+    # beside a table the pair-by-pair launch finds every block's gate closed
+    gated = "mlcg_filter_table_rows" in summary
     for name, (launches, total_ms) in summary.items():
         w = algorithmic_work(name, E, P, N, B)
+        if gated and name == "mlcg_filter_fwd_blocks":
+            w = None
         if w is not None and name in work:
             w = (w[0], work[name] / max(launches, 1), w[2])
         avg_ms = total_ms / max(launches, 1)
@@ -359,7 +385,7 @@ def gpu_leg(args):
     torch.cuda.synchronize()
     # per-kernel profiling pass (outside the timed region), every HIP entry
     # point bracketed by events, with the whole step on one stream (filter
-    # forwards in block order, weight-gradient reductions inline) so that no
+    # tables before the pairs' order, weight-gradient reductions inline) so that no
     # launch shares the GPU with another stream's work: stand-alone times
     ahead, side = _fused._FILTER_AHEAD, _fused._TMM_SIDE
     _fused._FILTER_AHEAD = _fused._TMM_SIDE = False
@@ -391,11 +417,11 @@ def gpu_leg(args):
     # and the device time of a step queued ahead of the GPU
     host_ms = _host_issue_ms(step)
     dev_ms = _device_ms_per_step(step)
-    # the same step with the filter forwards in block order on one stream
-    _fused._FILTER_AHEAD = False
+    # the same step with the filters' tables on a second stream
+    _fused._FILTER_AHEAD = True
     step()
-    noahead_ms, _ = _timed_steps(step, args.steps)
-    noahead_dev_ms = _device_ms_per_step(step)
+    ahead_ms, _ = _timed_steps(step, args.steps)
+    ahead_dev_ms = _device_ms_per_step(step)
     _fused._FILTER_AHEAD = ahead
     # the same step with the filter forward on the fp32 MFMA throughout
     # (MLCG_FILTER_FP32_STRICT) instead of split-fp16 products, for comparison
@@ -407,8 +433,8 @@ def gpu_leg(args):
     return {"ms_per_step": ms, "E": E, "P": P, "N": N, "B": B, "dominant": dominant,
             "strict_fp32_ms_per_step": strict_ms,
             "host_issue_ms": host_ms, "device_ms": dev_ms,
-            "filter_ahead_off": {"ms_per_step": round(noahead_ms, 4),
-                                 "device_ms_per_step": round(noahead_dev_ms, 4)},
+            "filter_ahead": {"ms_per_step": round(ahead_ms, 4),
+                             "device_ms_per_step": round(ahead_dev_ms, 4)},
             "dominant_row": dom, "kernels": warm, "loss": float(loss.detach()),
             "step_kernel_ms": round(sum(per_step.values()), 4)}
 
@@ -732,21 +758,30 @@ def fp16_leg(reps=5):
             gm(data)
             torch.cuda.synchronize()
             t.append(time.perf_counter() - t0)
-        # the filter kernel's stand-alone launch time: filter forwards in
-        # block order on one stream, bracketed by events
-        ahead = _fused._FILTER_AHEAD
+        # the filter kernel's stand-alone launch time, bracketed by events:
+        # pair by pair (the fp16 MFMA kernel, which serves smaller calls and
+        # filters that no table holds) and through the tables
+        ahead, table = _fused._FILTER_AHEAD, _fused._FILTER_TABLE
         _fused._FILTER_AHEAD = False
-        timer = _lib.LaunchTimer({"mlcg_filter_fwd"})
+        timer = _lib.LaunchTimer({"mlcg_filter_table", "mlcg_filter_table_check",
+                                  "mlcg_pair_bins", "mlcg_filter_table_rows"})
+        _lib.set_timer(timer)
+        for _ in range(2):
+            gm(data)
+        torch.cuda.synchronize()
+        table_us = sum(t for _, t in timer.summary().values()) / 2 * 1e3
+        _fused._FILTER_TABLE = False
+        timer = _lib.LaunchTimer({"mlcg_filter_fwd_blocks"})
         _lib.set_timer(timer)
         for _ in range(2):
             gm(data)
         torch.cuda.synchronize()
         _lib.set_timer(None)
-        _fused._FILTER_AHEAD = ahead
+        _fused._FILTER_AHEAD, _fused._FILTER_TABLE = ahead, table
     s = statistics.median(t)
-    n_l, tot = timer.summary()["mlcg_filter_fwd"]
+    n_l, tot = timer.summary()["mlcg_filter_fwd_blocks"]
     avg = tot / n_l
-    flops = 2 * 2 * (K_RBF * F + F * F) * P
+    flops = N_BLOCKS * 2 * 2 * (K_RBF * F + F * F) * P
     ach = flops / (avg * 1e-3) / 1e12
     return {"workload": "config4: 256 frames x 500-bead globules, rc 15 A, fp16 filter "
                         "linears (fp32 accumulate), energy + forces",
@@ -755,7 +790,8 @@ def fp16_leg(reps=5):
             "filter_roofline": {"kernel": "filter_fwd_f16_kernel", "bound": "mfma",
                                 "achieved": round(ach, 2), "peak": FP16_MFMA_PEAK_TFLOPS,
                                 "unit": "TFLOP/s", "frac": round(ach / FP16_MFMA_PEAK_TFLOPS, 4),
-                                "avg_launch_us": round(avg * 1e3, 2)}}
+                                "avg_launch_us": round(avg * 1e3, 2)},
+            "filter_tables_us": round(table_us, 2)}
 
 
 def md_leg(steps):
@@ -1148,7 +1184,7 @@ def main(argv=None):
                        "edges_per_s": g["E"] * N_BLOCKS / (eager_ms * 1e-3),
                        "host_issue_ms": round(g["host_issue_ms"], 4),
                        "device_ms": round(g["device_ms"], 4),
-                       "filter_ahead_off": g["filter_ahead_off"]},
+                       "filter_ahead": g["filter_ahead"]},
         "strict_fp32_filters_eager_step_ms": round(g["strict_fp32_ms_per_step"], 4),
         "roofline": roofline,
         "kernels_us_frac": brief,

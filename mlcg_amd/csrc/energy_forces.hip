@@ -6,8 +6,10 @@
 // The sweep is about eight launches per block of 2-10 us each on small systems,
 // so what bounds a small call is the host.  Issued one entry point at a time
 // from Python, a launch costs 10-20 us (allocation, checks, argument
-// conversion); from here it costs the launch alone.  The launches, their order
-// and their results are those of the separate entry points.
+// conversion); from here it costs the launch alone: energies and forces of one
+// 35-bead chain 541 -> 280 us in all, the training step on 24 x 57 beads 1074 with
+// the first sweep here and 851 with both, from 989-1296.  The launches, their
+// order and their results are those of the separate entry points.
 #include "common.h"
 
 namespace {

@@ -210,9 +210,9 @@ __device__ __forceinline__ void rbf_expnormal_fine(const RbfParams& rp, float ce
 // The elementwise functions of the filter in double, for the nodes of a table:
 // a node's rounding is shared by every pair near it (bonded pairs, a tenth of a
 // chain's, all lie in one cell) and does not average out over the pairs as in
-// the pair-by-pair kernels.  In float the gradients of an exponential-normal
-// basis, which depend on exp(-alpha d) - centre with a factor of some 45, were
-// 4e-6 off.  Envelope: identity, or cosine with lower bound 0.
+// the pair-by-pair kernels.  In float (the basis and alpha itself) the gradients
+// of an exponential-normal basis, which depend on exp(-alpha d) - centre with a
+// factor of some 45, were 4e-6 off.  Envelope: identity, or cosine with lower bound 0.
 __device__ __forceinline__ void cutoff_f64(int kind, float hi, double d, double& c, double& dc) {
   c = 1.0;
   dc = 0.0;

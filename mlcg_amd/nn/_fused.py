@@ -77,6 +77,10 @@ class FusedSpec:
     def __post_init__(self):
         self.grid_shape = ops.filter_grid_shape(self.filt)
 
+    def __getstate__(self):
+        # a copy or a saved model makes its own grids, on the device it runs on
+        return {**self.__dict__, "grids": {}}
+
 
 @dataclass
 class Params:
@@ -274,17 +278,23 @@ def _table_pays(spec: FusedSpec, pairs: int, nodes: int, reverse: bool) -> bool:
     """Whether the filters go through a table (csrc/filter_table.hip) instead of
     one network evaluation per pair.  The table costs its nodes and the ordering
     of the pairs once per call and, with a reverse sweep, some launches per
-    block; it saves time per pair and block.  Measured (device us, 35-bead
-    chains, Gaussian basis, 2561 nodes, direct / table): energies and forces,
-    3 blocks 42 k pairs 274 / 292, 84 k 393 / 375, 1 block 84 k 142 / 178;
-    force-matching step, 3 blocks 42 k 775 / 805, 84 k 1130 / 1043, 1 block 84 k
-    396 / 411; exponential-normal basis (7681 nodes), 2 blocks, trainable, 27 k
-    687 / 702, 55 k 918 / 772 (the gradient of the basis is then taken at the
-    nodes too, which saves three times as much a pair)."""
+    block; it saves time per pair and block.  Measured with 35-bead chains, us on
+    the device / in all, issued eagerly (direct, table).  Energies and forces,
+    Gaussian basis (2551 nodes), 3 blocks: 62 k pairs 311 / 338, 313 / 351, 106 k
+    443 / 465, 427 / 457, 215 k 756 / 759, 673 / 700; 1 block: 215 k 264 / 293,
+    273 / 300; exponential-normal basis (7242 nodes), 2 blocks: 137 k 346 / 374,
+    389 / 412.  Force-matching gradient, Gaussian, 3 blocks: 42 k 735 / 1241, 710 /
+    1176, 62 k 919 / 1061, 822 / 1174, 106 k 1312 / 1326, 1113 / 1263, 215 k 2261 /
+    2209, 1794 / 1827; 1 block: 106 k 479 / 714, 445 / 883, 215 k 800 / 840, 670 /
+    866; exponential-normal, trainable (the basis' gradient is then taken at the
+    nodes too, which saves three times as much a pair), 2 blocks: 55 k 726 / 1004,
+    669 / 1115, 137 k 1281 / 1292, 984 / 1143.  The lines lie between where the
+    device's time breaks even, which a captured step sees, and where an eager
+    call's does."""
     work = pairs * spec.num_blocks
     if not reverse:
-        return work >= 48 * nodes + 64_000
-    return work * (3 if spec.basis_trainable else 1) >= 32 * nodes + 22_000 * spec.num_blocks
+        return work >= 48 * nodes + 150_000
+    return work * (3 if spec.basis_trainable else 1) >= 32 * nodes + 50_000 * spec.num_blocks
 
 
 def _table_grid(spec: FusedSpec, filt, graph: ops.PairGraph, pos: torch.Tensor, reverse: bool):
@@ -304,9 +314,11 @@ def _table_grid(spec: FusedSpec, filt, graph: ops.PairGraph, pos: torch.Tensor, 
     return grid
 
 
-# The filters' tables on the side stream (MLCG_FILTER_AHEAD=0 makes them in order
-# on the caller's stream).
-_FILTER_AHEAD = os.environ.get("MLCG_FILTER_AHEAD", "1") != "0"
+# MLCG_FILTER_AHEAD=1 makes the filters' tables on the side stream, beside the
+# ordering of the pairs.  Off: each of the two fills the chip, and the streams'
+# waits cost more than the overlap gives (512 x 35 beads, captured step 1824 us with
+# it, 1812 without, eager step 2055 and 1977; MD step of 100 x 268 1738 and 1716).
+_FILTER_AHEAD = os.environ.get("MLCG_FILTER_AHEAD", "0") == "1"
 
 
 def _filter_weights(P: Params):
@@ -314,18 +326,19 @@ def _filter_weights(P: Params):
 
 
 def _table_filters(spec: FusedSpec, P: Params, st: "State", pos, graph) -> list:
-    """[(W, dW/dd)] of every block through its table.  The tables, which
-    depend on the weights alone, are made on the side stream while the caller's
-    stream orders the pairs; their buffers belong to the caller's stream, which
-    waits for the side stream before it goes on."""
-    main = torch.cuda.current_stream(pos.device)
-    side = _side_stream(main)
+    """[(W, dW/dd)] of every block through its table.  On the side stream
+    (_FILTER_AHEAD) the tables' buffers belong to the caller's stream, which waits
+    for the side stream before it goes on."""
     weights = _filter_weights(P)
-    tables, st.gates = out = ops.filter_table_buffers(st.grid, len(P.blocks))
     if _FILTER_AHEAD:
+        main = torch.cuda.current_stream(pos.device)
+        side = _side_stream(main)
+        tables, st.gates = out = ops.filter_table_buffers(st.grid, len(P.blocks))
         side.wait_stream(main)
-    with torch.cuda.stream(side if _FILTER_AHEAD else main):
-        ops.filter_tables(st.grid, st.filt, weights, out=out)
+        with torch.cuda.stream(side):
+            ops.filter_tables(st.grid, st.filt, weights, out=out)
+    else:
+        tables, st.gates = ops.filter_tables(st.grid, st.filt, weights)
     st.bins = ops.pair_bins(pos, graph, st.grid)
     st.dist = st.bins.dist
     if _FILTER_AHEAD:

@@ -1201,10 +1201,11 @@ def _pointers(tensors):
 def _block_weights(spec: FilterSpec, weights) -> list:
     """[(W1, b1, W2)] as a flat list of contiguous fp32 tensors."""
     F = NUM_FILTERS
-    flat = [t.detach().float().contiguous() for w in weights for t in w]
-    for k in range(0, len(flat), 3):
-        _check(tuple(flat[k].shape) == (F, spec.num_rbf) and tuple(flat[k + 1].shape) == (F,)
-               and tuple(flat[k + 2].shape) == (F, F), "filter weights have unexpected shapes")
+    flat = [t if t.dtype == torch.float32 and t.is_contiguous() else t.detach().float().contiguous()
+            for w in weights for t in w]
+    shapes = ((F, spec.num_rbf), (F,), (F, F))
+    _check(all(t.shape == shapes[i % 3] for i, t in enumerate(flat)),
+           "filter weights have unexpected shapes")
     require_device(*flat)
     return flat
 

@@ -523,3 +523,16 @@ def test_filter_grid_shape(kw, ok):
         assert 64 <= n <= ops.TABLE_MAX_NODES and (n - 1) * h <= rc < n * h
         k = np.arange(n)
         assert (k.astype(np.float32) * np.float32(h) == k * h).all()  # exact node distances
+
+
+def test_filter_grids_stay_out_of_copies():
+    import copy
+    import pickle
+
+    from mlcg_amd.nn._fused import FusedSpec
+
+    spec = FusedSpec(filt=_filter_spec(), filter_act=0, block_act=0, out_act=0, num_blocks=1,
+                     out_has_bias=[True, False])
+    spec.grids[0] = object()
+    for other in (copy.deepcopy(spec), pickle.loads(pickle.dumps(spec))):
+        assert other.grids == {} and other.grid_shape == spec.grid_shape
