@@ -395,7 +395,9 @@ int mlcg_filter_table_rows(const int32_t* records, const int32_t* n_pairs_dev,
  * wdbar [num_blocks, nodes, F] (mlcg_filter_table_combine, all blocks, whose
  * slots follow each other); tangent as gagg1 != NULL.  Every sum has a fixed
  * order.  mlcg_filter_bwd_blocks on the nodes then gives the weight
- * gradients. */
+ * gradients: mlcg_filter_table_combine also writes them as a pair list of
+ * `nodes` pairs, node_pos [nodes, 3], node_dist [nodes], node_pair_ij
+ * [2, nodes] and node_count [1]. */
 int64_t mlcg_filter_table_reverse_workspace_floats(int64_t max_pairs, int
     nodes);
 int mlcg_filter_table_reverse(const int32_t* records, const int32_t* start,
@@ -407,7 +409,9 @@ int mlcg_filter_table_reverse(const int32_t* records, const int32_t* start,
 int mlcg_filter_table_combine(const int32_t* run_start, int64_t max_pairs, int
                               nodes, int tangent, const float* slots, int
                               num_blocks, const uint32_t* gates, float* wbar,
-                              float* wdbar, void* stream);
+                              float* wdbar, float h, float* node_pos, float*
+                              node_dist, int32_t* node_pair_ij, int32_t*
+                              node_count, void* stream);
 
 /* Several blocks in one launch, gated (gates may be NULL).
  * mlcg_filter_fwd_blocks: weights and outputs as above; dist_out [P]: the

@@ -94,7 +94,8 @@ _SIGNATURES = {
         _F32, _I32, _F32, _F32, _I32, _P, _I32, _I32, _P, _I32, _P, _I64, _P],
     "mlcg_filter_table_rows": [_P, _P, _I64, _I32, _P, _P, _I32, _I32, _P, _P],
     "mlcg_filter_table_reverse": [_P, _P, _P, _I64, _I32, _P, _P, _P, _P, _P, _P, _P, _I64, _P],
-    "mlcg_filter_table_combine": [_P, _I64, _I32, _I32, _P, _I32, _P, _P, _P, _P],
+    "mlcg_filter_table_combine": [_P, _I64, _I32, _I32, _P, _I32, _P, _P, _P, _F32, _P, _P,
+        _P, _P, _P],
     "mlcg_filter_bwd_blocks_workspace_floats": [_I64, _I32, _I32],
     "mlcg_cfconv_gather": [_P, _P, _I32, _P, _P, _P, _I64, _I32, _P, _P],
     "mlcg_cfconv_gather_bwd": [_P, _P, _P, _P, _I32, _P, _P, _P, _I64, _I32, _P, _P, _I32,

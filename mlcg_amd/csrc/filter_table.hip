@@ -562,12 +562,32 @@ __device__ __forceinline__ void add_slots(const float* __restrict__ o, int first
   }
 }
 
+// The nodes as pairs {0, m} of the positions (m h, 0, 0), for the kernels that
+// then run on them.  Written here, by the first block whatever its gate: as
+// buffers of the call they live as long as what reads them, a recorded graph
+// included, without a launch of their own.
+struct NodePairs {
+  float h;
+  float *pos, *dist;  // [nodes, 3], [nodes]
+  int32_t *ij, *count;  // [2, nodes], [1]
+};
+
 template <bool kTan>
 __global__ __launch_bounds__(256) void table_combine_kernel(
     const int32_t* __restrict__ run_start, int nkeys, const float* __restrict__ block_slots,
     int64_t slot_stride, int nodes, const unsigned* __restrict__ gates,
-    float* __restrict__ block_wbar, float* __restrict__ block_wdbar) {
+    float* __restrict__ block_wbar, float* __restrict__ block_wdbar, NodePairs np) {
   const int blk = blockIdx.y;
+  if (blk == 0 && threadIdx.x == 0) {
+    const int m = blockIdx.x;
+    const float d = (float)m * np.h;  // exact
+    np.pos[3 * m] = d;
+    np.pos[3 * m + 1] = np.pos[3 * m + 2] = 0.0f;
+    np.dist[m] = d;
+    np.ij[m] = 0;
+    np.ij[nodes + m] = m;
+    if (m == 0) *np.count = nodes;
+  }
   if (!filter_table_serves(gates + blk * kGateWords)) return;
   const float* __restrict__ slots = block_slots + blk * slot_stride;
   float* __restrict__ wbar = block_wbar + (int64_t)blk * nodes * kF;
@@ -736,16 +756,20 @@ extern "C" int mlcg_filter_table_reverse(const int32_t* records, const int32_t* 
 extern "C" int mlcg_filter_table_combine(const int32_t* run_start, int64_t max_pairs, int nodes,
                                          int tangent, const float* slots, int num_blocks,
                                          const uint32_t* gates, float* wbar, float* wdbar,
+                                         float h, float* node_pos, float* node_dist,
+                                         int32_t* node_pair_ij, int32_t* node_count,
                                          void* stream) {
   MLCG_REQUIRE(table_shape_ok(nodes) && max_pairs >= 0 && num_blocks >= 1);
   MLCG_REQUIRE(run_start && slots && gates && wbar && wdbar);
+  MLCG_REQUIRE(node_pos && node_dist && node_pair_ij && node_count);
+  const NodePairs np{h, node_pos, node_dist, node_pair_ij, node_count};
   const int64_t stride = mlcg_filter_table_reverse_workspace_floats(max_pairs, nodes);
   const dim3 grid(nodes, num_blocks);
   if (tangent)
     hipLaunchKernelGGL((table_combine_kernel<true>), grid, dim3(256), 0, mlcg_stream(stream),
-                       run_start, nodes - 3, slots, stride, nodes, gates, wbar, wdbar);
+                       run_start, nodes - 3, slots, stride, nodes, gates, wbar, wdbar, np);
   else
     hipLaunchKernelGGL((table_combine_kernel<false>), grid, dim3(256), 0, mlcg_stream(stream),
-                       run_start, nodes - 3, slots, stride, nodes, gates, wbar, wdbar);
+                       run_start, nodes - 3, slots, stride, nodes, gates, wbar, wdbar, np);
   return mlcg_launch_status();
 }

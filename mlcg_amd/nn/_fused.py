@@ -70,7 +70,8 @@ class FusedSpec:
     basis_trainable: bool = False  # Params.basis carries (centers, widths)
     strict_fp32: bool = False  # filter forward on the fp32 MFMA throughout
     # the filters' distance grid: its shape (ops.filter_grid_shape of filt, None
-    # without one) and its tensors per device index
+    # without one) and its description per device index.  No tensors here: a
+    # recorded graph may outlive this object
     grid_shape: Optional[tuple] = None
     grids: dict = field(default_factory=dict)
 
@@ -78,7 +79,7 @@ class FusedSpec:
         self.grid_shape = ops.filter_grid_shape(self.filt)
 
     def __getstate__(self):
-        # a copy or a saved model makes its own grids, on the device it runs on
+        # a copy or a saved model describes its own grids, on the device it runs on
         return {**self.__dict__, "grids": {}}
 
 
@@ -299,9 +300,8 @@ def _table_pays(spec: FusedSpec, pairs: int, nodes: int, reverse: bool) -> bool:
 
 def _table_grid(spec: FusedSpec, filt, graph: ops.PairGraph, pos: torch.Tensor, reverse: bool):
     """The distance grid of this call's filters, or None where each pair's
-    filter is evaluated directly: too few pairs, strict fp32 filters, a filter
-    without a grid (ops.filter_grid_shape), or a stream capture that no call
-    has preceded (the grid's tensors come from the host)."""
+    filter is evaluated directly: too few pairs, strict fp32 filters, or a
+    filter without a grid (ops.filter_grid_shape)."""
     shape = spec.grid_shape
     if shape is None or spec.strict_fp32 or not pos.is_cuda or not graph.pair_capacity:
         return None
@@ -309,8 +309,9 @@ def _table_grid(spec: FusedSpec, filt, graph: ops.PairGraph, pos: torch.Tensor, 
             else _FILTER_TABLE and spec.num_blocks):
         return None
     grid = spec.grids.get(pos.device.index)
-    if grid is None and not torch.cuda.is_current_stream_capturing():
-        grid = spec.grids[pos.device.index] = ops.filter_grid(filt, pos.device)
+    if grid is None:
+        grid = spec.grids[pos.device.index] = ops.filter_grid(filt, pos.device,
+                                                              node_arrays=False)
     return grid
 
 
@@ -803,7 +804,7 @@ class _FilterReverse:
         spec, st = self.spec, self.st
         if self.slots is None or not self.grads:
             return self.grads, self.basis
-        grid, L, train = st.grid, len(self.grads), spec.basis_trainable
+        grid, L, train = st.grid.with_nodes(), len(self.grads), spec.basis_trainable
         weights = _filter_weights(self.P)
         self.grads = [ops.filter_grads(st.filt, st.pos.device) for _ in range(L)]
         wbar, wdbar = ops.filter_table_combine(grid, st.bins, st.graph,

@@ -10,7 +10,7 @@ from __future__ import annotations
 
 import ctypes
 import math
-from dataclasses import dataclass
+from dataclasses import dataclass, replace
 from typing import List, Optional, Tuple
 
 import torch
@@ -1077,15 +1077,27 @@ class FilterGrid:
     """Distance grid 0, h, .., (nodes - 1) h of a filter table over [0, rc], all
     exact in float32.  `cut`: distance from which the filter is exactly zero.
     pos / graph describe the nodes as pairs, for the kernels that take pairs;
-    dist holds their distances."""
+    dist holds their distances: written by filter_table_combine, and owned by the
+    call that reads them (a recorded graph finds them in its own pool)."""
 
     nodes: int
     h: float
     rc: float
     cut: float
-    pos: torch.Tensor
-    dist: torch.Tensor
-    graph: PairGraph
+    device: torch.device
+    pos: Optional[torch.Tensor] = None
+    dist: Optional[torch.Tensor] = None
+    graph: Optional[PairGraph] = None
+
+    def with_nodes(self) -> "FilterGrid":
+        """This grid with uninitialised node arrays of its own."""
+        n, dev = self.nodes, self.device
+        floats = torch.empty(4 * n, dtype=torch.float32, device=dev)
+        ints = torch.empty(2 * n + 1, dtype=torch.int32, device=dev)
+        graph = PairGraph(edge_index=None, rowptr=None, col=None,
+                          pair_ij=ints[:2 * n].view(2, n), pairptr=ints[2 * n:], eid2pair=None,
+                          frame_ptr=None, num_nodes=0, num_edges=2 * n, num_pairs=n)
+        return replace(self, pos=floats[:3 * n].view(n, 3), dist=floats[3 * n:], graph=graph)
 
 
 def filter_grid_shape(spec: FilterSpec) -> Optional[Tuple[int, float, float, float]]:
@@ -1118,25 +1130,14 @@ def filter_grid_shape(spec: FilterSpec) -> Optional[Tuple[int, float, float, flo
     return nodes, h, rc, float(spec.conv_hi) if spec.conv_cut_kind == 1 else 3.0e38
 
 
-def filter_grid(spec: FilterSpec, device) -> Optional[FilterGrid]:
-    """The grid with its device tensors (made on the host and copied, with one
-    synchronisation, so that any stream may use them)."""
+def filter_grid(spec: FilterSpec, device, node_arrays: bool = True) -> Optional[FilterGrid]:
+    """The filter's grid, with node arrays unless they are not wanted."""
     shape = filter_grid_shape(spec)
     if shape is None:
         return None
     nodes, h, rc, cut = shape
-    dist = torch.arange(nodes, dtype=torch.float32) * h
-    pos = torch.zeros(nodes, 3)
-    pos[:, 0] = dist
-    pair_ij = torch.zeros(2, nodes, dtype=torch.int32)
-    pair_ij[1] = torch.arange(nodes, dtype=torch.int32)
-    count = torch.full((1,), nodes, dtype=torch.int32)
-    pos, dist, pair_ij, count = (t.to(device) for t in (pos, dist, pair_ij, count))
-    torch.cuda.current_stream(device).synchronize()
-    graph = PairGraph(edge_index=None, rowptr=None, col=None, pair_ij=pair_ij, pairptr=count,
-                      eid2pair=None, frame_ptr=None, num_nodes=0, num_edges=2 * nodes,
-                      num_pairs=nodes)
-    return FilterGrid(nodes=nodes, h=h, rc=rc, cut=cut, pos=pos, dist=dist, graph=graph)
+    grid = FilterGrid(nodes=nodes, h=h, rc=rc, cut=cut, device=torch.device(device))
+    return grid.with_nodes() if node_arrays else grid
 
 
 @dataclass
@@ -1168,7 +1169,7 @@ def pair_bins(pos: torch.Tensor, graph: PairGraph, grid: FilterGrid) -> PairBins
 def filter_table_buffers(grid: FilterGrid, blocks: int) -> Tuple[torch.Tensor, torch.Tensor]:
     """(tables [L, 4, nodes + 1, F], gates [L, GATE_WORDS] cleared) for
     filter_tables."""
-    dev = grid.pos.device
+    dev = grid.device
     return (torch.empty(blocks, 4, grid.nodes + 1, NUM_FILTERS, dtype=torch.float32, device=dev),
             torch.zeros(blocks, GATE_WORDS, dtype=torch.int32, device=dev))
 
@@ -1180,7 +1181,7 @@ def filter_tables(grid: FilterGrid, spec: FilterSpec, weights, out=None
     `out` = filter_table_buffers(grid, len(weights)) by default (a caller that
     launches on another stream allocates them on the stream that consumes
     them)."""
-    dev = grid.pos.device
+    dev = grid.device
     L = len(weights)
     flat = _block_weights(spec, weights)
     tables, gates = filter_table_buffers(grid, L) if out is None else out
@@ -1363,7 +1364,7 @@ def filter_table_slots(grid: FilterGrid, graph: PairGraph, blocks: int) -> torch
     """[blocks, floats] partial sums of filter_table_reverse."""
     n = int(_lib.load().mlcg_filter_table_reverse_workspace_floats(graph.pair_capacity,
                                                                    grid.nodes))
-    return torch.empty(blocks, n, dtype=torch.float32, device=grid.pos.device)
+    return torch.empty(blocks, n, dtype=torch.float32, device=grid.device)
 
 
 def filter_table_reverse(grid: FilterGrid, bins: PairBins, graph: PairGraph,
@@ -1382,12 +1383,15 @@ def filter_table_reverse(grid: FilterGrid, bins: PairBins, graph: PairGraph,
 def filter_table_combine(grid: FilterGrid, bins: PairBins, graph: PairGraph, tangent: bool,
                          gates: torch.Tensor, slots: torch.Tensor
                          ) -> Tuple[torch.Tensor, torch.Tensor]:
-    """Adjoints (Wbar, Wdbar) [blocks, nodes, F] of the blocks' table values."""
+    """Adjoints (Wbar, Wdbar) [blocks, nodes, F] of the blocks' table values; also
+    writes the grid's node arrays."""
     L = slots.shape[0]
+    _check(grid.graph is not None, "filter_table_combine takes a grid with node arrays")
     wbar, wdbar = torch.empty(2, L, grid.nodes, NUM_FILTERS, dtype=torch.float32,
                               device=slots.device)
     call("mlcg_filter_table_combine", ptr(bins.runs), graph.pair_capacity, grid.nodes,
-         int(tangent), ptr(slots), L, ptr(gates), ptr(wbar), ptr(wdbar),
+         int(tangent), ptr(slots), L, ptr(gates), ptr(wbar), ptr(wdbar), grid.h, ptr(grid.pos),
+         ptr(grid.dist), ptr(grid.graph.pair_ij), ptr(grid.graph.pairptr),
          stream_handle(slots.device))
     return wbar, wdbar
 

@@ -238,3 +238,64 @@ def test_captured_train_step_requires_capturable_optimizer():
     opt = torch.optim.AdamW(model.parameters(), lr=1e-3)
     with pytest.raises(RuntimeError, match="capturable"):
         CapturedTrainStep(lambda d: nn.GradientsOut(model)(d), data, model, opt)
+
+
+def test_captured_step_outlives_the_kernel_description(monkeypatch):
+    """A recorded step through the filters' tables whose step function returns a
+    detached loss, so that only the graph itself holds what it reads; the
+    model's kernel description is then replaced (fp16 and strict filters
+    switched on and back for a validation call) and freed memory is written
+    over.  The replays still give the eager steps' parameters bit for bit."""
+    import gc
+
+    from mlcg_amd import nn, ops, synthetic
+    from mlcg_amd.nn import _fused
+    from mlcg_amd.pl import CapturedTrainStep
+
+    print("captured step across fp16 / strict filter switches", flush=True)
+    cfg = make_cfg(num_blocks=2, rc=20.0)
+    sd = R.random_state_dict(cfg, seed=37)
+    b = synthetic.config2(n_frames=16)
+    monkeypatch.setattr(_fused, "_FILTER_TABLE", True)
+    rows, seen = ops.filter_table_combine, []
+    monkeypatch.setattr(ops, "filter_table_combine",
+                        lambda *a: seen.append(len(seen)) or rows(*a))
+    runs = []
+    for captured in (False, True):
+        model = make_model(cfg, sd).train()
+        data = b.to_torch("cuda")
+        model.graph_capacity = 2 * (int(model.build_graph(data).num_edges * 1.25) // 2)
+        gm = nn.GradientsOut(model)
+        opt = torch.optim.AdamW(model.parameters(), lr=1e-3, fused=True, capturable=True)
+
+        def step(d):
+            opt.zero_grad(set_to_none=True)
+            out = gm(d)
+            out.out.update(**out.out[model.name])
+            loss = nn.ForceMSE()(out)
+            loss.backward()
+            opt.step()
+            return loss.detach()
+
+        params = []
+        cs = CapturedTrainStep(step, data, model, opt, warmup=1) if captured else step(data)
+        for k in range(3):
+            gm.eval()
+            for flag in ("fp16_filters", "strict_fp32_filters"):
+                setattr(model, flag, True)
+                gm(data.clone())
+                setattr(model, flag, False)
+                gm(data.clone())
+            gm.train()
+            gc.collect()
+            junk = [torch.full((1 << m,), 0x7fc00000, dtype=torch.int32, device="cuda")
+                    for m in range(8, 18) for _ in range(8)]  # NaN as a float
+            cs.step(data) if captured else step(data)
+            torch.cuda.synchronize()
+            del junk
+            params.append([p.detach().clone() for p in model.parameters()])
+        runs.append(params)
+    assert seen  # the steps went through the tables
+    for k, (a, c) in enumerate(zip(*runs)):
+        for x, y in zip(a, c):
+            assert torch.isfinite(x).all() and torch.equal(x, y), k

@@ -536,3 +536,24 @@ def test_filter_grids_stay_out_of_copies():
     spec.grids[0] = object()
     for other in (copy.deepcopy(spec), pickle.loads(pickle.dumps(spec))):
         assert other.grids == {} and other.grid_shape == spec.grid_shape
+
+
+def test_filter_grid_owns_no_device_memory(monkeypatch):
+    """A recorded training step may outlive the model's cached kernel
+    description (switching fp16 filters on and off replaces it), so neither the
+    description nor the grid it hands to a call holds a tensor."""
+    import types
+
+    import torch
+
+    from mlcg_amd.nn import _fused
+
+    spec = _fused.FusedSpec(filt=_filter_spec(), filter_act=0, block_act=0, out_act=0,
+                            num_blocks=1, out_has_bias=[True, False])
+    monkeypatch.setattr(_fused, "_FILTER_TABLE", True)
+    pos = types.SimpleNamespace(is_cuda=True, device=torch.device("cuda", 0))
+    graph = types.SimpleNamespace(pair_capacity=1000)
+    grid = _fused._table_grid(spec, spec.filt, graph, pos, True)
+    assert grid is spec.grids[0] and grid.nodes == spec.grid_shape[0]
+    assert not any(isinstance(v, torch.Tensor) for v in vars(grid).values())
+    assert grid.graph is None
