@@ -1368,7 +1368,7 @@ struct PairAdjoint {
   const float* dd;    //            ddot [P] (with g1)
 };
 
-// Blocks of one launch (blockIdx.y).
+// Blocks of one launch.
 struct BwdBlock {
   const float *W1, *b1, *W2;
   PairAdjoint adj;
@@ -1378,7 +1378,25 @@ struct BwdBlock {
 };
 struct BwdBatch {
   BwdBlock b[kMaxBlocks];
+  int n;
 };
+
+// Blocks of a launch whose gate lets them run, as bits.
+__device__ __forceinline__ unsigned bwd_running(const BwdBatch& batch) {
+  unsigned run = 0u;
+  for (int k = 0; k < batch.n; ++k)
+    if (!gate_closed(batch.b[k].gate)) run |= 1u << k;
+  return __builtin_amdgcn_readfirstlane(run);
+}
+
+// Workgroups of each running block: the launch's dealt out evenly, at most one
+// per 16 pairs.  Dealt on the device, since the gates are: with a share of a third
+// each, the one closed block of three would run on a third of the chip.
+__device__ __forceinline__ int bwd_share(int total, int64_t max_pairs, unsigned run) {
+  const int64_t tiles = max_pairs > 0 ? (max_pairs + 15) / 16 : 1;
+  const int most = total / __popc(run);
+  return (int)(tiles < most ? tiles : most);
+}
 
 __device__ __forceinline__ float4 ld4(const float* __restrict__ p, int64_t row, int col) {
   return *reinterpret_cast<const float4*>(p + row * kF + col);
@@ -1463,17 +1481,22 @@ __global__ __launch_bounds__(kBwdThreads) void filter_bwd_fused_kernel(
     const float* __restrict__ pos, const int32_t* __restrict__ pi,
     const int32_t* __restrict__ pj, const int32_t* __restrict__ n_pairs_dev,
     int64_t max_pairs, RbfParams rp, BwdBatch batch, float* __restrict__ partials) {
-  const BwdBlock& blk = batch.b[blockIdx.y];
+  unsigned run = bwd_running(batch);
+  if (run == 0u) return;
+  const int groups = bwd_share(gridDim.x, max_pairs, run);
+  const int turn = (int)blockIdx.x / groups;  // of the running blocks
+  if (turn >= __popc(run)) return;
+  const int group = (int)blockIdx.x - turn * groups;
+  for (int k = 0; k < turn; ++k) run &= run - 1u;
+  const BwdBlock& blk = batch.b[__builtin_ctz(run)];
   const FilterGate gate = blk.gate;
-  if (gate_closed(gate)) return;
   const float* __restrict__ W1 = blk.W1;
   const float* __restrict__ b1 = blk.b1;
   const float* __restrict__ W2 = blk.W2;
   const PairAdjoint adj = blk.adj;
   float* __restrict__ abar_out = blk.abar;
   float* __restrict__ adbar_out = blk.adbar;
-  float* __restrict__ partial =
-      partials + (int64_t)blockIdx.y * gridDim.x * bwd_partial_floats(rp.K);
+  float* __restrict__ partial = partials + (int64_t)turn * groups * bwd_partial_floats(rp.K);
   constexpr int KTMAX = (4 * KSMAX + 15) / 16;
   // basis rows span the compile-time maximum width (rows k >= K hold zeros),
   // so the k loops below run without data-dependent branches
@@ -1772,9 +1795,9 @@ __global__ __launch_bounds__(kBwdThreads) void filter_bwd_fused_kernel(
   // XCDs, and the workgroups of one XCD take one contiguous range of tiles
   // (strided among them), so the node rows of a frame's pairs are fetched
   // into that XCD's L2 only, not into every XCD's (config 2: 269.5 -> 265 us).
-  const int nx = (int)gridDim.x < kBwdXcds ? (int)gridDim.x : kBwdXcds;
-  const int xcd = blockIdx.x % nx, wl = blockIdx.x / nx;
-  const int64_t stride = gridDim.x / nx + (xcd < (int)(gridDim.x % nx) ? 1 : 0);
+  const int nx = groups < kBwdXcds ? groups : kBwdXcds;
+  const int xcd = group % nx, wl = group / nx;
+  const int64_t stride = groups / nx + (xcd < groups % nx ? 1 : 0);
   const int64_t t_start = tiles * xcd / nx + wl, t_end = tiles * (xcd + 1) / nx;
   if (np > 0) {  // uniform across the workgroup
     const int64_t p0 = clamp_pair(t_start);
@@ -2164,7 +2187,7 @@ __global__ __launch_bounds__(kBwdThreads) void filter_bwd_fused_kernel(
     for (int kt = 0; kt < KTMAX; ++kt) acc1[kt] *= f1;
   }
   // partial sums of this workgroup: [dW2 (F x F) | dW1 (F x Kp16) | db1 (F)]
-  float* out = partial + (int64_t)blockIdx.x * bwd_partial_floats(K);
+  float* out = partial + (int64_t)group * bwd_partial_floats(K);
 #pragma unroll
   for (int u = 0; u < kFT; ++u)
 #pragma unroll
@@ -2197,14 +2220,17 @@ __global__ __launch_bounds__(kBwdThreads) void filter_bwd_fused_kernel(
 constexpr int kRedOut = 64;
 
 __global__ __launch_bounds__(256) void filter_bwd_reduce_kernel(
-    const float* __restrict__ partials, int groups, int K, BwdBatch batch) {
+    const float* __restrict__ partials, int total_groups, int64_t max_pairs, int K,
+    BwdBatch batch) {
+  const unsigned run = bwd_running(batch), me = 1u << blockIdx.y;
+  if (!(run & me)) return;
   const BwdBlock& blk = batch.b[blockIdx.y];
-  if (gate_closed(blk.gate)) return;
+  const int groups = bwd_share(total_groups, max_pairs, run);
+  const int turn = __popc(run & (me - 1u));
   float* __restrict__ dW1 = blk.dW1;
   float* __restrict__ db1 = blk.db1;
   float* __restrict__ dW2 = blk.dW2;
-  const float* __restrict__ partial =
-      partials + (int64_t)blockIdx.y * groups * bwd_partial_floats(K);
+  const float* __restrict__ partial = partials + (int64_t)turn * groups * bwd_partial_floats(K);
   __shared__ float part[4][kRedOut];
   const int Kp16 = bwd_kp16(K);
   const int stride = bwd_partial_floats(K);
@@ -2240,12 +2266,11 @@ __global__ __launch_bounds__(256) void filter_bwd_reduce_kernel(
   if (slice == 0 && dst) *dst = (part[0][o] + part[1][o]) + (part[2][o] + part[3][o]);
 }
 
-// Workgroups of one of n blocks: one per CU in all (a workgroup's 144 KiB of LDS
-// leave no room for a second), so that a batch's weights are staged once.
+// Workgroups of n blocks: one per CU in all (a workgroup's 144 KiB of LDS leave
+// no room for a second), so that a batch's weights are staged once.
 int bwd_groups(int64_t max_pairs, int n) {
-  const int64_t tiles = (max_pairs + 15) / 16;
-  const int64_t most = 256 / n;
-  return (int)(tiles < most ? (tiles < 1 ? 1 : tiles) : most);
+  const int64_t tiles = max_pairs > 0 ? (max_pairs + 15) / 16 : 1;
+  return (int)(n * tiles < 256 ? n * tiles : 256);
 }
 
 // Kernels here use more than 64 KiB of dynamic LDS; raise their limit to the
@@ -2524,7 +2549,7 @@ int launch_filter_bwd(const float* pos, const int32_t* pair_ij, int64_t pair_str
     MLCG_REQUIRE((b.abar == nullptr) == (b.adbar == nullptr));
   }
   const int groups = bwd_groups(max_pairs, n);
-  MLCG_REQUIRE(workspace_floats >= (int64_t)n * groups * bwd_partial_floats(num_rbf));
+  MLCG_REQUIRE(workspace_floats >= (int64_t)groups * bwd_partial_floats(num_rbf));
   RbfParams rp = make_params(basis, centers, widths, alpha, num_rbf, rbf_cut_kind, rbf_lo,
                              rbf_hi, conv_cut_kind, conv_lo, conv_hi, act);
   hipStream_t s = mlcg_stream(stream);
@@ -2533,9 +2558,8 @@ int launch_filter_bwd(const float* pos, const int32_t* pair_ij, int64_t pair_str
   const bool small_k = num_rbf <= 64 && !fp32_strict;
   const size_t lds = sizeof(float) * bwd_lds_floats(small_k ? num_rbf : kMaxK);
   allow_lds_once();
-  const int grid = max_pairs == 0 ? 1 : groups;
 #define MLCG_BWD_LAUNCH(KS, NODES, B, A)                                                      \
-  hipLaunchKernelGGL((filter_bwd_fused_kernel<KS, NODES, B, A>), dim3(grid, n),              \
+  hipLaunchKernelGGL((filter_bwd_fused_kernel<KS, NODES, B, A>), dim3(groups),               \
                      dim3(kBwdThreads), lds, s, pos, pair_ij, pair_ij + pair_stride,         \
                      n_pairs_dev, max_pairs, rp, batch, workspace)
 #define MLCG_BWD_SMALL(NODES)                                   \
@@ -2556,7 +2580,7 @@ int launch_filter_bwd(const float* pos, const int32_t* pair_ij, int64_t pair_str
 #undef MLCG_BWD_LAUNCH
   const int total = kF * kF + kF * num_rbf + kF;
   hipLaunchKernelGGL(filter_bwd_reduce_kernel, dim3((total + kRedOut - 1) / kRedOut, n),
-                     dim3(256), 0, s, workspace, groups, num_rbf, batch);
+                     dim3(256), 0, s, workspace, groups, max_pairs, num_rbf, batch);
   return mlcg_launch_status();
 }
 
@@ -2574,6 +2598,7 @@ extern "C" int mlcg_filter_bwd(const float* pos, const int32_t* pair_ij, int64_t
                                int fp32_strict, void* stream) {
   MLCG_REQUIRE(max_pairs == 0 || (Wbar && Wdbar));
   BwdBatch batch = {};
+  batch.n = 1;
   batch.b[0] = BwdBlock{W1, b1, W2, {Wbar, Wdbar, nullptr, nullptr, nullptr, nullptr, nullptr},
                         abar_out, adbar_out, dW1, db1, dW2, {nullptr, 0}};
   return launch_filter_bwd(pos, pair_ij, pair_stride, n_pairs_dev, max_pairs, basis, centers,
@@ -2597,6 +2622,7 @@ extern "C" int mlcg_filter_bwd_cfconv(const float* pos, const int32_t* pair_ij,
   MLCG_REQUIRE(max_pairs == 0 || (gagg2 && y));
   MLCG_REQUIRE(!gagg1 || ddot);
   BwdBatch batch = {};
+  batch.n = 1;
   batch.b[0] = BwdBlock{W1, b1, W2,
                         {nullptr, nullptr, gagg2, y, gagg1, gagg1 ? ydot : nullptr, ddot},
                         abar_out, adbar_out, dW1, db1, dW2, {nullptr, 0}};
@@ -2610,7 +2636,7 @@ extern "C" int64_t mlcg_filter_bwd_blocks_workspace_floats(int64_t max_pairs, in
                                                            int num_blocks) {
   if (max_pairs < 0 || num_rbf < 1 || num_rbf > kMaxK || num_blocks < 1) return -1;
   const int n = num_blocks < kMaxBlocks ? num_blocks : kMaxBlocks;
-  return (int64_t)n * bwd_groups(max_pairs, n) * bwd_partial_floats(num_rbf);
+  return (int64_t)bwd_groups(max_pairs, n) * bwd_partial_floats(num_rbf);
 }
 
 extern "C" int mlcg_filter_bwd_blocks(const float* pos, const int32_t* pair_ij,
@@ -2626,6 +2652,7 @@ extern "C" int mlcg_filter_bwd_blocks(const float* pos, const int32_t* pair_ij,
   for (int first = 0; first < num_blocks; first += kMaxBlocks) {
     const int n = num_blocks - first < kMaxBlocks ? num_blocks - first : kMaxBlocks;
     BwdBatch batch = {};
+    batch.n = n;
     bool nodes = false;
     for (int k = 0; k < n; ++k) {
       auto at = [&](int x) { return static_cast<float*>(blocks[15 * (first + k) + x]); };

@@ -264,3 +264,38 @@ def test_gate_is_the_blocks_own():
     for a, b in zip(_step(model, True), _step(model, False)):
         assert rel_err(a, b) <= 1e-5, rel_err(a, b)
     ops.numerics_flags("cuda", clear=True)
+
+
+@pytest.mark.parametrize("n", [15, 700, 20001])
+@pytest.mark.parametrize("closed", [(0,), (1,), (0, 2), (0, 1, 2)])
+def test_closed_blocks_share_the_launch(n, closed):
+    """Of a three-block launch for the blocks whose gate is closed, those take
+    all the workgroups: the gradients equal, bit for bit, those of a launch of
+    the closed blocks alone, and the others' stay untouched.  The same for the
+    launch on the open ones."""
+    from mlcg_amd import ops
+
+    model = _model(blocks=3)
+    spec, P = model.fused_spec(), model.fused_params()
+    weights = [(b.W1, b.b1, b.W2) for b in P.blocks]
+    pos, graph = _pairs(_distances(n, 0.01, seed=n))
+    g = torch.Generator("cuda").manual_seed(n)
+    adj = [tuple(torch.randn(n, 128, device="cuda", generator=g) for _ in range(2))
+           for _ in range(3)]
+    gates = torch.zeros(3, ops.GATE_WORDS, dtype=torch.int32, device="cuda")
+    for k in closed:
+        gates[k, 8] = 0x7f800000  # a pre-activation's change per node: infinite
+    for want, blocks in ((0, closed), (1, [k for k in range(3) if k not in closed])):
+        def run(which):
+            grads = [tuple(t.fill_(7.0) for t in ops.filter_grads(spec.filt, "cuda"))
+                     for _ in which]
+            ops.filter_bwd_blocks(pos, graph, spec.filt, [weights[k] for k in which],
+                                  [adj[k] for k in which], grads,
+                                  gates[list(which)].contiguous(), want)
+            return grads
+
+        got = run(range(3))
+        alone = dict(zip(blocks, run(blocks))) if blocks else {}
+        for k in range(3):
+            for x, y in zip(got[k], alone.get(k, (7.0, 7.0, 7.0))):
+                assert torch.equal(x, y) if k in alone else bool((x == y).all()), (want, k)
