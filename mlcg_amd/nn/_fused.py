@@ -813,15 +813,22 @@ class _FilterReverse:
         nodes = ops.filter_bwd_blocks(grid.pos, grid.graph, st.filt, weights,
                                       list(zip(wbar, wdbar)), self.grads, st.gates, 1,
                                       pair_adjoints=train)
-        pairs = ops.filter_bwd_blocks(st.pos, st.graph, st.filt, weights, self.adjoints,
-                                      self.grads, st.gates, 0, pair_adjoints=train)
-        if train:
-            for k in range(L - 1, -1, -1):
-                W1, gate, first = weights[k][0], st.gates[k], self.basis is None
-                self.basis = ops.rbf_param_grad(grid.dist, grid.graph, st.filt, W1, *nodes[k],
-                                                out=self.basis, gate=gate, gate_want=1)
-                ops.rbf_param_grad(st.dist, st.graph, st.filt, W1, *pairs[k], out=self.basis,
-                                   accumulate=not first, gate=gate, gate_want=0)
+        if not train:
+            ops.filter_bwd_blocks(st.pos, st.graph, st.filt, weights, self.adjoints, self.grads,
+                                  st.gates, 0)
+            return self.grads, self.basis
+        for k in range(L - 1, -1, -1):
+            W1, gate, first = weights[k][0], st.gates[k], self.basis is None
+            self.basis = ops.rbf_param_grad(grid.dist, grid.graph, st.filt, W1, *nodes[k],
+                                            out=self.basis, gate=gate, gate_want=1)
+            # the pairs block by block: the first-layer adjoints are [P, F] each, the
+            # largest arrays of the step (3 blocks, 89 k pairs: peak 655 MiB against 830)
+            pairs, = ops.filter_bwd_blocks(st.pos, st.graph, st.filt, weights[k:k + 1],
+                                           self.adjoints[k:k + 1], self.grads[k:k + 1],
+                                           st.gates[k:k + 1], 0, pair_adjoints=True)
+            ops.rbf_param_grad(st.dist, st.graph, st.filt, W1, *pairs, out=self.basis,
+                               accumulate=not first, gate=gate, gate_want=0)
+            del pairs
         return self.grads, self.basis
 
 

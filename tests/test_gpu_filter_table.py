@@ -299,3 +299,27 @@ def test_closed_blocks_share_the_launch(n, closed):
         for k in range(3):
             for x, y in zip(got[k], alone.get(k, (7.0, 7.0, 7.0))):
                 assert torch.equal(x, y) if k in alone else bool((x == y).all()), (want, k)
+
+
+@pytest.mark.parametrize("table", [True, False])
+def test_one_block_of_first_layer_adjoints_at_a_time(table, monkeypatch):
+    """With a trainable basis the [P, F] first-layer adjoints of one block are
+    alive at a time, on either route."""
+    import weakref
+
+    from mlcg_amd import ops
+
+    make, alive, most = ops._pair_adjoint_outputs, [], [0]
+
+    def outputs(want, cap, F, dev):
+        out = make(want, cap, F, dev)
+        if want and cap > 10000:  # the pairs', not the grid nodes'
+            alive.extend(weakref.ref(t) for t in out)
+            most[0] = max(most[0], sum(r() is not None for r in alive))
+        return out
+
+    monkeypatch.setattr(ops, "_pair_adjoint_outputs", outputs)
+    model = _model("expnormal", trainable=True, blocks=3)
+    model.graph_capacity = 40000  # past the number of nodes
+    _step(model, table)
+    assert most[0] == 2
