@@ -349,9 +349,10 @@ int mlcg_filter_bwd(const float* pos, const int32_t* pair_ij,
  * the pre-activations' change per node, mlcg_filter_table_check the others.
  * A block's table serves when interpolating every second node at twice the
  * spacing from the others errs by less than 4e-6 of the largest value (1.6e-5
- * for derivatives; the interpolation used errs by 2^-4 of that), and no
- * pre-activation changes by more than 1/4 between nodes; non-finite values and
- * weights of magnitude 65504 or more never pass.  Entry points
+ * for derivatives; the interpolation used errs by 2^-4 of that), no
+ * pre-activation changes by more than 1/4 between nodes and no basis function
+ * is narrower than the spacing; non-finite values and weights of magnitude
+ * 65504 or more never pass.  Entry points
  * with a gate do their work only if the block's table serves (gate_want 1) or
  * does not (0), decided on the device. */
 enum { MLCG_GATE_WORDS = 12 };

@@ -540,6 +540,13 @@ __global__ __launch_bounds__(kThreads) void filter_table_kernel(
   for (int u = 0; u < kFT; ++u) a2[u] = *reinterpret_cast<const float4*>(W2 + 16 * u);
   const float4 bias = *reinterpret_cast<const float4*>(fb.b1[blk] + 16 * w + 4 * q);
   const float bv[4] = {bias.x, bias.y, bias.z, bias.w};
+  // A basis function exp(-b x^2) with b h^2 above 1, h the spacing, falls by more
+  // than 1/4 between neighbouring nodes and could pass between them unseen: it
+  // closes the gate.  x is the distance, or the exponential-normal basis'
+  // exp(alpha (lo - d)), whose slope is largest at d = 0.
+  const double step =
+      (double)h * (rp.basis == 0 ? 1.0 : rp.alpha64 * exp(rp.alpha64 * (double)rp.rbf_lo));
+  bool resolved = true;
   // the basis at the nodes, each wave its k steps
 #pragma unroll
   for (int t = 0; t < kTableTiles; ++t) {
@@ -549,9 +556,11 @@ __global__ __launch_bounds__(kThreads) void filter_table_kernel(
     cutoff_f64(rp.rbf_kind, rp.rbf_hi, d, crbf, dcrbf);
     for (int s = w; s < KSMAX; s += kWaves) {
       double g = 0.0, gd = 0.0;
-      if (4 * s + q < K)
-        rbf_f64(rp, rp.centers[4 * s + q], rp.widths[rp.basis == 0 ? 0 : 4 * s + q], d, crbf,
-                dcrbf, g, gd);
+      if (4 * s + q < K) {
+        const double wid = rp.widths[rp.basis == 0 ? 0 : 4 * s + q];
+        resolved = resolved && fabs(wid) * step * step <= 1.0;  // false for a NaN
+        rbf_f64(rp, rp.centers[4 * s + q], wid, d, crbf, dcrbf, g, gd);
+      }
       gs[t][0][4 * s + q][n] = (float)g;
       gs[t][1][4 * s + q][n] = (float)gd;
     }
@@ -569,7 +578,7 @@ __global__ __launch_bounds__(kThreads) void filter_table_kernel(
   for (int u = 0; u < kFT; ++u)
     big = fmaxf(big, fmaxf(fmaxf(fabsf(a2[u].x), fabsf(a2[u].y)),
                            fmaxf(fabsf(a2[u].z), fabsf(a2[u].w))));
-  if (!(big < kWeightBound)) steep = __float_as_uint(__builtin_huge_valf());
+  if (!(big < kWeightBound) || !resolved) steep = __float_as_uint(__builtin_huge_valf());
 #pragma unroll
   for (int t = 0; t < kTableTiles; ++t) {
     const int k = (blockIdx.x * kTableTiles + t) * 16 + n;

@@ -11,8 +11,10 @@
 // error is 2^-4 of the measured one: at the bounds below 2.5e-7 of the largest
 // value and 1e-6 of the largest derivative -- the rounding of the fp32
 // evaluation itself (3.4e-7 and 6e-7; the split-fp16 kernels' derivative:
-// 4.7e-6).  A pre-activation that changes by less than 1/4 per node cannot
-// hide a feature between two nodes.
+// 4.7e-6).  Basis functions narrower than the spacing, which could lie between
+// two nodes unseen, set the last word to infinity; of wider ones the nodes see
+// every feature, and a pre-activation that changes by less than 1/4 per node
+// leaves the activation none of its own.
 #pragma once
 
 #include "common.h"

@@ -323,3 +323,32 @@ def test_one_block_of_first_layer_adjoints_at_a_time(table, monkeypatch):
     model.graph_capacity = 40000  # past the number of nodes
     _step(model, table)
     assert most[0] == 2
+
+
+@pytest.mark.parametrize("basis", ["gaussian", "expnormal"])
+def test_narrow_basis_between_nodes_closes_the_gate(basis):
+    """Trained basis functions of a fiftieth of the grid's spacing, centred
+    between nodes: every node sees a smooth filter (the functions are e^-300
+    there), the pairs at the centres do not, so they go pair by pair.  A
+    centre's float rounding (1e-6 A, a fortieth of the width) takes 3e-4 off a
+    peak: 1e-2 of the largest value."""
+    from mlcg_amd import ops
+
+    model = _model(basis, num_rbf=50, trainable=True)
+    h = ops.filter_grid_shape(model.fused_spec().filt)[1]
+    d = ((torch.arange(50).double() * RC / 50 / h).floor() + 0.5) * h
+    alpha = 5.0 / RC
+    with torch.no_grad():
+        if basis == "gaussian":
+            model.rbf_layer.coeff.fill_(-0.5 / (0.02 * h) ** 2)
+            model.rbf_layer.offset.copy_(d)
+        else:
+            slope = alpha * torch.exp(-alpha * d)
+            model.rbf_layer.betas.copy_(0.5 / (0.02 * h * slope) ** 2)
+            model.rbf_layer.means.copy_(torch.exp(-alpha * d))
+    dist = d.float()
+    spec, b, grid, pos, graph, tables, gates, bins = _setup(model, dist)
+    out, = ops.filter_rows(grid, bins, pos, graph, spec.filt, [(b.W1, b.b1, b.W2)], tables, gates)
+    ref = _filters64(model, dist)[0]
+    assert (out[0].double().cpu() - ref).abs().max() <= 1e-2 * ref.abs().max()
+    ops.numerics_flags("cuda", clear=True)
