@@ -1390,12 +1390,11 @@ struct BwdBatch {
   int n;
 };
 
-// Blocks of a launch whose gate lets them run, as bits.
+// Blocks of a launch whose gate lets them run, as bits: lane k looks at block k's,
+// so that a workgroup waits for one gate's words, not for all blocks' in turn.
 __device__ __forceinline__ unsigned bwd_running(const BwdBatch& batch) {
-  unsigned run = 0u;
-  for (int k = 0; k < batch.n; ++k)
-    if (!gate_closed(batch.b[k].gate)) run |= 1u << k;
-  return __builtin_amdgcn_readfirstlane(run);
+  const int k = mlcg_lane();
+  return (unsigned)__ballot(k < batch.n && !gate_closed(batch.b[k < batch.n ? k : 0].gate));
 }
 
 // Workgroups of each running block: the launch's dealt out evenly, at most one

@@ -30,11 +30,12 @@ struct FilterGate {
 };
 
 __device__ __forceinline__ bool filter_table_serves(const unsigned* __restrict__ g) {
-  return __uint_as_float(g[0]) <= kGateValueTol * __uint_as_float(g[4]) &&
-         __uint_as_float(g[1]) <= kGateDerivTol * __uint_as_float(g[5]) &&
-         __uint_as_float(g[2]) <= kGateValueTol * __uint_as_float(g[6]) &&
-         __uint_as_float(g[3]) <= kGateDerivTol * __uint_as_float(g[7]) &&
-         __uint_as_float(g[8]) <= kGateSlope;
+  // & and not &&: the words are read together, not one after the other
+  return (__uint_as_float(g[0]) <= kGateValueTol * __uint_as_float(g[4])) &
+         (__uint_as_float(g[1]) <= kGateDerivTol * __uint_as_float(g[5])) &
+         (__uint_as_float(g[2]) <= kGateValueTol * __uint_as_float(g[6])) &
+         (__uint_as_float(g[3]) <= kGateDerivTol * __uint_as_float(g[7])) &
+         (__uint_as_float(g[8]) <= kGateSlope);
 }
 
 __device__ __forceinline__ bool gate_closed(const FilterGate& gate) {
