@@ -10,7 +10,7 @@ from __future__ import annotations
 
 import ctypes
 import math
-from dataclasses import dataclass, replace
+from dataclasses import dataclass
 from typing import List, Optional, Tuple
 
 import torch
@@ -1092,12 +1092,13 @@ class FilterGrid:
     def with_nodes(self) -> "FilterGrid":
         """This grid with uninitialised node arrays of its own."""
         n, dev = self.nodes, self.device
-        floats = torch.empty(4 * n, dtype=torch.float32, device=dev)
-        ints = torch.empty(2 * n + 1, dtype=torch.int32, device=dev)
         graph = PairGraph(edge_index=None, rowptr=None, col=None,
-                          pair_ij=ints[:2 * n].view(2, n), pairptr=ints[2 * n:], eid2pair=None,
+                          pair_ij=torch.empty(2, n, dtype=torch.int32, device=dev),
+                          pairptr=torch.empty(1, dtype=torch.int32, device=dev), eid2pair=None,
                           frame_ptr=None, num_nodes=0, num_edges=2 * n, num_pairs=n)
-        return replace(self, pos=floats[:3 * n].view(n, 3), dist=floats[3 * n:], graph=graph)
+        return FilterGrid(n, self.h, self.rc, self.cut, dev,
+                          torch.empty(n, 3, dtype=torch.float32, device=dev),
+                          torch.empty(n, dtype=torch.float32, device=dev), graph)
 
 
 def filter_grid_shape(spec: FilterSpec) -> Optional[Tuple[int, float, float, float]]:
