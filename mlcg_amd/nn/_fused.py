@@ -279,23 +279,29 @@ def _table_pays(spec: FusedSpec, pairs: int, nodes: int, reverse: bool) -> bool:
     """Whether the filters go through a table (csrc/filter_table.hip) instead of
     one network evaluation per pair.  The table costs its nodes and the ordering
     of the pairs once per call and, with a reverse sweep, some launches per
-    block; it saves time per pair and block.  Measured with 35-bead chains, us on
-    the device / in all, issued eagerly (direct, table).  Energies and forces,
-    Gaussian basis (2551 nodes), 3 blocks: 62 k pairs 311 / 338, 313 / 351, 106 k
-    443 / 465, 427 / 457, 215 k 756 / 759, 673 / 700; 1 block: 215 k 264 / 293,
-    273 / 300; exponential-normal basis (7242 nodes), 2 blocks: 137 k 346 / 374,
-    389 / 412.  Force-matching gradient, Gaussian, 3 blocks: 42 k 735 / 1241, 710 /
-    1176, 62 k 919 / 1061, 822 / 1174, 106 k 1312 / 1326, 1113 / 1263, 215 k 2261 /
-    2209, 1794 / 1827; 1 block: 106 k 479 / 714, 445 / 883, 215 k 800 / 840, 670 /
-    866; exponential-normal, trainable (the basis' gradient is then taken at the
-    nodes too, which saves three times as much a pair), 2 blocks: 55 k 726 / 1004,
-    669 / 1115, 137 k 1281 / 1292, 984 / 1143.  The lines lie between where the
-    device's time breaks even, which a captured step sees, and where an eager
-    call's does."""
+    block; it saves time per pair and block.
+
+    Measured with 35-bead chains.  Energies and forces, us issued eagerly (direct,
+    table): Gaussian basis (2551 nodes), 3 blocks, 63 k pairs 451, 439; 107 k 563,
+    541; 161 k 713, 664; 1 block, 170 k 320, 330; 219 k 366, 365; 296 k 423, 421.
+
+    Force-matching step, us eagerly, then recorded in a graph with 1.25 times the
+    pairs as capacity (direct, table each).  Gaussian, 1 block, 134 k pairs 775,
+    844, recorded 586, 521; 161 k 845, 846, 664, 576; 177 k 852, 844, 706, 603; 219 k
+    947, 876, 831, 701.  2 blocks, 93 k 1003, 1027, 818, 726; 107 k 1093, 1032, 937,
+    813.  3 blocks, 63 k 1176, 1216, 967, 870; 76 k 1252, 1195, 1068, 934.
+    Exponential-normal (7242 nodes), trainable (the basis' gradient is then taken
+    at the nodes too, which saves three times as much a pair), 2 blocks, 55 k 1021,
+    1180, 751, 692; 71 k 1094, 1163, 829, 754; 89 k 1199, 1162, 961, 814.  The line
+    is where eager steps of a Gaussian basis break even; recorded ones, with no
+    host cost, do so at fewer pairs.  With the trainable basis eager steps break
+    even only at 80 k pairs, but the line lies at 57 k: in between they lose 6 %
+    and recorded ones gain 9 %."""
     work = pairs * spec.num_blocks
     if not reverse:
         return work >= 48 * nodes + 150_000
-    return work * (3 if spec.basis_trainable else 1) >= 32 * nodes + 50_000 * spec.num_blocks
+    return (work * (3 if spec.basis_trainable else 1)
+            >= 32 * nodes + 78_000 + 17_000 * spec.num_blocks)
 
 
 def _table_grid(spec: FusedSpec, filt, graph: ops.PairGraph, pos: torch.Tensor, reverse: bool):
@@ -395,9 +401,9 @@ def forward(spec: FusedSpec, P: Params, pos: torch.Tensor, types: torch.Tensor,
             rev_seed: Optional[torch.Tensor] = None,
             reverse: bool = True) -> Tuple[torch.Tensor, State]:
     """Energies [B] and the saved state; reverse: a parameter sweep (reverse2) is
-    likely to follow, which only the choice of the filters' route looks at.  With rev_seed, the output network's
-    kernel also forms the adjoint a following reverse1(seed=rev_seed) starts
-    from."""
+    likely to follow, which only the choice of the filters' route looks at.
+    With rev_seed, the output network's kernel also forms the adjoint a
+    following reverse1(seed=rev_seed) starts from."""
     st = State(pos=pos, types=types, graph=graph, filt=filter_spec(spec, P))
     if (P.emb.dim() == 2 and P.emb.shape[1] == ops.NUM_FILTERS
             and P.emb.dtype == torch.float32 and types.dtype == torch.int64):

@@ -557,3 +557,21 @@ def test_filter_grid_owns_no_device_memory(monkeypatch):
     assert grid is spec.grids[0] and grid.nodes == spec.grid_shape[0]
     assert not any(isinstance(v, torch.Tensor) for v in vars(grid).values())
     assert grid.graph is None
+
+
+@pytest.mark.parametrize("blocks,pairs,exp_trainable,table", [
+    (1, 133_733, False, False), (1, 161_193, False, False), (1, 190_568, False, True),
+    (2, 92_945, False, False), (2, 107_150, False, True),
+    (3, 63_007, False, False), (3, 76_132, False, True),
+    (2, 54_677, True, False), (2, 88_643, True, True),
+])
+def test_filter_route_of_a_training_step(blocks, pairs, exp_trainable, table):
+    """The sizes on both sides of where an eagerly issued force-matching step
+    was measured to break even between the two routes."""
+    from mlcg_amd.nn import _fused
+
+    filt = _filter_spec() if not exp_trainable else _filter_spec(
+        basis=1, alpha=5 / 30.0, num_rbf=64, rbf_hi=30.0, conv_hi=30.0)
+    spec = _fused.FusedSpec(filt=filt, filter_act=0, block_act=0, out_act=0, num_blocks=blocks,
+                            out_has_bias=[True, False], basis_trainable=exp_trainable)
+    assert _fused._table_pays(spec, pairs, spec.grid_shape[0], True) == table
