@@ -956,12 +956,13 @@ class EnergyForces(torch.autograd.Function):
 
 class Energy(torch.autograd.Function):
     """E [B] with a first-order backward that is itself differentiable
-    (EnergyGrad), for generic autograd.grad(E, pos, create_graph=True) use."""
+    (EnergyGrad), for generic autograd.grad(E, pos, create_graph=True) use.
+    grad: gradients are enabled in the caller."""
 
     @staticmethod
-    def forward(ctx, spec, types, batch, graph, pos, *flat):
+    def forward(ctx, spec, types, batch, graph, grad, pos, *flat):
         P = Params.unflat(spec, list(flat))
-        E, st = forward(spec, P, pos.detach(), types, graph, save=True)
+        E, st = forward(spec, P, pos.detach(), types, graph, save=True, reverse=grad)
         ctx.spec, ctx.P, ctx.st, ctx.batch = spec, P, st, batch
         ctx.save_for_backward(pos, *flat)
         return E
@@ -970,7 +971,7 @@ class Energy(torch.autograd.Function):
     def backward(ctx, Ebar):
         pos, *flat = ctx.saved_tensors
         out = EnergyGrad.apply(ctx.spec, ctx.st, ctx.batch, Ebar, pos, *flat)
-        return (None, None, None, None, *out)
+        return (None, None, None, None, None, *out)
 
 
 class EnergyGrad(torch.autograd.Function):

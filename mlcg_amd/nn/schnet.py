@@ -356,7 +356,8 @@ class SchNet(torch.nn.Module):
         pos = data.pos
         batch = data.batch if "batch" in data else torch.zeros(
             pos.shape[0], dtype=torch.long, device=pos.device)
-        E = _fused.Energy.apply(spec, data.atom_types, batch, graph, pos.float(), *P.flat())
+        E = _fused.Energy.apply(spec, data.atom_types, batch, graph, torch.is_grad_enabled(),
+                                pos.float(), *P.flat())
         data.out[self.name] = {ENERGY_KEY: E}
         return data
 

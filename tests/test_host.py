@@ -575,3 +575,32 @@ def test_filter_route_of_a_training_step(blocks, pairs, exp_trainable, table):
     spec = _fused.FusedSpec(filt=filt, filter_act=0, block_act=0, out_act=0, num_blocks=blocks,
                             out_has_bias=[True, False], basis_trainable=exp_trainable)
     assert _fused._table_pays(spec, pairs, spec.grid_shape[0], True) == table
+
+
+def test_energies_without_gradients_take_the_forward_route(monkeypatch):
+    """Energies alone, with gradients disabled, weigh the table without its
+    reverse."""
+    import types
+
+    import torch
+
+    from mlcg_amd.data import AtomicData
+    from mlcg_amd.nn import SchNet, _fused, schnet
+
+    seen = []
+
+    def apply(spec, types, batch, graph, grad, pos, *flat):
+        seen.append(grad)
+        return pos.sum()
+
+    monkeypatch.setattr(_fused, "Energy", types.SimpleNamespace(apply=apply))
+    monkeypatch.setattr(schnet, "require_device", lambda *a: None)
+    model = types.SimpleNamespace(
+        name=SchNet.name, fused_spec=lambda: object(), build_graph=lambda d: None,
+        fused_params=lambda: types.SimpleNamespace(flat=lambda: []))
+    data = AtomicData(pos=torch.zeros(2, 3), atom_types=torch.ones(2, dtype=torch.long))
+    data.out = {}
+    SchNet.forward(model, data)
+    with torch.no_grad():
+        SchNet.forward(model, data)
+    assert seen == [True, False]
