@@ -1108,7 +1108,12 @@ def filter_grid_shape(spec: FilterSpec) -> Optional[Tuple[int, float, float, flo
     the smallest width of the basis functions over 52 (Gaussian) or over 32
     (exponential-normal, whose functions widen from zero distance on): the
     check then passes with a margin of 30 and 4, i.e. for filters 2.4 and 1.4
-    times as sharp as their basis."""
+    times as sharp as their basis.  Of those up to a tenth narrower, the widest
+    is taken that leaves at most 1/8 of a cell between the last node and rc (the
+    least, next to TABLE_MAX_NODES):
+    past the last node the interpolation weights grow, to 15 in sum a whole cell
+    away (a filter that does not vanish at rc: 1.7e-6 of the largest value
+    there, 4e-7 elsewhere)."""
     rc = float(spec.rbf_hi)
     K = int(spec.num_rbf)
     if not (0.0 < rc < 1e30) or K < 2:
@@ -1124,10 +1129,16 @@ def filter_grid_shape(spec: FilterSpec) -> Optional[Tuple[int, float, float, flo
             return None
         fine = math.sqrt(2.0) / (K * spec.alpha) / 32.0
     ulp = 2.0 ** (math.floor(math.log2(fine)) - 10)
-    h = math.floor(fine / ulp) * ulp
-    nodes = int(math.floor(rc / h)) + 1
-    if nodes < 64 or nodes > TABLE_MAX_NODES:
+    most = math.floor(fine / ulp)
+    if not 64 <= int(rc / (most * ulp)) + 1 <= TABLE_MAX_NODES:
         return None
+    best = 1.0
+    for m in range(most, math.ceil(0.9 * most) - 1, -1):
+        cells = rc / (m * ulp)
+        if int(cells) + 1 > TABLE_MAX_NODES or best <= 0.125:
+            break
+        if cells - int(cells) < best:
+            best, h, nodes = cells - int(cells), m * ulp, int(cells) + 1
     return nodes, h, rc, float(spec.conv_hi) if spec.conv_cut_kind == 1 else 3.0e38
 
 

@@ -4,8 +4,9 @@ a model whose filters the table cannot hold to the pair-by-pair kernels.
 
 Tolerances: rows and gradients against float64.  A row is a sum of four table
 values (each within the fp32 evaluation's 1e-6 of the largest, weights summing
-to at most 1.25 in magnitude) plus an interpolation error below 2.5e-7 of it:
-2e-6 of the largest value, 4e-6 for derivatives.  Gradients are sums over the
+to at most 1.7 in magnitude, where a cell has no node on one side) plus an
+interpolation error below 2.5e-7 of it: 2e-6 of the largest value, 4e-6 for
+derivatives.  Gradients are sums over the
 pairs of fp32 products: 3e-6 of each tensor's norm.
 """
 
@@ -352,3 +353,59 @@ def test_narrow_basis_between_nodes_closes_the_gate(basis):
     ref = _filters64(model, dist)[0]
     assert (out[0].double().cpu() - ref).abs().max() <= 1e-2 * ref.abs().max()
     ops.numerics_flags("cuda", clear=True)
+
+
+def _cut64(cutoff, t):
+    if cutoff.kind_id == 0:
+        return torch.ones_like(t).unsqueeze(1)
+    hi = cutoff.cutoff_upper
+    return (0.5 * (torch.cos(t * math.pi / hi) + 1.0) * (t < hi)).unsqueeze(1)
+
+
+@pytest.mark.parametrize("rc,num_rbf,basis", [(15.0, 40, "gaussian"), (12.0, 50, "gaussian"),
+                                              (18.5, 50, "expnormal"), (2.0, 5, "gaussian")])
+@pytest.mark.parametrize("rbf_cut,conv_hi", [("cosine", 1.0), ("cosine", 1.3),
+                                             ("cosine", None), ("identity", None)])
+def test_rows_in_the_first_and_last_cells(rc, num_rbf, basis, rbf_cut, conv_hi):
+    """Rows of pairs within two cells of zero distance and of the cutoff, also
+    where the filter does not vanish there, against float64: the fp32 sums of
+    the nodes' values (3e-7 of the largest) times the weights' sum (1.6) and the
+    interpolation (2.5e-7) make 7.5e-7, for derivatives 1.5e-6."""
+    from mlcg_amd import nn, ops
+
+    torch.manual_seed(5)
+    cut = nn.CosineCutoff(0.0, rc) if rbf_cut == "cosine" else nn.IdentityCutoff(0.0, rc)
+    conv = nn.IdentityCutoff(0.0, rc) if conv_hi is None else nn.CosineCutoff(0.0, conv_hi * rc)
+    make = nn.GaussianBasis if basis == "gaussian" else nn.ExpNormalBasis
+    model = nn.StandardSchNet(make(cut, num_rbf=num_rbf), conv, [64], num_interactions=1).cuda()
+    spec, b = model.fused_spec(), model.fused_params().blocks[0]
+    with torch.no_grad():
+        b.b1.normal_(0.0, 0.1)
+    grid = ops.filter_grid(spec.filt, torch.device("cuda:0"))
+    x = torch.rand(600, generator=torch.Generator().manual_seed(1)) * 2 * grid.h
+    dist = torch.cat([x, rc - x, torch.tensor([rc])])
+    pos, graph = _pairs(dist)
+    tables, gates = ops.filter_tables(grid, spec.filt, [(b.W1, b.b1, b.W2)])
+    bins = ops.pair_bins(pos, graph, grid)
+    out, = ops.filter_rows(grid, bins, pos, graph, spec.filt, [(b.W1, b.b1, b.W2)], tables, gates)
+    p = {k: v.detach().double().cpu() for k, v in model.state_dict().items()}
+
+    def f(t):
+        u = t.unsqueeze(1)
+        if basis == "gaussian":
+            g = torch.exp(p["rbf_layer.coeff"] * (u - p["rbf_layer.offset"]) ** 2)
+        else:
+            g = torch.exp(-p["rbf_layer.betas"]
+                          * (torch.exp(-model.rbf_layer.alpha * u) - p["rbf_layer.means"]) ** 2)
+        a = torch.tanh((g * _cut64(cut, t)) @ b.W1.detach().double().cpu().t()
+                       + b.b1.detach().double().cpu())
+        return (a @ b.W2.detach().double().cpu().t()) * _cut64(conv, t)
+
+    def both(t):
+        t = t.double()
+        return torch.func.jvp(f, (t,), (torch.ones_like(t),))
+
+    wide = both(torch.linspace(0, rc, 4001))
+    for got, ref, big, tol in zip(out, both(dist), wide, (7.5e-7, 1.5e-6)):
+        err = ((got.double().cpu() - ref).abs().max() / big.abs().max()).item()
+        assert err <= tol, err

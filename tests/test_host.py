@@ -521,6 +521,7 @@ def test_filter_grid_shape(kw, ok):
     if ok:
         n, h, rc, cut = shape
         assert 64 <= n <= ops.TABLE_MAX_NODES and (n - 1) * h <= rc < n * h
+        assert rc - (n - 1) * h <= 0.125 * h  # every pair close to or between nodes
         k = np.arange(n)
         assert (k.astype(np.float32) * np.float32(h) == k * h).all()  # exact node distances
 
