@@ -1206,6 +1206,15 @@ def filter_tables(grid: FilterGrid, spec: FilterSpec, weights, out=None
     return tables, gates
 
 
+def filter_tables_serve(gates: torch.Tensor) -> torch.Tensor:
+    """[blocks] bool: whether a block's pairs go through its table, as the kernels
+    decide it from these gates (csrc/filter_gate.h), or one by one: its filters
+    are too sharp for the grid or not finite."""
+    g = gates.view(torch.float32)
+    tol = torch.tensor([4e-6, 1.6e-5, 4e-6, 1.6e-5], device=g.device)
+    return (g[:, :4] <= tol * g[:, 4:8]).all(1) & (g[:, 8] <= 0.25)
+
+
 def _pointers(tensors):
     """Host array of device addresses (None -> NULL)."""
     return (ctypes.c_void_p * len(tensors))(*[ptr(t) for t in tensors])

@@ -82,7 +82,7 @@ def _filters64(model, d):
     return torch.func.jvp(f, (t,), (torch.ones_like(t),))
 
 
-def _setup(model, dist):
+def _setup(model, dist, open_gate=True):
     from mlcg_amd import ops
 
     spec, P = model.fused_spec(), model.fused_params()
@@ -90,6 +90,7 @@ def _setup(model, dist):
     pos, graph = _pairs(dist)
     b = P.blocks[0]
     tables, gates = ops.filter_tables(grid, spec.filt, [(b.W1, b.b1, b.W2)])
+    assert ops.filter_tables_serve(gates).tolist() == [open_gate]
     return spec, b, grid, pos, graph, tables, gates, ops.pair_bins(pos, graph, grid)
 
 
@@ -208,21 +209,36 @@ def _batch(frames=40, beads=20):
     return synthetic._flatten(pos, types, 5, forces).to_torch("cuda")
 
 
-def _step(model, table):
-    from mlcg_amd import nn
+def _step(model, table, open_gates=None):
+    """A force-matching step by the given route; open_gates: of each block, as
+    the step's own check left them (all, by default)."""
+    from mlcg_amd import nn, ops
     from mlcg_amd.nn import _fused
 
     saved, _fused._FILTER_TABLE = _fused._FILTER_TABLE, table
+    make, gates = ops.filter_tables, []
+
+    def tables(*args, **kw):
+        out = make(*args, **kw)
+        gates.append(out[1])
+        return out
+
+    ops.filter_tables = tables
     try:
         model.zero_grad(set_to_none=True)
         gm = nn.GradientsOut(model).train()
         d = gm(_batch())
         out = d.out["SchNet"]
         torch.nn.functional.mse_loss(out["forces"], d.forces).backward()
+        assert len(gates) == int(table)
+        if table:
+            want = open_gates or [True] * len(model.interaction_blocks)
+            assert ops.filter_tables_serve(gates[0]).tolist() == want
         return [out["energy"].detach(), out["forces"].detach()] + [
             p.grad.clone() for p in model.parameters()]
     finally:
         _fused._FILTER_TABLE = saved
+        ops.filter_tables = make
 
 
 @pytest.mark.parametrize("basis,trainable", [("gaussian", False), ("gaussian", True),
@@ -245,7 +261,8 @@ def test_closed_gate_gives_the_pairwise_result(poison):
     if poison != "sharp":
         with torch.no_grad():
             model.interaction_blocks[1].conv.filter_network.layers[2].weight[3, 5] = float(poison)
-    table, direct = _step(model, True), _step(model, False)
+    table = _step(model, True, [False, False] if poison == "sharp" else [True, False])
+    direct = _step(model, False)
     assert torch.equal(table[0].nan_to_num(7.0), direct[0].nan_to_num(7.0))
     assert torch.equal(table[1].nan_to_num(7.0), direct[1].nan_to_num(7.0))
     for a, b in zip(table[2:], direct[2:]):
@@ -262,7 +279,7 @@ def test_gate_is_the_blocks_own():
     model = _model(blocks=10)  # more blocks than one launch takes
     with torch.no_grad():
         model.interaction_blocks[0].conv.filter_network.layers[0].weight.mul_(400.0)
-    for a, b in zip(_step(model, True), _step(model, False)):
+    for a, b in zip(_step(model, True, [False] + [True] * 9), _step(model, False)):
         assert rel_err(a, b) <= 1e-5, rel_err(a, b)
     ops.numerics_flags("cuda", clear=True)
 
@@ -348,7 +365,7 @@ def test_narrow_basis_between_nodes_closes_the_gate(basis):
             model.rbf_layer.betas.copy_(0.5 / (0.02 * h * slope) ** 2)
             model.rbf_layer.means.copy_(torch.exp(-alpha * d))
     dist = d.float()
-    spec, b, grid, pos, graph, tables, gates, bins = _setup(model, dist)
+    spec, b, grid, pos, graph, tables, gates, bins = _setup(model, dist, open_gate=False)
     out, = ops.filter_rows(grid, bins, pos, graph, spec.filt, [(b.W1, b.b1, b.W2)], tables, gates)
     ref = _filters64(model, dist)[0]
     assert (out[0].double().cpu() - ref).abs().max() <= 1e-2 * ref.abs().max()
@@ -386,6 +403,7 @@ def test_rows_in_the_first_and_last_cells(rc, num_rbf, basis, rbf_cut, conv_hi):
     dist = torch.cat([x, rc - x, torch.tensor([rc])])
     pos, graph = _pairs(dist)
     tables, gates = ops.filter_tables(grid, spec.filt, [(b.W1, b.b1, b.W2)])
+    assert ops.filter_tables_serve(gates).all()
     bins = ops.pair_bins(pos, graph, grid)
     out, = ops.filter_rows(grid, bins, pos, graph, spec.filt, [(b.W1, b.b1, b.W2)], tables, gates)
     p = {k: v.detach().double().cpu() for k, v in model.state_dict().items()}

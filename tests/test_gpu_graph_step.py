@@ -5,6 +5,8 @@ parameters bit for bit.  The capture follows torch's rules: a capturable
 optimizer (a non-capturable one raises inside the capture region), warm-up
 and capture on one side stream, no timing events inside the capture."""
 
+import contextlib
+
 import pytest
 import torch
 
@@ -12,6 +14,28 @@ from oracle import schnet_ref as R
 from tests.helpers import make_cfg, make_model
 
 pytestmark = pytest.mark.gpu
+
+
+@contextlib.contextmanager
+def _route(table):
+    """The filters' route for the steps inside, which these small batches would
+    not choose by themselves, and that they took it."""
+    from mlcg_amd import ops
+    from mlcg_amd.nn import _fused
+
+    saved, _fused._FILTER_TABLE = _fused._FILTER_TABLE, table
+    combine, calls = ops.filter_table_combine, []
+
+    def counted(*args):
+        calls.append(args[0].nodes)
+        return combine(*args)
+
+    ops.filter_table_combine = counted
+    try:
+        yield
+        assert bool(calls) == table
+    finally:
+        _fused._FILTER_TABLE, ops.filter_table_combine = saved, combine
 
 
 def test_captured_training_step_matches_eager():
@@ -126,10 +150,11 @@ def _step_run(cfg, sd, b, ahead, tmm_side, n_steps=3, captured=False, capturable
 
 
 def test_stream_arrangements_bit_identical():
-    """The filter forwards issued ahead on the side stream, and the
-    weight-gradient reductions on the side stream, change only where kernels
-    run, never what they compute: every arrangement gives the in-order
-    single-stream step's losses, forces and parameters bit for bit."""
+    """The filters' tables made on the side stream beside the ordering of the
+    pairs (which the pair-by-pair route has none of), and the weight-gradient
+    reductions on the side stream, change only where kernels run, never what
+    they compute: every arrangement gives the in-order single-stream step's
+    losses, forces and parameters bit for bit."""
     from mlcg_amd import synthetic
 
     print("stream arrangements, 3 blocks, 16 frames", flush=True)
@@ -175,8 +200,8 @@ def test_node_weight_images_step_bit_identical():
 def test_captured_train_step_api_matches_eager():
     """mlcg_amd.pl.CapturedTrainStep (one warm-up step, then replays that
     each load a second resident copy of the batch) gives the eager steps'
-    losses and parameters bit for bit, with the filter forwards ahead on the
-    side stream inside the graph."""
+    losses and parameters bit for bit, with the side stream's work (the tables,
+    the weight gradients) inside the graph."""
     from mlcg_amd import synthetic
 
     print("CapturedTrainStep, 3 blocks, 16 frames", flush=True)
@@ -240,26 +265,21 @@ def test_captured_train_step_requires_capturable_optimizer():
         CapturedTrainStep(lambda d: nn.GradientsOut(model)(d), data, model, opt)
 
 
-def test_captured_step_outlives_the_kernel_description(monkeypatch):
-    """A recorded step through the filters' tables whose step function returns a
-    detached loss, so that only the graph itself holds what it reads; the
-    model's kernel description is then replaced (fp16 and strict filters
-    switched on and back for a validation call) and freed memory is written
-    over.  The replays still give the eager steps' parameters bit for bit."""
+def test_captured_step_outlives_the_kernel_description():
+    """A recorded step whose step function returns a detached loss, so that only
+    the graph itself holds what it reads; the model's kernel description is then
+    replaced (fp16 and strict filters switched on and back for a validation
+    call) and freed memory is written over.  The replays still give the eager
+    steps' parameters bit for bit."""
     import gc
 
-    from mlcg_amd import nn, ops, synthetic
-    from mlcg_amd.nn import _fused
+    from mlcg_amd import nn, synthetic
     from mlcg_amd.pl import CapturedTrainStep
 
     print("captured step across fp16 / strict filter switches", flush=True)
     cfg = make_cfg(num_blocks=2, rc=20.0)
     sd = R.random_state_dict(cfg, seed=37)
     b = synthetic.config2(n_frames=16)
-    monkeypatch.setattr(_fused, "_FILTER_TABLE", True)
-    rows, seen = ops.filter_table_combine, []
-    monkeypatch.setattr(ops, "filter_table_combine",
-                        lambda *a: seen.append(len(seen)) or rows(*a))
     runs = []
     for captured in (False, True):
         model = make_model(cfg, sd).train()
@@ -295,7 +315,71 @@ def test_captured_step_outlives_the_kernel_description(monkeypatch):
             del junk
             params.append([p.detach().clone() for p in model.parameters()])
         runs.append(params)
-    assert seen  # the steps went through the tables
     for k, (a, c) in enumerate(zip(*runs)):
         for x, y in zip(a, c):
             assert torch.isfinite(x).all() and torch.equal(x, y), k
+
+
+@pytest.mark.parametrize("test", [
+    test_captured_training_step_matches_eager, test_stream_arrangements_bit_identical,
+    test_node_weight_images_step_bit_identical, test_captured_train_step_api_matches_eager,
+    test_captured_train_step_overflow_raises_at_check,
+    test_captured_step_outlives_the_kernel_description,
+], ids=lambda t: t.__name__[5:])
+def test_through_the_filter_tables(test):
+    """The same with the filters through their tables: recorded, with more pair
+    capacity than live pairs and with less than the batch has, and with the
+    tables made on the side stream."""
+    with _route(True):
+        test()
+
+
+def test_captured_step_across_the_filter_route(monkeypatch):
+    """A batch whose pairs are too few for the tables in an eager step, while the
+    recorded step's edge capacity (1.25 times as many) is past the line: the two
+    take different routes, and losses and gradients agree to the filters'
+    rounding (1e-5 of each tensor's norm)."""
+    from mlcg_amd import nn, ops, synthetic
+    from mlcg_amd.pl import CapturedTrainStep
+    from tests.helpers import rel_err
+
+    print("captured step on the other side of the route, 150 frames", flush=True)
+    calls = []
+    combine = ops.filter_table_combine
+    monkeypatch.setattr(ops, "filter_table_combine", lambda *a: calls.append(1) or combine(*a))
+    cfg = make_cfg(num_blocks=3, rc=20.0)
+    sd = R.random_state_dict(cfg, seed=38)
+    batch = synthetic.config2(n_frames=150)
+
+    def build():
+        # a model, an optimizer and a batch of its own for each way: gradient
+        # accumulation nodes of a step that is still referred to (data.out)
+        # belong to its stream, and a recording must not find them
+        model = make_model(cfg, sd).train()
+        gm = nn.GradientsOut(model)
+        opt = torch.optim.AdamW(model.parameters(), lr=0.0, weight_decay=0.0, fused=True,
+                                capturable=True)
+
+        def step(d):
+            opt.zero_grad(set_to_none=True)
+            out = gm(d)
+            out.out.update(**out.out[model.name])
+            loss = nn.ForceMSE()(out)
+            loss.backward()
+            opt.step()
+            return loss
+
+        return model, opt, step, batch.to_torch("cuda")
+
+    model, _, step, data = build()
+    eager = [step(data).detach().clone()] + [p.grad.clone() for p in model.parameters()]
+    assert not calls
+    model, opt, step, data = build()
+    cs = CapturedTrainStep(step, data, model, opt, warmup=1)
+    assert calls
+    for _ in range(3):
+        loss = cs.step(data)
+        torch.cuda.synchronize()
+        for a, b in zip(eager, [loss.detach()] + [p.grad for p in model.parameters()]):
+            assert rel_err(a, b) <= 1e-5
+    cs.check()
