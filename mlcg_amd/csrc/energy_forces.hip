@@ -42,7 +42,8 @@ struct Layout {
 // ... and of the tangent and second reverse sweep, which also reads a kept Layout.
 struct Layout2 {
   int blocks;
-  int xdot(int k) const { return k - 1; }  // input tangent of block k >= 1; blocks: the last's output
+  // input tangent of block k >= 1; k = blocks: of the last block's output
+  int xdot(int k) const { return k - 1; }
   int ydot(int k) const { return blocks + k; }  // k >= 1
   int aggdot(int k) const { return 2 * blocks + k; }
   int zdot(int k) const { return 3 * blocks + k; }

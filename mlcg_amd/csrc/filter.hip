@@ -2866,13 +2866,12 @@ extern "C" int64_t mlcg_rbf_param_grad_workspace_floats(int64_t max_pairs, int n
 }
 
 static int rbf_param_grad_impl(const float* dist, const int32_t* n_pairs_dev,
-                                   int64_t max_pairs, int basis, const float* centers,
-                                   const float* widths, double alpha, int num_rbf,
-                                   int rbf_cut_kind, float rbf_lo, float rbf_hi,
-                                   const float* W1, int num_filters, const float* abar,
-                                   const float* adbar, int accumulate, float* dcenters,
-                                   float* dwidths, float* workspace, int64_t workspace_floats,
-                                   const FilterGate& gate, void* stream) {
+                               int64_t max_pairs, int basis, const float* centers,
+                               const float* widths, double alpha, int num_rbf, int rbf_cut_kind,
+                               float rbf_lo, float rbf_hi, const float* W1, int num_filters,
+                               const float* abar, const float* adbar, int accumulate,
+                               float* dcenters, float* dwidths, float* workspace,
+                               int64_t workspace_floats, const FilterGate& gate, void* stream) {
   if (!valid_params(basis, num_rbf, rbf_cut_kind, 0, 0, num_filters))
     return MLCG_ERR_UNSUPPORTED;
   MLCG_REQUIRE(max_pairs >= 0 && centers && widths && W1 && dcenters && dwidths && workspace);
@@ -2914,16 +2913,23 @@ extern "C" int mlcg_rbf_param_grad(const float* dist, const int32_t* n_pairs_dev
                                    const float* adbar, int accumulate, float* dcenters,
                                    float* dwidths, float* workspace, int64_t workspace_floats,
                                    void* stream) {
-  return rbf_param_grad_impl(dist, n_pairs_dev, max_pairs, basis, centers, widths, alpha, num_rbf, rbf_cut_kind, rbf_lo, rbf_hi, W1, num_filters, abar, adbar, accumulate, dcenters, dwidths, workspace, workspace_floats, FilterGate{nullptr, 0}, stream);
+  return rbf_param_grad_impl(dist, n_pairs_dev, max_pairs, basis, centers, widths, alpha, num_rbf,
+                             rbf_cut_kind, rbf_lo, rbf_hi, W1, num_filters, abar, adbar,
+                             accumulate, dcenters, dwidths, workspace, workspace_floats,
+                             FilterGate{nullptr, 0}, stream);
 }
 
 extern "C" int mlcg_rbf_param_grad_gated(const float* dist, const int32_t* n_pairs_dev,
-                                   int64_t max_pairs, int basis, const float* centers,
-                                   const float* widths, double alpha, int num_rbf,
-                                   int rbf_cut_kind, float rbf_lo, float rbf_hi,
-                                   const float* W1, int num_filters, const float* abar,
-                                   const float* adbar, int accumulate, float* dcenters,
-                                   float* dwidths, float* workspace, int64_t workspace_floats,
-                                   const uint32_t* gate, int gate_want, void* stream) {
-  return rbf_param_grad_impl(dist, n_pairs_dev, max_pairs, basis, centers, widths, alpha, num_rbf, rbf_cut_kind, rbf_lo, rbf_hi, W1, num_filters, abar, adbar, accumulate, dcenters, dwidths, workspace, workspace_floats, FilterGate{gate, gate_want}, stream);
+                                         int64_t max_pairs, int basis, const float* centers,
+                                         const float* widths, double alpha, int num_rbf,
+                                         int rbf_cut_kind, float rbf_lo, float rbf_hi,
+                                         const float* W1, int num_filters, const float* abar,
+                                         const float* adbar, int accumulate, float* dcenters,
+                                         float* dwidths, float* workspace,
+                                         int64_t workspace_floats, const uint32_t* gate,
+                                         int gate_want, void* stream) {
+  return rbf_param_grad_impl(dist, n_pairs_dev, max_pairs, basis, centers, widths, alpha, num_rbf,
+                             rbf_cut_kind, rbf_lo, rbf_hi, W1, num_filters, abar, adbar,
+                             accumulate, dcenters, dwidths, workspace, workspace_floats,
+                             FilterGate{gate, gate_want}, stream);
 }

@@ -11,12 +11,15 @@
 // error is 2^-4 of the measured one: at the bounds below 2.5e-7 of the largest
 // value and 1e-6 of the largest derivative -- the rounding of the fp32
 // evaluation itself (3.4e-7 and 6e-7; the split-fp16 kernels' derivative:
-// 4.7e-6).  The cutoff distance, up to 1/8 of a cell past the last node, has its
-// error measured as it is used: of the truncation of the cells beside the ends,
-// and compared with the same bounds.  Basis functions narrower than the spacing, which could lie between
-// two nodes unseen, set the last word to infinity; of wider ones the nodes see
-// every feature, and a pre-activation that changes by less than 1/4 per node
-// leaves the activation none of its own.
+// 4.7e-6).  The cutoff distance, up to 1/8 of a cell past the last node, has
+// its error measured as it is used: of the truncation of the cells beside the
+// ends, and compared with the same bounds.
+//
+// Basis functions narrower than the spacing, which could lie between two nodes
+// unseen, set the last word to infinity; of wider ones the nodes see every
+// feature, and a pre-activation that changes by less than 1/4 per node leaves
+// the activation none of its own.  So do weights of 65504 or more, which the
+// split kernels report.
 #pragma once
 
 #include "common.h"

@@ -338,8 +338,8 @@ __device__ __forceinline__ float4 lerp4(const float4* r, const float w[4]) {
 
 // Rows of the pairs: a wave reads a stencil's eight table rows once for all its
 // pairs, so the launch is bound by the rows it writes: 217 k pairs, three blocks
-// 138 us, 4.8 TB/s, where the network pair by pair takes 87-92 us a block; 3.0 M
-// pairs in fp16 875 us, 5.3 TB/s, against 1447.
+// 133 us, 5.2 TB/s, where the network pair by pair takes 87-92 us a block; 3.0 M
+// pairs in fp16 866 us, 5.6 TB/s, against 1447.
 constexpr int kMaxBlocks = 8;  // blocks of a launch (blockIdx.y)
 struct RowsBatch {
   void *W[kMaxBlocks], *Wd[kMaxBlocks];
@@ -395,10 +395,10 @@ __global__ __launch_bounds__(256) void table_rows_kernel(
 // Bound by the node rows (4 KiB a pair).  A key of R runs deals its records out
 // in turn, so that every wave sweeps the batch from its first frame to its
 // last: the waves of an XCD are in about the same frames at the same time and
-// find more of their rows in its L2 (22 % against 17 % with contiguous runs).
-// The rest comes at the 7.3 TB/s of the memory-side cache: 217 k pairs of 512 x
-// 35 beads 110 us a block and 8 for table_combine_kernel, where the pair-by-pair
-// backward takes 241-254.
+// find some of their rows in its L2 (219 k pairs of 512 x 35 beads 22 %, 879 k of
+// 512 x 100 beads 9 %).  The rest comes from the memory-side cache, 6.4 and 7.3
+// TB/s: 105 and 450 us a block and 6 and 10 for table_combine_kernel, where the
+// pair-by-pair backward takes 241-254 us at the smaller size.
 //
 // Bonded pairs share one distance, so a single key can hold a tenth of the
 // pairs: a workgroup whose runs all have one key adds its waves' blocks first
@@ -433,9 +433,9 @@ __device__ __forceinline__ int run_key(const int32_t* __restrict__ run_start, in
 template <bool kTan, bool kYd>
 __global__ __launch_bounds__(kRevWaves * MLCG_WAVE) void table_reverse_kernel(
     const int4* __restrict__ recs, const int32_t* __restrict__ start,
-    const int32_t* __restrict__ run_start, int nkeys, const float* __restrict__ g2, const float* __restrict__ y, const float* __restrict__ g1,
-    const float* __restrict__ yd, const float* __restrict__ dd, FilterGate gate,
-    float* __restrict__ slots) {
+    const int32_t* __restrict__ run_start, int nkeys, const float* __restrict__ g2,
+    const float* __restrict__ y, const float* __restrict__ g1, const float* __restrict__ yd,
+    const float* __restrict__ dd, FilterGate gate, float* __restrict__ slots) {
   if (gate_closed(gate)) return;
   __shared__ __align__(16) float2 fold[kRevWaves][8][MLCG_WAVE];
   const int l = mlcg_lane();
@@ -689,8 +689,9 @@ extern "C" int mlcg_filter_table_check(const float* tables, int num_blocks, int 
 }
 
 extern "C" int mlcg_filter_table_rows(const int32_t* records, const int32_t* n_pairs_dev,
-                                      int64_t max_pairs, int nodes, const float* tables, const uint32_t* gates, int num_blocks,
-                                      int f16, void* const* outputs, void* stream) {
+                                      int64_t max_pairs, int nodes, const float* tables,
+                                      const uint32_t* gates, int num_blocks, int f16,
+                                      void* const* outputs, void* stream) {
   MLCG_REQUIRE(table_shape_ok(nodes) && max_pairs >= 0 && num_blocks >= 1);
   if (max_pairs == 0) return MLCG_OK;
   MLCG_REQUIRE(records && n_pairs_dev && tables && gates && outputs);
@@ -740,9 +741,9 @@ extern "C" int mlcg_filter_table_reverse(const int32_t* records, const int32_t* 
   hipStream_t s = mlcg_stream(stream);
   // every key may leave one run partly filled
   const dim3 grid(mlcg_div_up((max_pairs + kRev - 1) / kRev + nkeys, kRevWaves));
-#define MLCG_REV(T, Y)                                                                        \
-  hipLaunchKernelGGL((table_reverse_kernel<T, Y>), grid, dim3(kRevWaves * MLCG_WAVE), 0, s, recs, start,      \
-                     run_start, nkeys, gagg2, y, gagg1, ydot, ddot, g, slots)
+#define MLCG_REV(T, Y)                                                                      \
+  hipLaunchKernelGGL((table_reverse_kernel<T, Y>), grid, dim3(kRevWaves * MLCG_WAVE), 0, s, \
+                     recs, start, run_start, nkeys, gagg2, y, gagg1, ydot, ddot, g, slots)
   if (gagg1 && ydot)
     MLCG_REV(true, true);
   else if (gagg1)

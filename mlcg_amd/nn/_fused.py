@@ -322,9 +322,11 @@ def _table_grid(spec: FusedSpec, filt, graph: ops.PairGraph, pos: torch.Tensor, 
 
 
 # MLCG_FILTER_AHEAD=1 makes the filters' tables on the side stream, beside the
-# ordering of the pairs.  Off: each of the two fills the chip, and the streams'
-# waits cost more than the overlap gives (512 x 35 beads, captured step 1824 us with
-# it, 1812 without, eager step 2055 and 1977; MD step of 100 x 268 1738 and 1716).
+# ordering of the pairs; the results are the same.  Off: each of the two fills the
+# chip, and the streams' waits cost more than the overlap gives (512 x 35 beads,
+# captured step 1824 us with it, 1812 without, eager step 2055 and 1977; MD step of
+# 100 x 268 1738 and 1716).  It stays as a switch because programs set it: with the
+# filters pair by pair, where the overlap did pay, it was how to turn it off.
 _FILTER_AHEAD = os.environ.get("MLCG_FILTER_AHEAD", "0") == "1"
 
 

@@ -902,13 +902,12 @@ def filter_fwd(pos: torch.Tensor, graph: PairGraph, spec: FilterSpec, W1: torch.
                "filter_fwd out tensors must be contiguous [pair_capacity, 128] of the result dtype")
     dist = torch.empty(cap, dtype=torch.float32, device=pos.device) if want_dist else None
     W1c, b1c, W2c = (t.detach().float().contiguous() for t in (W1, b1, W2))
-    args = (ptr(pos), ptr(graph.pair_ij), cap, ptr(graph.n_pairs_dev), cap,
-            *spec.basis_args(), spec.num_rbf, spec.rbf_cut_kind, spec.rbf_lo,
-            spec.rbf_hi, spec.conv_cut_kind, spec.conv_lo, spec.conv_hi, spec.act, ptr(W1c),
-            ptr(b1c), ptr(W2c), F,
-            FILTER_FP16 if f16 else (FILTER_FP32_STRICT if strict_fp32 else FILTER_FP32),
-            ptr(W), ptr(Wd), ptr(dist))
-    call("mlcg_filter_fwd", *args, stream_handle(pos.device))
+    call("mlcg_filter_fwd", ptr(pos), ptr(graph.pair_ij), cap, ptr(graph.n_pairs_dev), cap,
+         *spec.basis_args(), spec.num_rbf, spec.rbf_cut_kind, spec.rbf_lo,
+         spec.rbf_hi, spec.conv_cut_kind, spec.conv_lo, spec.conv_hi, spec.act, ptr(W1c),
+         ptr(b1c), ptr(W2c), F,
+         FILTER_FP16 if f16 else (FILTER_FP32_STRICT if strict_fp32 else FILTER_FP32),
+         ptr(W), ptr(Wd), ptr(dist), stream_handle(pos.device))
     return W, Wd, dist
 
 
@@ -988,12 +987,11 @@ def filter_bwd(pos: torch.Tensor, graph: PairGraph, spec: FilterSpec, W1: torch.
     dW1, db1, dW2 = _filter_grads(F, K, dev)
     W1c, b1c, W2c = (t.detach().float().contiguous() for t in (W1, b1, W2))
     ab, adb = _pair_adjoint_outputs(pair_adjoints, cap, F, dev)
-    args = (ptr(pos), ptr(graph.pair_ij), cap, ptr(graph.n_pairs_dev), cap,
-            *spec.basis_args(), K, spec.rbf_cut_kind, spec.rbf_lo, spec.rbf_hi,
-            spec.conv_cut_kind, spec.conv_lo, spec.conv_hi, spec.act, ptr(W1c), ptr(b1c),
-            ptr(W2c), F, ptr(Wbar.contiguous()), ptr(Wdbar.contiguous()), ptr(dW1), ptr(db1),
-            ptr(dW2), ptr(ab), ptr(adb), ptr(ws), nws, int(strict_fp32))
-    call("mlcg_filter_bwd", *args, stream_handle(dev))
+    call("mlcg_filter_bwd", ptr(pos), ptr(graph.pair_ij), cap, ptr(graph.n_pairs_dev), cap,
+         *spec.basis_args(), K, spec.rbf_cut_kind, spec.rbf_lo, spec.rbf_hi,
+         spec.conv_cut_kind, spec.conv_lo, spec.conv_hi, spec.act, ptr(W1c), ptr(b1c),
+         ptr(W2c), F, ptr(Wbar.contiguous()), ptr(Wdbar.contiguous()), ptr(dW1), ptr(db1),
+         ptr(dW2), ptr(ab), ptr(adb), ptr(ws), nws, int(strict_fp32), stream_handle(dev))
     if pair_adjoints:
         return dW1, db1, dW2, ab, adb
     return dW1, db1, dW2
@@ -1020,12 +1018,12 @@ def filter_bwd_cfconv(pos: torch.Tensor, graph: PairGraph, spec: FilterSpec,
     W1c, b1c, W2c = (t.detach().float().contiguous() for t in (W1, b1, W2))
     c = lambda t: None if t is None else t.contiguous()  # noqa: E731
     ab, adb = _pair_adjoint_outputs(pair_adjoints, cap, F, dev)
-    args = (ptr(pos), ptr(graph.pair_ij), cap, ptr(graph.n_pairs_dev),
-            cap, *spec.basis_args(), K, spec.rbf_cut_kind, spec.rbf_lo, spec.rbf_hi,
-            spec.conv_cut_kind, spec.conv_lo, spec.conv_hi, spec.act, ptr(W1c), ptr(b1c),
-            ptr(W2c), F, ptr(c(gagg2)), ptr(c(y)), ptr(c(gagg1)), ptr(c(ydot)), ptr(ddot),
-            ptr(dW1), ptr(db1), ptr(dW2), ptr(ab), ptr(adb), ptr(ws), nws, int(strict_fp32))
-    call("mlcg_filter_bwd_cfconv", *args, stream_handle(dev))
+    call("mlcg_filter_bwd_cfconv", ptr(pos), ptr(graph.pair_ij), cap, ptr(graph.n_pairs_dev),
+         cap, *spec.basis_args(), K, spec.rbf_cut_kind, spec.rbf_lo, spec.rbf_hi,
+         spec.conv_cut_kind, spec.conv_lo, spec.conv_hi, spec.act, ptr(W1c), ptr(b1c),
+         ptr(W2c), F, ptr(c(gagg2)), ptr(c(y)), ptr(c(gagg1)), ptr(c(ydot)), ptr(ddot),
+         ptr(dW1), ptr(db1), ptr(dW2), ptr(ab), ptr(adb), ptr(ws), nws, int(strict_fp32),
+         stream_handle(dev))
     if pair_adjoints:
         return dW1, db1, dW2, ab, adb
     return dW1, db1, dW2

@@ -7,9 +7,12 @@ around them, so on a slow host the GPU waits between launches.  For batches
 of one fixed shape (the usual CG case: one molecule, a fixed number of frames
 per batch) the whole step can be recorded once and replayed with a single
 host call per step.  Each replay first copies the new batch into the
-recorded input tensors (device to device); the results are those of the
-eager step bit for bit (the kernels, their order and their launch shapes are
-the same).
+recorded input tensors (device to device); the results are those of an
+eager step with the same edge capacity bit for bit (the kernels, their order
+and their launch shapes are the same).  An eager step that sizes its graph
+exactly counts its own, fewer pairs when it chooses between the two ways of
+evaluating the filters (nn/_fused.py, _table_pays): between the two counts
+the results differ by the filters' rounding, about 4e-7.
 
 Requirements, checked at construction:
 - the optimizer is capturable (``torch.optim.AdamW(..., capturable=True)``);
@@ -20,6 +23,11 @@ Requirements, checked at construction:
   with more edges than the capacity sets the graph's overflow flag instead of
   growing it: ``check()`` (one host synchronisation) raises if any replay
   since the last check overflowed.
+
+Not checked: outputs of an earlier step of the same parameters (a loss, a
+batch's ``out``) must not be referred to any more when the step is recorded.
+They keep torch's gradient accumulation nodes, which run on the stream they
+were made on, and a recording that finds such a node fails.
 """
 
 from __future__ import annotations

@@ -427,3 +427,22 @@ def test_rows_in_the_first_and_last_cells(rc, num_rbf, basis, rbf_cut, conv_hi):
     for got, ref, big, tol in zip(out, both(dist), wide, (7.5e-7, 1.5e-6)):
         err = ((got.double().cpu() - ref).abs().max() / big.abs().max()).item()
         assert err <= tol, err
+
+
+@pytest.mark.parametrize("basis,act,num_rbf", [("gaussian", "tanh", 50), ("expnormal", "ssp", 64),
+                                               ("gaussian", "ssp", 100)])
+@pytest.mark.parametrize("mode", ["split", "strict", "fp16"])
+def test_blocks_forward_equals_the_single_one(basis, act, num_rbf, mode):
+    """filter_fwd_blocks, which the model calls, gives every block filter_fwd's
+    rows bit for bit: what is shown of the one holds for the other."""
+    from mlcg_amd import ops
+
+    model = _model(basis, act, num_rbf, blocks=9)  # more than one launch takes
+    spec, P = model.fused_spec(), model.fused_params()
+    pos, graph = _pairs(_distances(2001, 0.01))
+    kw = dict(f16=mode == "fp16", strict_fp32=mode == "strict")
+    weights = [(b.W1, b.b1, b.W2) for b in P.blocks]
+    rows, dist = ops.filter_fwd_blocks(pos, graph, spec.filt, weights, **kw)
+    for w, (W, Wd) in zip(weights, rows):
+        ref = ops.filter_fwd(pos, graph, spec.filt, *w, **kw)
+        assert torch.equal(W, ref[0]) and torch.equal(Wd, ref[1]) and torch.equal(dist, ref[2])
