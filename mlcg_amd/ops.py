@@ -1292,7 +1292,8 @@ def energy_forces_ok(pos: torch.Tensor, types: torch.Tensor, graph: PairGraph, w
     square, width = weights[1:1 + 5 * n], NUM_FILTERS
     return (n >= 1 and weights[0].dim() == 2 and weights[0].shape[1] == width
             and all(square[5 * k + i].shape == shape for k in range(n) for i in (0, 1, 3))
-            and all(square[5 * k + i].numel() == width for k in range(n) for i in (2, 4))
+            and all(square[5 * k + i] is not None and square[5 * k + i].numel() == width
+                    for k in range(n) for i in (2, 4))
             and hidden in OUT_HIDDEN and weights[-4].shape == (hidden, width)
             and weights[-2].numel() == hidden)
 
